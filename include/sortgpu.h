@@ -82,7 +82,9 @@ const char* sortgpu_last_error(const sortgpu_ctx* ctx);
  *      accel/fast_bvh.hpp:109-136) ----
  * pos: nverts x 3 floats; idx: ntris x 3 vertex indices; quads: nquads records. The SAH
  * 8-wide (or 4-wide) tree is built on the host, flattened into the device layout and
- * uploaded. Input arrays are copied; the caller keeps ownership. An empty scene yields a
+ * uploaded, with a second tree over the same primitives that closest- and any-hit queries step
+ * through to the same results (about 70 MB for a million triangles; scenes whose coordinates are not
+ * finite, pass 1e12 or lie 4,096 times their size from the origin go without). Input arrays are copied; the caller keeps ownership. An empty scene yields a
  * valid handle whose queries all miss (m_isValid = false, fast_bvh.hpp:112-114). At most
  * 2^30 - 1 primitives (triangles + quads) per tree (SORTGPU_ERR_ARG beyond). */
 int sortgpu_accel_build(sortgpu_ctx* ctx, const float* pos, uint32_t nverts, const uint32_t* idx,
@@ -221,8 +223,10 @@ int sortgpu_accel_errors(sortgpu_accel* accel, void* stream, uint32_t* flags);
  * idle lanes of a wave that trigger refilling them with new rays from the work queue (default 16,
  * 1..64); lds_entries = traversal-stack entries per lane kept in LDS (8 or 16,
  * default 16); blocks_per_cu = cap on resident workgroups per CU (default: occupancy limit);
- * leaf_batch = lanes of a wave holding a leaf that end a node-walking phase (default 32, 1..64);
- * leaf_min = a leaf-testing phase ends when fewer lanes hold a leaf (default 1, 1..64);
+ * leaf_batch = lanes of a wave holding a leaf that end a node-walking phase (default 16 for closest
+ * and any hit, 32 for transparent shadows and trees without a walk tree; 1..64);
+ * leaf_min = a leaf-testing phase ends when fewer lanes hold a leaf (default 1, 1..64; transparent
+ * shadows and trees without a walk tree only);
  * reorder = traversal order of sortgpu_trace_closest / _any / _attenuation / _multi and
  * sortgpu_pool_trace batches: 0 (default) sorts batches of at least 262,144 rays by origin cell
  * (128^3 grid over the scene box; pooled rays by scene, then by cell in their scene's box) before the
@@ -364,7 +368,9 @@ int sortgpu_render_stage_times(sortgpu_scene* scene, float out_ms[3], uint32_t* 
 typedef struct sortgpu_server sortgpu_server;
 
 typedef struct sortgpu_server_opts {
-    uint64_t hbm_budget;     /* bytes the server may hold: scenes + films + workspace (0 = 96 GiB) */
+    uint64_t hbm_budget;     /* bytes the server may hold: scenes + films + workspace (0 = 96 GiB);
+                                a scene that would not fit alone is loaded without the second tree
+                                of its accelerator (sortgpu_accel_build) */
     uint32_t wave_paths;     /* path slots per wave (0 = 33,554,432; 248 B of workspace each) */
     uint32_t max_active;     /* requests admitted at once, 1..32 (0 = 32) */
     uint32_t inflight_waves; /* waves in flight at once, 1..4 (0 = 3), each on a stream and path

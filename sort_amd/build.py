@@ -36,10 +36,10 @@ DEVICE = [
     "-munsafe-fp-atomics",
 ]
 
-HOST_SOURCES = ["api.cpp", "accel_device.cpp", "bvh_build.cpp", "pool.cpp", "serve_engine.cpp", "serve_api.cpp",
+HOST_SOURCES = ["api.cpp", "accel_device.cpp", "bvh_build.cpp", "walk_tree.cpp", "pool.cpp", "serve_engine.cpp", "serve_api.cpp",
                 "scene_file.cpp", "hit_surface.cpp"]
 # compiled as HIP: kernels, and host code that shares device record types with them
-DEVICE_SOURCES = ["trace.hip", "order.hip", "multihit.hip", "film_out.hip", "pt.hip", "pt_host.cpp", "pt_api.cpp", "serve_device.cpp"]
+DEVICE_SOURCES = ["trace.hip", "walk.hip", "order.hip", "multihit.hip", "film_out.hip", "pt.hip", "pt_host.cpp", "pt_api.cpp", "serve_device.cpp"]
 # the vector-memory probe bench.py measures the traversal's ceiling with (benchmark code, its own
 # library beside its source; not part of libsortgpu)
 PROBE_SRC = os.path.join(ROOT, "measure", "chunk_probe.hip")

@@ -43,6 +43,9 @@ struct sortgpu_accel {
     void* d_nodes = nullptr;
     sortgpu::PrimRec* d_prims = nullptr;
     sortgpu::QuadRec* d_quads = nullptr;
+    sortgpu::WalkNode* d_wnodes = nullptr;
+    sortgpu::PrimRec* d_wrecs = nullptr;
+    sortgpu::WalkAux* d_waux = nullptr;
     uint32_t* d_counters = nullptr;
     uint32_t* d_error = nullptr;
     unsigned long long* d_stats = nullptr;

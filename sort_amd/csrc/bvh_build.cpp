@@ -70,12 +70,7 @@ inline Box union_of(const Box& a, const Box& b) {  // free Union(BBox, BBox), bb
 
 // Build primitive: bounds, centroid and id together so that binning and partitioning stream
 // one array (40 B per primitive).
-struct BPrim {
-    float mn[3];
-    float mx[3];
-    float c[3];
-    uint32_t id;
-};
+using BPrim = BuildPrim;
 
 struct BNode {
     uint32_t off = 0, cnt = 0, child_cnt = 0;
@@ -401,6 +396,27 @@ struct Flattener {
     }
 };
 
+// The tree as an array in breadth-first order, for the walk-tree builder.
+std::vector<SrcNode> source_nodes(const BNode* root, size_t count) {
+    std::vector<SrcNode> src;
+    std::vector<const BNode*> at;
+    src.reserve(count);
+    at.reserve(count);
+    at.push_back(root);
+    src.push_back({root->off, root->cnt, 0, 0});
+    for (size_t i = 0; i < at.size(); i++) {
+        const BNode* n = at[i];
+        src[i].first = (uint32_t)at.size();
+        src[i].nchild = n->child_cnt;
+        for (uint32_t j = 0; j < n->child_cnt; j++) {
+            const BNode* c = n->child[j].get();
+            at.push_back(c);
+            src.push_back({c->off, c->cnt, 0, 0});
+        }
+    }
+    return src;
+}
+
 }  // namespace
 
 bool build_tree(const BuildInput& in, BuiltTree& out, std::string& err) {
@@ -547,6 +563,7 @@ bool build_tree(const BuildInput& in, BuiltTree& out, std::string& err) {
         out.prims = std::move(F.prims);
         out.dump = std::move(F.dump);
     }
+    build_walk_tree(in, B.P, source_nodes(root.get(), out.n_inner + out.n_leaves), out.bbox, nthreads, out.walk);
     out.build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return true;
 }

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "layout.h"
+#include "walk_tree.h"
 
 namespace sortgpu {
 
@@ -49,6 +50,7 @@ struct BuiltTree {
     std::vector<unsigned char> node_bytes;  // n_inner NodeRec<width>
     std::vector<PrimRec> prims;             // leaf records (+1 zero record)
     std::vector<QuadRec> quads;
+    WalkTree walk;                          // empty when the scene cannot have one
 };
 
 // Returns false and sets err on invalid input.

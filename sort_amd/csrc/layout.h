@@ -60,16 +60,48 @@ struct alignas(16) QuadRec {
 };
 static_assert(sizeof(QuadRec) == 80, "QuadRec must be 80 B");
 
+// Walk tree (walk_tree.cpp): a 4-wide tree over the same primitives that the closest- and any-hit
+// kernel steps through (walk.hip). Its boxes are quantised outwards on a grid of its node, 48 bytes
+// a node (three 16-byte loads instead of the eight or fourteen of a NodeRec<8>), and every leaf
+// slot is one record of at most two triangles, or one quad.
+//
+// Slots: inner children first (node indices child_base + slot), then leaves (record indices
+// rec_base + slot - inner count), then unused slots. Plane q of an axis lies at base + q * 2^(e - 127).
+struct alignas(16) WalkNode {
+    float base[3];
+    uint8_t exp[3];       // biased exponent e of the grid step per axis
+    uint8_t counts;       // inner children | (all children << 4)
+    uint32_t child_base;  // node index of the first inner child
+    uint32_t rec_base;    // record index of the first leaf child
+    uint8_t lo_x[4], hi_x[4], lo_y[4], hi_y[4], lo_z[4], hi_z[4];
+};
+static_assert(sizeof(WalkNode) == 48, "WalkNode must be 48 B");
+
+// Beside each walk record: the box of the Fast-BVH leaf that holds its primitives, as its parent
+// node's planes bound it, that leaf's number, and the places of A and B among the leaf's primitives
+// (16 bits each; 0xFFFF: 65,535 or more).
+struct alignas(16) WalkAux {
+    float lo[3], hi[3];
+    uint32_t leaf;
+    uint32_t places;
+};
+static_assert(sizeof(WalkAux) == 32, "WalkAux must be 32 B");
+
 // Everything a traversal kernel needs about one tree.
 struct TreeView {
     const void* nodes;      // NodeRec<W>*
     const PrimRec* prims;
     const QuadRec* quads;
+    const WalkNode* wnodes; // walk tree (null: none)
+    const PrimRec* wrecs;
+    const WalkAux* waux;
     uint32_t root;          // child reference of the root (leaf when the tree is one leaf)
     uint32_t valid;         // 0: every query misses
     uint32_t max_stack;     // (W-1)*(depth-1)+1
     uint32_t width;
     float bbox[6];          // enlarged scene box (root slab test)
+    uint32_t walk_stack;    // most stack entries a walk-tree traversal holds; 0: no walk tree
+    uint32_t pad;
 };
 
 }  // namespace sortgpu

@@ -15,7 +15,7 @@ using namespace sortgpu;
 
 struct sortgpu_pool {
     sortgpu_ctx* ctx = nullptr;
-    uint32_t n = 0, width = 8, max_stack = 1;
+    uint32_t n = 0, width = 8, max_stack = 1, walk_stack = 0;
     void* d_block = nullptr;       // all node / primitive / quad records
     TreeView* d_views = nullptr;   // n tree views
     uint32_t* d_counters = nullptr;
@@ -40,7 +40,8 @@ int sortgpu_pool_create(sortgpu_ctx* ctx, sortgpu_accel* const* accels, uint32_t
         set_error(ctx, "sortgpu_pool_create: host-only context");
         return SORTGPU_ERR_STATE;
     }
-    uint32_t width = 0, max_stack = 1;
+    uint32_t width = 0, max_stack = 1, walk_stack = 0;
+    bool walk = true;  // every tree has a walk tree
     size_t total = 0;
     for (uint32_t i = 0; i < n; i++) {
         const sortgpu_accel* a = accels[i];
@@ -54,10 +55,18 @@ int sortgpu_pool_create(sortgpu_ctx* ctx, sortgpu_accel* const* accels, uint32_t
                 return SORTGPU_ERR_ARG;
             }
             width = a->host.width;
+            walk &= a->host.walk.stack != 0;
         }
         max_stack = std::max(max_stack, a->host.max_stack);
         total += align256(a->host.node_bytes.size()) + align256(a->host.prims.size() * sizeof(PrimRec)) +
                  align256(a->host.quads.size() * sizeof(QuadRec));
+        walk_stack = std::max(walk_stack, a->host.walk.stack);
+    }
+    if (!walk) walk_stack = 0;
+    for (uint32_t i = 0; i < n && walk_stack; i++) {
+        const WalkTree& w = accels[i]->host.walk;
+        total += align256(w.nodes.size() * sizeof(WalkNode)) + align256(w.recs.size() * sizeof(PrimRec)) +
+                 align256(w.aux.size() * sizeof(WalkAux));
     }
     if (!width) width = 8;
     if (max_stack > trace_max_stack_supported()) {
@@ -74,6 +83,7 @@ int sortgpu_pool_create(sortgpu_ctx* ctx, sortgpu_accel* const* accels, uint32_t
     p->n = n;
     p->width = width;
     p->max_stack = max_stack;
+    p->walk_stack = walk_stack;
     hipError_t e;
     auto fail = [&](hipError_t err, const char* what) {
         int r = hip_fail(ctx, err, what);
@@ -110,6 +120,19 @@ int sortgpu_pool_create(sortgpu_ctx* ctx, sortgpu_accel* const* accels, uint32_t
         if (qb && (e = hipMemcpy(base + off, h.quads.data(), qb, hipMemcpyHostToDevice)) != hipSuccess)
             return fail(e, "hipMemcpy(pool quads)");
         off += align256(qb);
+        if (walk_stack && h.walk.stack) {
+            auto put = [&](const void* src, size_t bytes) -> void* {
+                void* dst = base + off;
+                if (e == hipSuccess) e = hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+                off += align256(bytes);
+                return dst;
+            };
+            v.wnodes = static_cast<const WalkNode*>(put(h.walk.nodes.data(), h.walk.nodes.size() * sizeof(WalkNode)));
+            v.wrecs = static_cast<const PrimRec*>(put(h.walk.recs.data(), h.walk.recs.size() * sizeof(PrimRec)));
+            v.waux = static_cast<const WalkAux*>(put(h.walk.aux.data(), h.walk.aux.size() * sizeof(WalkAux)));
+            if (e != hipSuccess) return fail(e, "hipMemcpy(pool walk tree)");
+            v.walk_stack = h.walk.stack;
+        }
         v.root = h.root_ref;
         v.valid = h.valid ? 1u : 0u;
         v.max_stack = h.max_stack;
@@ -179,6 +202,7 @@ int sortgpu_pool_trace(sortgpu_pool* p, const sortgpu_ray* d_rays, const uint32_
     a.n_trees = p->n;
     a.width = p->width;
     a.max_stack = p->max_stack;
+    a.walk_stack = p->walk_stack;
     apply_tuning(p->ctx, a);
     hipStream_t s = static_cast<hipStream_t>(stream);
     // traversal order of a large batch: by scene, then by origin cell in that scene's box (results

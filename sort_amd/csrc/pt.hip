@@ -618,6 +618,7 @@ hipError_t pt_bounces(const PtLaunch& L, uint32_t npaths, hipStream_t s) {
             ta.n_trees = L.n_trees;
             ta.width = L.tree_width;
             ta.max_stack = L.tree_max_stack;
+            ta.walk_stack = L.tree_walk_stack;
         }
         if ((e = mark(0)) != hipSuccess || (e = launch_trace(ta, false, false, s, L.num_cus)) != hipSuccess ||
             (e = mark(1)) != hipSuccess)

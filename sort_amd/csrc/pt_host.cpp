@@ -187,10 +187,15 @@ int prepare_scene(sortgpu_ctx* ctx, const sortgpu_accel* acc, const sortgpu_scen
         im.tree.nodes = nullptr;
         im.tree.prims = nullptr;
         im.tree.quads = nullptr;
+        im.tree.wnodes = nullptr;
+        im.tree.wrecs = nullptr;
+        im.tree.waux = nullptr;
+        im.tree.walk_stack = with_tree ? acc->host.walk.stack : 0;
         if (with_tree) {
             im.nodes = acc->host.node_bytes;
             im.prims = acc->host.prims;
             im.quads = acc->host.quads;
+            im.walk = acc->host.walk;
         }
         im.idx = acc->idx;
         im.pos = acc->pos;
@@ -298,18 +303,23 @@ int prepare_scene(sortgpu_ctx* ctx, const sortgpu_accel* acc, const sortgpu_scen
 namespace {
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-template <class T>
-size_t vbytes(const std::vector<T>& v) {
-    return v.size() * sizeof(T);
+template <class V>
+size_t vbytes(const V& v) {
+    return v.size() * sizeof(typename V::value_type);
 }
 
 // Walks the arrays of an image in block order, calling f(host data, bytes, device pointer slot).
 template <class F>
-void for_each_array(const SceneImage& im, SceneDev& d, F f) {
+void for_each_array(const SceneImage& im, bool lean, SceneDev& d, F f) {
     if (im.with_tree) {
         f(im.nodes.data(), vbytes(im.nodes), reinterpret_cast<const void**>(&d.tree.nodes));
         f(im.prims.data(), vbytes(im.prims), reinterpret_cast<const void**>(&d.tree.prims));
         f(im.quads.data(), vbytes(im.quads), reinterpret_cast<const void**>(&d.tree.quads));
+    }
+    if (im.with_tree && !lean) {
+        f(im.walk.nodes.data(), vbytes(im.walk.nodes), reinterpret_cast<const void**>(&d.tree.wnodes));
+        f(im.walk.recs.data(), vbytes(im.walk.recs), reinterpret_cast<const void**>(&d.tree.wrecs));
+        f(im.walk.aux.data(), vbytes(im.walk.aux), reinterpret_cast<const void**>(&d.tree.waux));
     }
     f(im.idx.data(), vbytes(im.idx), reinterpret_cast<const void**>(&d.idx));
     f(im.pos.data(), vbytes(im.pos), reinterpret_cast<const void**>(&d.pos));
@@ -324,20 +334,21 @@ void for_each_array(const SceneImage& im, SceneDev& d, F f) {
 }
 }  // namespace
 
-size_t SceneImage::block_bytes() const {
+size_t SceneImage::block_bytes(bool lean) const {
     size_t total = 0;
     SceneDev d{};
-    for_each_array(*this, d, [&](const void*, size_t n, const void**) { total += align256(n); });
+    for_each_array(*this, lean, d, [&](const void*, size_t n, const void**) { total += align256(n); });
     return std::max<size_t>(total, 256);
 }
 
-int SceneImage::place(sortgpu_ctx* ctx, void* block, SceneDev& out, hipStream_t s) const {
+int SceneImage::place(sortgpu_ctx* ctx, void* block, SceneDev& out, hipStream_t s, bool lean) const {
     out = dev;
     out.tree = tree;
+    if (lean) out.tree.walk_stack = 0;
     size_t off = 0;
     hipError_t e = hipSuccess;
     char* base = static_cast<char*>(block);
-    for_each_array(*this, out, [&](const void* src, size_t n, const void** slot) {
+    for_each_array(*this, lean, out, [&](const void* src, size_t n, const void** slot) {
         *slot = nullptr;
         if (!n) return;
         *slot = base + off;

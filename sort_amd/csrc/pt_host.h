@@ -59,6 +59,7 @@ struct SceneImage {
     std::vector<unsigned char> nodes;
     std::vector<PrimRec> prims;
     std::vector<QuadRec> quads;
+    WalkTree walk;
     std::vector<uint32_t> idx, tri_mat;
     std::vector<float> pos, nrm, tan, cdf;
     std::vector<float> transp;          // 4 per primitive id when some material is transparent, else empty
@@ -66,13 +67,13 @@ struct SceneImage {
     std::vector<LightRec> lights;
     std::vector<int32_t> quad_light;
     SceneDev dev{};                     // counts and environment; pointers unset
-    // Bytes of the device block (every array 256-byte aligned).
-    size_t block_bytes() const;
+    // Bytes of the device block (every array 256-byte aligned); lean: without the walk tree.
+    size_t block_bytes(bool lean = false) const;
     // Copies the arrays into `block` (a device allocation of block_bytes()) and fills `out` with
     // their device addresses; without a tree of its own, out.tree's record pointers stay null
     // for the caller to set.
     // The copies are enqueued on `s`; the image must stay alive until they complete.
-    int place(sortgpu_ctx* ctx, void* block, SceneDev& out, hipStream_t s) const;
+    int place(sortgpu_ctx* ctx, void* block, SceneDev& out, hipStream_t s, bool lean = false) const;
 };
 
 // Validates `desc` against the accelerator's geometry and prepares the scene image (with a copy of

@@ -25,6 +25,7 @@ struct PtLaunch {
     uint32_t n_trees;
     uint32_t tree_width;        // node width of the tree table
     uint32_t tree_max_stack;    // deepest stack over the tree table
+    uint32_t tree_walk_stack;   // deepest walk-tree stack over it; 0: not every tree has one
     PathState ps;
     Queues q;
     uint32_t max_depth;         // deepest request of the wave

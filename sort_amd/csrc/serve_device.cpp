@@ -152,22 +152,28 @@ class HipDevice : public Device {
         if (sh.im.tree.max_stack > trace_max_stack_supported())
             return (err = "tree too deep for the traversal stack", SORTGPU_ERR_ARG);
         max_stack_ = std::max(max_stack_, sh.im.tree.max_stack);
+        walk_stack_ = std::max(walk_stack_, sh.im.walk.stack);
         sh.bytes = sh.im.block_bytes();
         *bytes = sh.bytes;
         scenes_.push_back(std::move(sh));
         return SORTGPU_OK;
     }
 
+    size_t lean_bytes(uint32_t id) const override {
+        return scenes_[id].im.walk.stack ? scenes_[id].im.block_bytes(true) : 0;
+    }
+    void use_lean(uint32_t id, bool lean) override { scenes_[id].lean = lean; }
+
     int load_scene(uint32_t id, std::string& err) override {
         ctx_bind(ctx_);
         SceneHost& sh = scenes_[id];
-        hipError_t e = hipMalloc(&sh.block, sh.bytes);
+        hipError_t e = hipMalloc(&sh.block, sh.lean ? sh.im.block_bytes(true) : sh.bytes);
         if (e != hipSuccess) {
             sh.block = nullptr;
             return (err = hip_msg("hipMalloc(scene)", e), hip_rc(e));
         }
         SceneDev d;
-        int rc = sh.im.place(ctx_, sh.block, d, s_up_);
+        int rc = sh.im.place(ctx_, sh.block, d, s_up_, sh.lean);
         if (rc) {
             hipStreamSynchronize(s_up_);
             hipFree(sh.block);
@@ -278,14 +284,18 @@ class HipDevice : public Device {
         if (e == hipSuccess && rc == SORTGPU_OK) {
             // a wave holding a scene with transparent materials answers its shadow rays with the
             // transparent-shadow walk (opaque scenes' rays in it get the same results as any-hit)
-            bool att = false;
-            for (const Chunk& c : w.chunks) att |= !scenes_[c.req->p.scene].im.transp.empty();
-            PtLaunch L = wave_launch(k, w.max_depth, att);
+            bool att = false, walk = true;  // walk: every scene of the wave has its walk tree here
+            for (const Chunk& c : w.chunks) {
+                const SceneHost& sh = scenes_[c.req->p.scene];
+                att |= !sh.im.transp.empty();
+                walk &= !sh.im.tree.valid || (sh.im.walk.stack != 0 && !sh.lean);
+            }
+            PtLaunch L = wave_launch(k, w.max_depth, att, walk);
             L.paths_cap = ct.total_paths;
             L.pix_cap = ct.total_pix;
             if (graphs_) {
                 hipGraphExec_t x = nullptr;
-                if ((rc = wave_graph(k, w.max_depth, att, &x)) == SORTGPU_OK) e = hipGraphLaunch(x, s);
+                if ((rc = wave_graph(k, w.max_depth, att, walk, &x)) == SORTGPU_OK) e = hipGraphLaunch(x, s);
             } else {
                 e = pt_wave_paths(L, s);
             }
@@ -369,6 +379,7 @@ class HipDevice : public Device {
     struct SceneHost {
         SceneImage im;
         size_t bytes = 0;
+        bool lean = false;  // loaded (or to be loaded) without its walk tree
         void* block = nullptr;
     };
     struct Ev {
@@ -378,7 +389,7 @@ class HipDevice : public Device {
 
     // Launch parameters of the waves of stream k: its workspace, its descriptor and its own work
     // counter (waves of one stream run one after another).
-    PtLaunch wave_launch(uint32_t k, uint32_t depth, bool att) const {
+    PtLaunch wave_launch(uint32_t k, uint32_t depth, bool att, bool walk) const {
         PtLaunch L;
         std::memset(&L, 0, sizeof(L));
         L.trace.counter = d_counters_ + k * kCounterStride;
@@ -390,6 +401,7 @@ class HipDevice : public Device {
         L.n_trees = max_scenes_;
         L.tree_width = width_ ? width_ : 8;
         L.tree_max_stack = max_stack_;
+        L.tree_walk_stack = walk ? walk_stack_ : 0;
         L.ps = ws_[k].ps;
         L.q = ws_[k].q;
         L.max_depth = depth;
@@ -403,24 +415,25 @@ class HipDevice : public Device {
     // sized for the workspace's capacity; the kernels read the wave's exact counts from its
     // descriptor). Captured on first use per depth, again when a scene changes the tree table's
     // width or stack depth or the context's tuning changes. The graph holds kernel launches only.
-    int wave_graph(uint32_t k, uint32_t depth, bool att, hipGraphExec_t* out) {
+    int wave_graph(uint32_t k, uint32_t depth, bool att, bool walk, hipGraphExec_t* out) {
         GraphKey key;
         std::memset(&key, 0, sizeof(key));
         key.tuning = ctx_->tuning;
         key.width = width_;
         key.max_stack = max_stack_;
+        key.walk_stack = walk_stack_;
         if (std::memcmp(&key, &graph_key_, sizeof(key)) != 0) {
             drop_graphs();
             graph_key_ = key;
         }
-        const uint32_t gk = 2 * depth + (att ? 1u : 0u);
+        const uint32_t gk = 4 * depth + (walk ? 2u : 0u) + (att ? 1u : 0u);
         auto it = gexec_[k].find(gk);
         if (it != gexec_[k].end()) {
             *out = it->second;
             return SORTGPU_OK;
         }
         hipStream_t s = s_[k];
-        PtLaunch L = wave_launch(k, depth, att);
+        PtLaunch L = wave_launch(k, depth, att, walk);
         L.paths_cap = cap_;
         L.pix_cap = cap_;
         hipGraph_t g = nullptr;
@@ -471,10 +484,10 @@ class HipDevice : public Device {
     uint32_t cap_, max_scenes_, ns_;
     bool graphs_;
     WaveDesc* d_desc_[kMaxStreams] = {};
-    std::map<uint32_t, hipGraphExec_t> gexec_[kMaxStreams];  // key: 2 * depth + transparent-shadow form
+    std::map<uint32_t, hipGraphExec_t> gexec_[kMaxStreams];  // key: 4 * depth + 2 * walk-tree form + transparent-shadow form
     struct GraphKey {  // what a captured wave graph bakes in besides the depth
         sortgpu_tuning tuning;
-        uint32_t width, max_stack;
+        uint32_t width, max_stack, walk_stack;
     };
     GraphKey graph_key_{};
     hipStream_t s_[kMaxStreams] = {};
@@ -493,7 +506,7 @@ class HipDevice : public Device {
     uint32_t* d_error_ = nullptr;
     uint32_t slot_ = 0;
     std::vector<SceneHost> scenes_;
-    uint32_t width_ = 0, max_stack_ = 1;
+    uint32_t width_ = 0, max_stack_ = 1, walk_stack_ = 0;
     std::mutex ev_mu_;  // guards evs_, spare_ and wave_us_ (the blocking wait runs unlocked)
     std::deque<Ev> evs_;
     std::vector<hipEvent_t> spare_;

@@ -308,7 +308,7 @@ bool Engine::evict_for(size_t need, uint32_t keep_scene) {
         if (victim < 0) return false;
         dev_->unload_scene((uint32_t)victim);
         scenes_[victim].resident = false;
-        used_ -= scenes_[victim].bytes;
+        used_ -= scenes_[victim].held;
         n_evict_++;
     }
     return true;
@@ -321,25 +321,34 @@ void Engine::admit() {
     while (!queue_.empty() && active_.size() < o_.max_active) {
         Request* r = queue_.front();
         SceneState& s = scenes_[r->p.scene];
-        const size_t need = (s.resident ? 0 : s.bytes) + r->film_bytes;
+        size_t need = (s.resident ? 0 : s.bytes) + r->film_bytes;
+        bool lean = false;
         if (!evict_for(need, r->p.scene)) {
-            if (active_.empty() && inflight_.empty()) {
+            // the whole budget is not enough for it: its smaller form, if that fits
+            const size_t small = s.resident ? 0 : dev_->lean_bytes(r->p.scene);
+            if (active_.empty() && inflight_.empty() && small && evict_for(small + r->film_bytes, r->p.scene)) {
+                lean = true;
+            } else if (active_.empty() && inflight_.empty()) {
                 finish(r, SORTGPU_REQ_FAILED, SORTGPU_ERR_BUDGET,
                        "needs " + std::to_string(need) + " bytes; the HBM budget is " + std::to_string(o_.budget) +
                            " with " + std::to_string(used_) + " in use");
                 continue;
+            } else {
+                return;
             }
-            return;
         }
         std::string err;
         int rc;
         if (!s.resident) {
-            if ((rc = reserve(s.bytes, err)) || (rc = dev_->load_scene(r->p.scene, err))) {
+            const size_t bytes = lean ? dev_->lean_bytes(r->p.scene) : s.bytes;
+            dev_->use_lean(r->p.scene, lean);
+            if ((rc = reserve(bytes, err)) || (rc = dev_->load_scene(r->p.scene, err))) {
                 finish(r, SORTGPU_REQ_FAILED, rc, "scene load failed: " + err);
                 continue;
             }
             s.resident = true;
-            used_ += s.bytes;
+            s.held = bytes;
+            used_ += bytes;
             n_loads_++;
         }
         if ((rc = reserve(r->film_bytes, err)) || (rc = dev_->alloc_film(*r, err))) {

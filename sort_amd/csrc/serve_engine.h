@@ -67,6 +67,10 @@ class Device {
     // Host-side registration; returns the HBM bytes the scene takes when resident.
     virtual int add_scene(const sortgpu_accel* acc, const sortgpu_scene_desc* desc, uint32_t id, size_t* bytes,
                           std::string& err) = 0;
+    // Bytes of the scene's smaller form, without what only makes its traversal faster (0: there is
+    // none), and whether the next load_scene loads that form.
+    virtual size_t lean_bytes(uint32_t) const { return 0; }
+    virtual void use_lean(uint32_t, bool) {}
     virtual int load_scene(uint32_t id, std::string& err) = 0;
     virtual void unload_scene(uint32_t id) = 0;
     virtual int alloc_film(Request& r, std::string& err) = 0;  // zeroed; sets r.film
@@ -109,6 +113,7 @@ class Engine {
   private:
     struct SceneState {
         size_t bytes = 0;
+        size_t held = 0;         // bytes it was loaded with
         bool resident = false;
         uint32_t refs = 0;       // active requests on it
         uint64_t lru = 0;

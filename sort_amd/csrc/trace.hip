@@ -471,6 +471,9 @@ static hipError_t launch_w(const TraceArgs& a, bool any, bool stats, hipStream_t
 hipError_t launch_trace(const TraceArgs& a, bool any, bool stats, hipStream_t stream, int num_cus) {
     if (a.n == 0) return hipSuccess;
     const bool multi = a.trees != nullptr;
+    // (a walk launch's counter runs up to a few million past n: no such batch may wrap it)
+    if (!stats && (multi ? a.walk_stack : a.tree.walk_stack) && a.n <= 0xf0000000u)
+        return launch_walk(a, any, stream, num_cus);
     const uint32_t width = multi ? a.width : a.tree.width;
     if (width == 8) return multi ? launch_w<8, true>(a, any, stats, stream, num_cus)
                                  : launch_w<8, false>(a, any, stats, stream, num_cus);

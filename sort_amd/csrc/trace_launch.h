@@ -22,6 +22,7 @@ struct TraceArgs {
     uint32_t n_trees;
     uint32_t width;                // node width shared by every tree of the table
     uint32_t max_stack;            // deepest worst-case stack over the table
+    uint32_t walk_stack;           // deepest walk-tree stack over the table; 0: not every tree has one
     // tuning (0 = default)
     uint32_t refill;               // idle lanes that trigger a refill (default 16)
     uint32_t lds_entries;          // LDS stack entries per lane: 8 or 16 (default 16)
@@ -47,8 +48,10 @@ struct TraceArgs {
     float4* occ_rec = nullptr;
 };
 
-// Launches the closest (any = false) or any-hit traversal on `stream`.
+// Launches the closest (any = false) or any-hit traversal on `stream`: through the walk trees where
+// every tree has one, else (and for the statistics) through the Fast-BVH.
 hipError_t launch_trace(const TraceArgs& a, bool any, bool stats, hipStream_t stream, int num_cus);
+hipError_t launch_walk(const TraceArgs& a, bool any, hipStream_t stream, int num_cus);  // walk.hip
 // Launches the transparent-shadow attenuation walk (single tree with a.transp, or the multi-scene
 // form with a.trees and a.transps): out receives one float4 per ray (attenuation r, g, b, and the
 // number of surfaces passed as a float), at stride a.out_stride.

@@ -1,0 +1,58 @@
+// Host builder of the walk tree (layout.h WalkNode), derived from the finished Fast-BVH.
+//
+// The Fast-BVH decides what a query returns: which leaves a ray may take hits from and which of two
+// equal hits wins. The walk tree only finds candidates, so its shape is free. It keeps the
+// Fast-BVH's upper splits (each node's children arranged as a binary tree by surface area), goes
+// on splitting inside its leaves down to two triangles, and folds the binary tree into 4-wide nodes,
+// opening the largest child first.
+#pragma once
+#include <stdint.h>
+#include <memory>
+#include <vector>
+
+#include "layout.h"
+
+namespace sortgpu {
+
+// One primitive as the Fast-BVH build leaves it (in its primitive order).
+struct BuildPrim {
+    float mn[3];
+    float mx[3];
+    float c[3];  // centroid
+    uint32_t id;
+};
+
+// A Fast-BVH node: primitives [off, off + cnt); children are src[first .. first + nchild), after
+// their parent; a leaf has none.
+struct SrcNode {
+    uint32_t off, cnt, first, nchild;
+};
+
+// Vectors whose resize() leaves new elements unset: the builder's threads fill them, and touching
+// 70 MB for a million triangles on one thread first would cost as much as the rest of the build.
+template <class T> struct Unset : std::allocator<T> {
+    template <class U> struct rebind { using other = Unset<U>; };
+    template <class U> void construct(U* p) noexcept { ::new (static_cast<void*>(p)) U; }
+    template <class U, class... A> void construct(U* p, A&&... a) { ::new (static_cast<void*>(p)) U(std::forward<A>(a)...); }
+};
+template <class T> using RawVec = std::vector<T, Unset<T>>;
+
+struct WalkTree {
+    RawVec<WalkNode> nodes;
+    RawVec<PrimRec> recs;
+    RawVec<WalkAux> aux;
+    uint32_t stack = 0;  // most stack entries a traversal holds (0: no walk tree)
+};
+
+struct BuildInput;
+
+// Deepest walk-tree traversal stack the kernels hold (walk.hip).
+constexpr uint32_t kWalkMaxStack = 8 + 256;
+
+// Leaves `out` empty when the tree cannot have a walk tree: boxes not finite or past 1e12 (the
+// kernel's error bounds need finite products), far smaller than their distance from the origin
+// (its padding would swallow them), records past 4 GiB, or a deeper stack than kWalkMaxStack.
+void build_walk_tree(const BuildInput& in, const std::vector<BuildPrim>& prims, const std::vector<SrcNode>& src,
+                     const float bbox[6], unsigned threads, WalkTree& out);
+
+}  // namespace sortgpu

@@ -1,0 +1,172 @@
+"""Closest and any hit through the walk tree against the oracle, bit for bit, where its candidates and
+the Fast-BVH's rules are hardest to keep together: equal hits (doubled triangles, coplanar overlaps,
+rays through shared vertices and edges), leaf boxes without thickness, rays along the axes, scenes far
+from the origin, origins far from the scene, directions and windows at the edge of what the walk tree
+takes, trees of one to a few records, and depth-limited leaves of hundreds of primitives."""
+import numpy as np
+import pytest
+import torch
+
+from oracle.oracle import OracleBvh
+from sort_amd import MISS, Obvh, Qbvh, batch, scenes
+
+pytestmark = pytest.mark.gpu
+
+FLT_MAX = np.float32(3.4028234663852886e38)
+
+
+def _doubled(g):
+    """A soup, every triangle again as it is, turned around, or starting at another vertex."""
+    pos, _ = scenes.soup(1500, seed=5)
+    t = pos.reshape(-1, 3, 3) * np.float32(1.0)
+    c = t.mean(axis=1, keepdims=True)
+    t = (c + (t - c) * np.float32(8.0)).astype(np.float32)
+    order = np.array([[0, 1, 2], [0, 2, 1], [1, 2, 0]])[g.integers(0, 3, len(t))]
+    t = np.concatenate([t, np.take_along_axis(t, order[:, :, None], axis=1)])
+    return scenes.tris_to_mesh(list(t[g.permutation(len(t))])), None
+
+
+def _grid(g, n=24, axis=2):
+    """Two parallel sheets of axis-aligned squares with shared corners at multiples of 1/n."""
+    tris = []
+    for z in (0.25, 0.75):
+        for i in range(n):
+            for j in range(n):
+                p = [(i / n, j / n, z), ((i + 1) / n, j / n, z), ((i + 1) / n, (j + 1) / n, z), (i / n, (j + 1) / n, z)]
+                p = [tuple(np.roll(q, axis - 2)) for q in p]
+                tris += [np.array([p[0], p[1], p[2]], np.float32), np.array([p[0], p[2], p[3]], np.float32)]
+    return scenes.tris_to_mesh(tris), None
+
+
+def _overlap(g):
+    """Coplanar triangles of all sizes on one plane, over one another, with quad lights on it too."""
+    t = g.uniform(0.0, 1.0, (600, 3, 3)).astype(np.float32)
+    t[:, 1:] = t[:, :1] + (t[:, 1:] - np.float32(0.5)) * np.exp(g.uniform(-4, 0, (600, 1, 1))).astype(np.float32)
+    t[:, :, 1] = np.float32(0.5)
+    quads = [scenes.translate_quad((float(x), 0.5, float(z)), 0.2) for x, z in g.uniform(0.2, 0.8, (4, 2))]
+    return scenes.tris_to_mesh(list(t)), quads
+
+
+def _rays(g, n, mesh):
+    """Random rays, rays along the axes, and rays aimed at vertices and edge midpoints."""
+    pos = mesh[0]
+    lo, hi = pos.min(axis=0), pos.max(axis=0)
+    ext = np.float32(max(float((hi - lo).max()), 1e-3))
+    o = (lo + (hi - lo) * g.uniform(-0.4, 1.4, (n, 3)) + ext * g.normal(0, 0.3, (n, 3))).astype(np.float32)
+    d = g.normal(size=(n, 3)).astype(np.float32)
+    k = np.arange(n)
+    v = pos[g.integers(0, len(pos), n)]
+    w = pos[(g.integers(0, len(pos) // 3, n) * 3)[:, None] + np.array([0, 1])].mean(axis=1).astype(np.float32)
+    d = np.where((k % 4 == 1)[:, None], v - o, np.where((k % 4 == 2)[:, None], w - o, d)).astype(np.float32)
+    ax = k % 4 == 3
+    d[ax] = 0
+    d[ax, k[ax] // 4 % 3] = np.where(k[ax] // 12 % 2, 1.0, -1.0)
+    on = ax & (k % 8 == 7)  # through a vertex, along an axis
+    o[on] = (v - 2 * ext * d)[on]
+    d[k % 16 == 5] *= np.float32(3.0)
+    return o, d
+
+
+SCENES = {"doubled": _doubled, "grid z": _grid, "grid x": lambda g: _grid(g, axis=0), "overlap": _overlap}
+
+
+def _check(acc, ob, rays, label):
+    print(f"[walk] {label} width={acc.width} rays={len(rays)}", flush=True)
+    d = torch.from_numpy(np.ascontiguousarray(rays)).cuda()
+    hits, occ = acc.get_intersect(d).cpu().numpy(), acc.is_occluded(d).cpu().numpy()
+    ref, ref_occ = ob.closest(rays, threads=16), ob.occluded(rays, threads=16)
+    bad = np.nonzero(np.any(hits.view(np.uint32) != ref.view(np.uint32), axis=1))[0]
+    assert bad.size == 0, f"{label}: {bad.size} closest differ, ray {rays[bad[0]]}: {hits[bad[0]]} {ref[bad[0]]}"
+    assert np.array_equal(occ, ref_occ), label
+    acc.check_errors()
+    return hits
+
+
+def _build(ctx, width, mesh, quads, **kw):
+    acc = (Obvh if width == 8 else Qbvh)(ctx, **kw).build(mesh[0], mesh[1], quads)
+    return acc, OracleBvh(mesh[0], mesh[1], quads, width=width, max_depth=kw.get("max_node_depth", 28),
+                          max_leaf=kw.get("max_pri_in_leaf", 16))
+
+
+@pytest.mark.parametrize("width", [8, 4])
+@pytest.mark.parametrize("scene", list(SCENES))
+def test_ties_flat_boxes_and_axis_rays(gpu_ctx, width, scene):
+    g = np.random.default_rng(len(scene) + width)
+    mesh, quads = SCENES[scene](g)
+    for kw in ({}, {"max_node_depth": 3}, {"max_pri_in_leaf": 1}):
+        acc, ob = _build(gpu_ctx, width, mesh, quads, **kw)
+        o, d = _rays(g, 12000, mesh)
+        hits = _check(acc, ob, scenes.make_rays(o, d, 0.0, FLT_MAX), f"{scene} {kw}")
+        assert np.mean(hits[:, 1].view(np.uint32) != MISS) > 0.1
+        tmin = g.uniform(0, 0.5, len(o)).astype(np.float32)
+        _check(acc, ob, scenes.make_rays(o, d, tmin, tmin + g.uniform(0, 1, len(o)).astype(np.float32)), "windowed")
+
+
+@pytest.mark.parametrize("width", [8, 4])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 8, 9, 16, 17, 33])
+def test_few_triangles(gpu_ctx, width, n):
+    g = np.random.default_rng(n)
+    mesh = scenes.tris_to_mesh(list(g.uniform(0, 1, (n, 3, 3)).astype(np.float32)))
+    acc, ob = _build(gpu_ctx, width, mesh, [scenes.translate_quad((0.5, 1.2, 0.5), 0.5)] if n % 2 else None)
+    _check(acc, ob, scenes.make_rays(*_rays(g, 3000, mesh), 0.0, FLT_MAX), f"{n} triangles")
+
+
+@pytest.mark.parametrize("shift,scale,away", [(0.0, 1.0, 50.0), (1000.0, 1.0, 0.0), (3e4, 1.0, 0.0), (0.0, 1e-4, 0.0),
+                                              (0.0, 1e6, 0.0), (0.0, 1.0, 1e5), (0.0, 1e9, 0.0)])
+def test_far_scenes_and_origins(gpu_ctx, shift, scale, away):
+    """A scene past the origin by more than 4,096 times its size has no walk tree, and an origin as far
+    out leaves it; short of that both use it."""
+    g = np.random.default_rng(9)
+    pos, idx = scenes.soup(3000, seed=8)
+    t = pos.reshape(-1, 3, 3)
+    c = t.mean(axis=1, keepdims=True)
+    t = ((c + (t - c) * 10) * scale + shift).astype(np.float32)
+    mesh = scenes.tris_to_mesh(list(t))
+    acc, ob = _build(gpu_ctx, 8, mesh, None)
+    o, d = _rays(g, 8000, mesh)
+    if away:
+        target = mesh[0][g.integers(0, len(mesh[0]), len(o))]
+        d = (target - o).astype(np.float32)
+        d /= np.linalg.norm(d, axis=1, keepdims=True)
+        o = (target - np.float32(away) * d).astype(np.float32)
+    _check(acc, ob, scenes.make_rays(o, d, 0.0, FLT_MAX), f"shift {shift} scale {scale} away {away}")
+
+
+@pytest.mark.parametrize("lds", [8, 16])
+def test_windows_directions_and_pool(gpu_ctx, lds):
+    """Negative, infinite and empty windows, directions from 1e-14 to 1e14 long, zero and near-zero
+    components, mixed among ordinary rays; the same rays against three scenes of a pool at once."""
+    g = np.random.default_rng(3)
+    pos, idx = scenes.soup(4000, seed=21)
+    t = pos.reshape(-1, 3, 3)
+    c = t.mean(axis=1, keepdims=True)
+    mesh = scenes.tris_to_mesh(list((c + (t - c) * 6).astype(np.float32)))
+    acc, ob = _build(gpu_ctx, 8, mesh, None)
+    o, d = _rays(g, 16384, mesh)
+    k = np.arange(len(o))
+    r = scenes.make_rays(o, d, 0.0, FLT_MAX)
+    r[k % 16 == 0, 3] = np.float32(-0.5)
+    r[k % 16 == 1, 3] = np.float32(-2.0)
+    r[k % 16 == 2, 7] = np.inf
+    r[k % 16 == 3, 7] = np.float32(-1.0)
+    r[k % 16 == 4, 3] = np.float32(-0.0)
+    r[k % 16 == 6, 4:7] *= np.float32(1e-14)
+    r[k % 16 == 8, 4:7] *= np.float32(1e14)
+    r[k % 16 == 9, 4:7] *= np.float32(1e-4)
+    r[k % 16 == 10, 4] = np.float32(2e-6)
+    r[k % 16 == 11, 5:7] *= np.float32(1e-7)
+    try:
+        batch.set_tuning(gpu_ctx, lds_entries=lds)
+        hits = _check(acc, ob, r, f"windows lds {lds}")
+        accs = [acc] + [Obvh(gpu_ctx).build(*scenes.soup(n, seed=n)) for n in (700, 40)]
+        pool = batch.Pool(gpu_ctx, accs)
+        sid = (k % 3).astype(np.int32)
+        got = pool.trace(torch.from_numpy(r).cuda(), torch.from_numpy(sid).cuda()).cpu().numpy()
+        pool.check_errors()
+    finally:
+        batch.set_tuning(gpu_ctx)
+    assert np.array_equal(got[sid == 0].view(np.uint32), hits[sid == 0].view(np.uint32))
+    for i in (1, 2):
+        one = accs[i].get_intersect(torch.from_numpy(r).cuda()).cpu().numpy()
+        assert np.array_equal(got[sid == i].view(np.uint32), one[sid == i].view(np.uint32))
+    pool.close()

@@ -223,8 +223,9 @@ int sortgpu_accel_errors(sortgpu_accel* accel, void* stream, uint32_t* flags);
  * idle lanes of a wave that trigger refilling them with new rays from the work queue (default 16,
  * 1..64); lds_entries = traversal-stack entries per lane kept in LDS (8 or 16,
  * default 16); blocks_per_cu = cap on resident workgroups per CU (default: occupancy limit);
- * leaf_batch = lanes of a wave holding a leaf that end a node-walking phase (default 16 for closest
- * and any hit, 32 for transparent shadows and trees without a walk tree; 1..64);
+ * leaf_batch = lanes of a wave holding a leaf that end a node-walking phase (default 24 of 64 lanes at
+ * work, in proportion of fewer, for closest and any hit; 32 for transparent shadows and trees without
+ * a walk tree; 1..64);
  * leaf_min = a leaf-testing phase ends when fewer lanes hold a leaf (default 1, 1..64; transparent
  * shadows and trees without a walk tree only);
  * reorder = traversal order of sortgpu_trace_closest / _any / _attenuation / _multi and

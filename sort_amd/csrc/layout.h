@@ -66,7 +66,9 @@ static_assert(sizeof(QuadRec) == 80, "QuadRec must be 80 B");
 // slot is one record of at most two triangles, or one quad.
 //
 // Slots: inner children first (node indices child_base + slot), then leaves (record indices
-// rec_base + slot - inner count), then unused slots. Plane q of an axis lies at base + q * 2^(e - 127).
+// rec_base + slot - inner count), then unused slots: their box is the node's far corner alone, and a
+// ray that meets it tests a record of another node, which does no harm (kWalkPadRecs empty records
+// end the array). Plane q of an axis lies at base + q * 2^(e - 127).
 struct alignas(16) WalkNode {
     float base[3];
     uint8_t exp[3];       // biased exponent e of the grid step per axis
@@ -76,6 +78,8 @@ struct alignas(16) WalkNode {
     uint8_t lo_x[4], hi_x[4], lo_y[4], hi_y[4], lo_z[4], hi_z[4];
 };
 static_assert(sizeof(WalkNode) == 48, "WalkNode must be 48 B");
+
+constexpr uint32_t kWalkPadRecs = 4;
 
 // Beside each walk record: the box of the Fast-BVH leaf that holds its primitives, as its parent
 // node's planes bound it, that leaf's number, and the places of A and B among the leaf's primitives

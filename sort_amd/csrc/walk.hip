@@ -150,6 +150,21 @@ __device__ __forceinline__ void load_ray(const void* rays, uint32_t i, RayK& r) 
     r.dx = q1.x; r.dy = q1.y; r.dz = q1.z; r.tmax = q1.w;
 }
 
+constexpr float FLT_INF = __builtin_inff();
+
+// Three floats at any word, as one load.
+struct __attribute__((packed, aligned(4))) Float3 {
+    float x, y, z;
+};
+
+// The value of the even lane of this lane's pair; the value of the pair's other lane.
+__device__ __forceinline__ uint32_t quad_even(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xA0, 0xf, 0xf, true);  // quad_perm [0, 0, 2, 2]
+}
+__device__ __forceinline__ float quad_swap(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, true));  // [1, 0, 3, 2]
+}
+
 struct Best {
     float t, u, v;
     uint32_t prim;  // kNone: nothing found
@@ -231,7 +246,8 @@ __device__ __forceinline__ void exact_walk(const TreeView& tv, RayK& r, uint2* s
 }
 
 template <bool ANY, bool MULTI, int LDS, int SPILL>
-__global__ __launch_bounds__(kBlock) void k_walk(TraceArgs a) {
+// 4 waves per SIMD (128 VGPRs): 5 spilled in the rarely taken parts and gained nothing.
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_walk(TraceArgs a) {
     __shared__ uint2 s_st[LDS * kBlock];  // (reference, entry distance), [entry][thread]
     constexpr int CAP = LDS + SPILL;
     uint2 sp_st[SPILL];  // deeper entries; also the stack of exact_walk, whose lane has none of its own left
@@ -240,35 +256,49 @@ __global__ __launch_bounds__(kBlock) void k_walk(TraceArgs a) {
     const uint32_t lane = __lane_id();
     const uint32_t n_rays = a.n_dev ? *a.n_dev : a.n;
     const uint32_t refill = a.refill ? a.refill : 16u;
-    const uint32_t leaf_batch = a.leaf_batch ? a.leaf_batch : 16u;
+    const uint32_t leaf_batch = a.leaf_batch ? a.leaf_batch : 24u;
     const WalkNode* __restrict__ nodes = a.tree.wnodes;
     const PrimRec* __restrict__ recs = a.tree.wrecs;
 
     RayK r;
     Slabs s;
-    uint32_t cur = kNone;  // node or leaf to visit next; kNone: pop the stack
+    uint32_t cur = kNone;   // node to visit next (or the next leaf, while `leaf` is taken); kNone: pop the stack
+    uint32_t leaf = kNone;  // leaf waiting for the wave's leaf phase
     uint32_t ray_id = kNone;
     uint32_t hit = kNone;  // nearest candidate: record * 2 + (0: A or the quad, 1: B)
     float bt = FLT_MAX, bu = 0.f, bv = 0.f;
-    float lim = FLT_MAX;     // search bound: bt and the slack above it
+    float lim = FLT_MAX;     // search bound: the window's end, then bt and the slack above it
     float second = FLT_MAX;  // second nearest distance met
     float slack = 0.f;
     int sp = 0;
     bool more = true, overflow = false, open = false;  // open: exact_walk has to answer
-    // Rays are handed to a wave `chunk` at a time, [own, own_end) still to be started: one atomic on
-    // the launch's counter takes about 8.5 ns of the whole chip's time.
-    const uint32_t chunk = min(max(n_rays / (gridDim.x * (kBlock / 64) * 8u), 64u), 512u);
-    uint32_t own = 0, own_end = 0;
+    // Handing out the rays. One atomic on the launch's counter takes about 8.5 ns of the whole chip's
+    // time (measured: 4.19M rays, 16 at a time, spent 2.2 ms there), so every workgroup has a share of
+    // its own that its waves take from through LDS. Of a large batch only three quarters are shares,
+    // dealt 64 rays at a time so that all workgroups move through the order together (a contiguous
+    // share each has them all over the tree at once: 2.05 instead of 1.87 ms for 4.19M
+    // bounce rays); the rest goes out
+    // through the counter, in chunks that shrink with what is left, so that the workgroups end
+    // together. A batch with less than a full wave of rays for each wave spreads over all of them, on
+    // the first `seats` lanes of each.
+    const uint32_t waves = gridDim.x * (kBlock / 64);
+    const uint32_t seats = min((n_rays + waves - 1) / waves, 64u);
+    const bool dealt = n_rays >= 128u * waves;
+    const uint32_t share = dealt ? (n_rays - n_rays / 4u) / (gridDim.x * 64u) * 64u : (n_rays + gridDim.x - 1) / gridDim.x;
+    const uint32_t pooled = min(share * gridDim.x, n_rays);  // first ray that the counter hands out
+    __shared__ uint32_t s_next, s_out;  // rays of the share taken; whether the counter has run out
+    if (tid == 0) {
+        s_next = 0;
+        s_out = pooled >= n_rays ? 1u : 0u;
+    }
+    __syncthreads();
+    bool sharing = true;             // the share may have rays left
+    uint32_t own = 0, own_end = 0;   // this wave's chunk of the rest
+    more = lane < seats;
 
-    auto push = [&](uint32_t ref, uint32_t t) {
-        if (sp < LDS) s_st[sp * kBlock + tid] = make_uint2(ref, t);
-        else if (sp < CAP) sp_st[sp - LDS] = make_uint2(ref, t);
-        else overflow = true;
-        sp++;
-    };
 
     while (true) {
-        const bool idle = cur == kNone && sp == 0;
+        const bool idle = cur == kNone && leaf == kNone && sp == 0;
         const uint64_t want = __ballot(idle && (more || ray_id != kNone));
         const uint64_t busy = __ballot(!idle);
         if (want == 0 && busy == 0) break;
@@ -327,25 +357,45 @@ __global__ __launch_bounds__(kBlock) void k_walk(TraceArgs a) {
             // ---- take new ones ----
             const uint64_t take = __ballot(idle && more);
             if (take != 0) {
-                const uint32_t cnt = (uint32_t)__popcll(take), left = own_end - own;
-                uint32_t next = 0;
-                if (cnt > left) {
-                    if (lane == 0) next = atomicAdd(a.counter, chunk);
-                    next = __builtin_amdgcn_readfirstlane(next);
-                }
+                const uint32_t cnt = (uint32_t)__popcll(take);
                 const uint32_t rank = (uint32_t)__popcll(take & ((1ull << lane) - 1ull));
-                const uint32_t k = rank < left ? own + rank : next + (rank - left);
-                if (cnt > left) {
-                    own = next + (cnt - left);
-                    own_end = next + chunk;
+                uint32_t k = 0;
+                bool given = false, out = false;  // a lane without a ray waits for the next refill; out: there is none
+                if (sharing) {
+                    uint32_t v = 0;
+                    if (lane == 0) v = atomicAdd(&s_next, cnt);
+                    v = __builtin_amdgcn_readfirstlane(v);
+                    sharing = v + cnt < share;
+                    v += rank;
+                    k = dealt ? ((((v >> 6) * gridDim.x + blockIdx.x) << 6) | (v & 63u)) : blockIdx.x * share + v;
+                    given = v < share && k < pooled;
                 } else {
-                    own += cnt;
+                    if (own == own_end) {
+                        uint32_t done = 0;
+                        if (lane == 0) done = __hip_atomic_load(&s_out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        out = __builtin_amdgcn_readfirstlane(done) != 0;
+                        if (!out) {
+                            const uint32_t rest = n_rays - max(own_end, pooled);
+                            const uint32_t chunk = max(min(rest / (2u * waves), 256u), 32u);
+                            if (lane == 0) own = atomicAdd(a.counter, chunk);
+                            own = pooled + __builtin_amdgcn_readfirstlane(own);
+                            own_end = min(own + chunk, n_rays);
+                            out = own >= n_rays;
+                            if (out && lane == 0)
+                                __hip_atomic_store(&s_out, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        }
+                    }
+                    k = own + rank;
+                    given = k < own_end;
+                    own = min(own + cnt, own_end);
                 }
+                if (out) more = false;
                 if (idle && more) {
-                    if (k < n_rays) {
+                    if (given) {
                         const uint32_t my = a.order ? a.order[k] : k;
                         load_ray(a.rays, my, r);
-                        bt = lim = second = FLT_MAX;
+                        bt = second = FLT_MAX;
+                        lim = r.tmax;
                         bu = bv = 0.f;
                         hit = kNone;
                         open = false;
@@ -371,29 +421,41 @@ __global__ __launch_bounds__(kBlock) void k_walk(TraceArgs a) {
                         } else if (!a.occ_slot) {
                             static_cast<uint8_t*>(a.out)[my] = 0;
                         }
-                    } else {
-                        more = false;
                     }
                 }
             }
             continue;
         }
-        // ---- node phase: lanes that hold no leaf step through inner nodes ----
+        // ---- node phase: lanes step through inner nodes; the first leaf that one meets waits while it
+        // walks on, the second stops it ----
+        // `leaf_batch` of 64 lanes at work, in proportion of fewer (a fixed number has a thinly filled
+        // wave walk on and on past the leaves that would have ended its rays: 1.87 -> 1.74 ms for 4.19M
+        // bounce rays, 0.47 -> 0.44 for 2.07M camera rays)
+        const uint32_t batch = (leaf_batch * (uint32_t)__popcll(busy) + 63u) / 64u;
         while (true) {
             const bool walk = (int32_t)cur >= 0 || (cur == kNone && sp > 0);
-            if (__ballot(walk) == 0 || (uint32_t)__popcll(__ballot(cur != kNone && (int32_t)cur < 0)) >= leaf_batch) break;
-            if (walk && cur == kNone) {
+            if (__ballot(walk) == 0 || (uint32_t)__popcll(__ballot(leaf != kNone)) >= batch) break;
+            const bool pop = walk && cur == kNone;
+            // Stack accesses are LDS ones unless some lane of the wave is past the entries there: a
+            // choice per lane would make every access a generic one.
+            if (__ballot(pop && sp > LDS) == 0) {
+                if (pop) {
+                    --sp;
+                    const uint2 e = s_st[sp * kBlock + tid];
+                    if (__uint_as_float(e.y) <= lim) cur = e.x;
+                }
+            } else if (pop) {
                 --sp;
-                // the LDS read is unconditional (clamped index) so that it stays an LDS access
-                uint2 e = s_st[(sp < LDS ? sp : LDS - 1) * kBlock + tid];
-                if (sp >= LDS) e = sp_st[sp - LDS < SPILL ? sp - LDS : 0];
+                uint2 e;
+                if (sp < LDS) e = s_st[sp * kBlock + tid];
+                else e = sp_st[min(sp - LDS, SPILL - 1)];
                 if (__uint_as_float(e.y) <= lim) cur = e.x;
             }
             if (walk && (int32_t)cur >= 0) {
-                const uint4* np = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(nodes) + cur * 48u);
+                const uint4* np = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(nodes) + (((cur << 1) + cur) << 4));
                 const uint4 q0 = np[0], q1 = np[1], q2 = np[2];
                 const uint32_t meta = q0.w;
-                const uint32_t ni = (meta >> 24) & 15u, nc = meta >> 28;
+                const uint32_t ni = (meta >> 24) & 15u;
                 const float gx = __uint_as_float((meta & 0xffu) << 23) * s.rx;
                 const float gy = __uint_as_float(((meta >> 8) & 0xffu) << 23) * s.ry;
                 const float gz = __uint_as_float(((meta >> 16) & 0xffu) << 23) * s.rz;
@@ -405,7 +467,6 @@ __global__ __launch_bounds__(kBlock) void k_walk(TraceArgs a) {
                 const uint32_t wnx = px ? q1.z : q1.w, wfx = px ? q1.w : q1.z;
                 const uint32_t wny = py ? q2.x : q2.y, wfy = py ? q2.y : q2.x;
                 const uint32_t wnz = pz ? q2.z : q2.w, wfz = pz ? q2.w : q2.z;
-                const float hi = fminf(r.tmax, lim);
                 uint32_t key[4];
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
@@ -413,10 +474,9 @@ __global__ __launch_bounds__(kBlock) void k_walk(TraceArgs a) {
                     const float t0 = fmaxf(fmaxf(__builtin_fmaf(q(wnx), gx, nx), __builtin_fmaf(q(wny), gy, ny)),
                                            fmaxf(__builtin_fmaf(q(wnz), gz, nz), r.tmin));
                     const float t1 = fminf(fminf(__builtin_fmaf(q(wfx), gx, fx), __builtin_fmaf(q(wfy), gy, fy)),
-                                           fminf(__builtin_fmaf(q(wfz), gz, fz), hi));
+                                           fminf(__builtin_fmaf(q(wfz), gz, fz), lim));
                     // distances are not negative: their bits order as they do; the slot rides in the last two
-                    const bool in = (t0 <= t1) & ((uint32_t)j < nc);
-                    key[j] = in ? ((__float_as_uint(t0) & ~3u) | (uint32_t)j) : kNone;
+                    key[j] = t0 <= t1 ? ((__float_as_uint(t0) & ~3u) | (uint32_t)j) : kNone;
                 }
                 const uint32_t leaf_at = (q1.y | REF_LEAF) - ni;
                 auto ref = [&](uint32_t k) {
@@ -433,64 +493,138 @@ __global__ __launch_bounds__(kBlock) void k_walk(TraceArgs a) {
                 order(key[0], key[2]);
                 order(key[1], key[3]);
                 order(key[1], key[2]);
-                if (key[3] != kNone) push(ref(key[3]), key[3]);
-                if (key[2] != kNone) push(ref(key[2]), key[2]);
-                if (key[1] != kNone) push(ref(key[1]), key[1]);
+                // Farthest first. An entry that is no hit is written as well and then written over:
+                // the slot above the top is free.
+                if (__ballot(sp + 3 > LDS) == 0) {
+#pragma unroll
+                    for (int i = 3; i >= 1; i--) {
+                        s_st[sp * kBlock + tid] = make_uint2(ref(key[i]), key[i]);
+                        sp += key[i] != kNone ? 1 : 0;
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 3; i >= 1; i--) {
+                        if (key[i] == kNone) continue;
+                        const uint2 e = make_uint2(ref(key[i]), key[i]);
+                        if (sp < LDS) s_st[sp * kBlock + tid] = e;
+                        else if (sp < CAP) sp_st[sp - LDS] = e;
+                        // not reached: the host sizes the stack for the tree
+                        if (sp < CAP) sp++;
+                        else overflow = true;
+                    }
+                }
                 cur = key[0] != kNone ? ref(key[0]) : kNone;
-                // only reachable on overflow (the host sizes the stack for the tree)
-                if (sp > CAP) sp = CAP;
+            }
+            if (cur != kNone && (int32_t)cur < 0 && leaf == kNone) {
+                leaf = cur;
+                cur = kNone;
             }
         }
-        // ---- leaf phase: every lane that holds a leaf tests its record ----
-        if (cur != kNone && (int32_t)cur < 0) {
-            const uint32_t ri = cur & ~REF_LEAF;
-            const PrimRec pr = load_prim(recs, ri);
-            cur = kNone;
+        // ---- leaf phase: the waiting leaves' triangles, one to a lane ----
+        // Leaf number i of the wave has its A tested by lane 2i and its B by lane 2i + 1, with the ray
+        // fetched from the lane that owns it: twenty leaves keep forty lanes busy for one triangle's
+        // time, where their owners would take two. At most 32 leaves a round; others wait.
+        const uint64_t holders = __ballot(leaf != kNone);
+        if (holders == 0) continue;
+        const uint32_t rank = (uint32_t)__popcll(holders & ((1ull << lane) - 1ull));
+        const bool mine = leaf != kNone && rank < 32u;
+        // lane 2i learns which lane owns leaf i; lane 2i + 1 has it from its neighbour
+        int owner = __builtin_amdgcn_ds_permute((int)((mine ? 2u * rank : 63u) << 2), mine ? (int)lane : -1);
+        owner = (int)quad_even((uint32_t)owner);
+        const bool tester = (lane >> 1) < (uint32_t)__popcll(holders);
+        const int from = owner << 2;
+        auto fetch = [&](float x) { return __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(x))); };
+        RayK w;
+        w.okx = fetch(r.okx); w.oky = fetch(r.oky); w.okz = fetch(r.okz);
+        w.sx = fetch(r.sx); w.sy = fetch(r.sy); w.sz = fetch(r.sz);
+        w.tmin = fetch(r.tmin);
+        w.tmax = fetch(r.tmax);
+        w.ky = __builtin_amdgcn_ds_bpermute(from, r.ky);
+        const uint32_t ri = leaf & ~REF_LEAF;
+        const char* tp = nullptr;
+        if (MULTI) {
+            const uint64_t at = reinterpret_cast<uint64_t>(recs + ri);
+            const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)(uint32_t)at);
+            const uint32_t up = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)(uint32_t)(at >> 32));
+            tp = reinterpret_cast<const char*>(((uint64_t)up << 32) | lo);
+        } else {
+            const uint32_t at = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)(ri * (uint32_t)sizeof(PrimRec)));
+            tp = reinterpret_cast<const char*>(recs) + at;
+        }
+        float t = FLT_INF, u = 0.f, v = 0.f;
+        bool quad = false;
+        if (tester) {
+            w.kz = w.ky == 2 ? 0 : w.ky + 1;
+            w.kx = w.kz == 2 ? 0 : w.kz + 1;
+            const Float3* vp = reinterpret_cast<const Float3*>(tp + (lane & 1u) * sizeof(Tri));
+            const Float3 p0 = vp[0], p1 = vp[1], p2 = vp[2];
+            const Tri x{p0.x, p0.y, p0.z, p1.x, p1.y, p1.z, p2.x, p2.y, p2.z};
+            quad = __builtin_isnan(p1.x);  // a quad's record (no triangle of a walk tree holds a NaN)
+            float tt, uu, vv;
+            if (tri_test(w, x, tt, uu, vv)) {
+                t = tt;
+                u = uu;
+                v = vv;
+            }
+        }
+        // the nearer of A and B (A where they are equal), and the other one's distance
+        const float to = quad_swap(t), uo = quad_swap(u), vo = quad_swap(v);
+        const bool take_b = to < t;  // as lane 2i sees it
+        float other = take_b ? t : (to == t ? FLT_INF : to);
+        if (quad) other = -1.0f;
+        const int back = (int)((2u * min(rank, 31u)) << 2);
+        auto result = [&](float x) { return __int_as_float(__builtin_amdgcn_ds_bpermute(back, __float_as_int(x))); };
+        const float rt = result(take_b ? to : t), ru = result(take_b ? uo : u), rv = result(take_b ? vo : v);
+        const float ro = result(other);
+        const bool rb = __builtin_amdgcn_ds_bpermute(back, take_b ? 1 : 0) != 0;
+        if (mine) {
+            leaf = kNone;
+            if (cur != kNone && (int32_t)cur < 0) {
+                leaf = cur;
+                cur = kNone;
+            }
             // A tie of two triangles of one Fast-BVH leaf (a mesh with doubled faces has one at every
             // hit): the one that comes first there wins. False: not such a tie.
-            float tie_u = 0.f, tie_v = 0.f;
-            auto same_leaf_order = [&](uint32_t rec, uint32_t which) {
-                if (rec == hit >> 1) return (pr.id_a & PR_FLAG) == 0;  // A and B of one record: A comes first
+            auto same_leaf_order = [&](uint32_t which, float tie_u, float tie_v) {
                 const TreeView& tv = MULTI ? a.trees[a.ray_scene[ray_id]] : a.tree;
-                const WalkAux &x = tv.waux[rec], &y = tv.waux[hit >> 1];
+                if ((recs[ri].id_a & PR_FLAG) || (recs[hit >> 1].id_a & PR_FLAG)) return false;
+                if (ri == hit >> 1) return true;  // the same record again
+                const WalkAux &x = tv.waux[ri], &y = tv.waux[hit >> 1];
                 const uint32_t px = (x.places >> (16u * which)) & 0xffffu, py = (y.places >> (16u * (hit & 1u))) & 0xffffu;
-                if (x.leaf != y.leaf || px == 0xffffu || py == 0xffffu || (pr.id_a & PR_FLAG) ||
-                    (recs[hit >> 1].id_a & PR_FLAG))
-                    return false;
+                if (x.leaf != y.leaf || px == 0xffffu || py == 0xffffu) return false;
                 if (px < py) {
-                    hit = 2 * rec + which;
+                    hit = 2 * ri + which;
                     bu = tie_u;
                     bv = tie_v;
                 }
                 return true;
             };
-            auto found = [&](float t, float u, float v, uint32_t which) {
-                tie_u = u;
-                tie_v = v;
-                if (t < bt) {
+            auto found = [&](float ft, float fu, float fv, uint32_t which) {
+                if (ft < bt) {
                     second = bt;
-                    bt = t;
-                    bu = u;
-                    bv = v;
+                    bt = ft;
+                    bu = fu;
+                    bv = fv;
                     hit = 2 * ri + which;
-                    lim = t + (slack + 4e-7f * t);
-                } else if (!ANY) {
-                    if (t == bt && same_leaf_order(ri, which)) return;
-                    second = fminf(second, t);
+                    lim = ft + (slack + 4e-7f * ft);
+                } else if (!ANY && !(ft == bt && same_leaf_order(which, fu, fv))) {
+                    second = fminf(second, ft);
                 }
             };
-            if (pr.id_a & PR_FLAG) {
+            if (ro < 0.0f) {
                 const TreeView& tv = MULTI ? a.trees[a.ray_scene[ray_id]] : a.tree;
-                RayK w;
-                load_ray(a.rays, ray_id, w);
-                float t;
-                if (quad_test(w, tv.quads[__float_as_uint(pr.a.p0x)], FLT_MAX, t)) found(t, 0.f, 0.f, 0u);
-            } else {
-                float t, u, v;
-                if (tri_test(r, pr.a, t, u, v)) found(t, u, v, 0u);
-                if ((pr.id_b & PR_ID) != PR_NONE && tri_test(r, pr.b, t, u, v)) found(t, u, v, 1u);
+                RayK q;
+                load_ray(a.rays, ray_id, q);
+                float ft;
+                if (quad_test(q, tv.quads[__float_as_uint(recs[ri].a.p0x)], FLT_MAX, ft)) found(ft, 0.f, 0.f, 0u);
+            } else if (rt < FLT_INF) {
+                found(rt, ru, rv, rb ? 1u : 0u);
+                second = fminf(second, ro);
             }
-            if (ANY && hit != kNone) sp = 0;
+            if (ANY && hit != kNone) {
+                sp = 0;
+                cur = leaf = kNone;
+            }
         }
     }
     if (overflow) atomicOr(a.error, kFlagStackOverflow);
@@ -508,7 +642,8 @@ hipError_t launch(const TraceArgs& a, hipStream_t stream, int num_cus) {
     if (e != hipSuccess) return e;
     if (per_cu < 1) per_cu = 1;
     if (a.blocks_per_cu && (int)a.blocks_per_cu < per_cu) per_cu = (int)a.blocks_per_cu;
-    const uint64_t want = ((uint64_t)a.n + kBlock - 1) / kBlock;
+    // as many waves as run at once, down to four rays each
+    const uint64_t want = ((uint64_t)a.n + 15) / 16;
     uint64_t grid = (uint64_t)num_cus * (uint64_t)per_cu;
     if (want < grid) grid = want;
     if (grid < 1) grid = 1;

@@ -6,6 +6,7 @@
 #include <cfloat>
 #include <cmath>
 #include <cstring>
+#include <limits>
 #include <memory>
 #include <thread>
 
@@ -267,6 +268,7 @@ struct Builder {
         if (id >= in.ntris) {
             const uint32_t q = id - in.ntris;
             std::memcpy(&r.a.p0x, &q, sizeof(q));
+            r.a.p1x = std::numeric_limits<float>::quiet_NaN();  // never hit as a triangle
             r.id_a = id | PR_FLAG;
         } else {
             put_tri(r.a, id);
@@ -326,9 +328,8 @@ struct Builder {
             }
             w.exp[k] = (uint8_t)e;
             for (uint32_t j = 0; j < 4; j++) {
-                if (j >= n) {  // unused slot: an inverted box (its slot number rules it out as well)
-                    lo[k][j] = 255;
-                    hi[k][j] = 0;
+                if (j >= n) {  // unused slot
+                    lo[k][j] = hi[k][j] = 255;
                     continue;
                 }
                 const Bin& x = bins[c[j]];
@@ -420,11 +421,16 @@ struct Builder {
         }
         // the kernel's offsets into both arrays are 32-bit bytes, and a record index shares its
         // word with the leaf bit
-        if (stack > kWalkMaxStack || nbase[np] * sizeof(WalkNode) > UINT32_MAX || rbase[np] * sizeof(PrimRec) > UINT32_MAX)
+        if (stack > kWalkMaxStack || nbase[np] * sizeof(WalkNode) > UINT32_MAX || (rbase[np] + kWalkPadRecs) * sizeof(PrimRec) > UINT32_MAX)
             return;
         out.nodes.resize(nbase[np]);
-        out.recs.resize(rbase[np]);
-        out.aux.resize(rbase[np]);
+        out.recs.resize(rbase[np] + kWalkPadRecs);
+        out.aux.resize(rbase[np] + kWalkPadRecs);
+        PrimRec none;  // a triangle of three equal corners is never hit
+        std::memset(&none, 0, sizeof(none));
+        none.id_b = PR_NONE | PR_FLAG;
+        std::fill(out.recs.begin() + rbase[np], out.recs.end(), none);
+        std::fill(out.aux.begin() + rbase[np], out.aux.end(), WalkAux{});
         std::copy(top.nodes.begin(), top.nodes.end(), out.nodes.begin());
         std::copy(top.recs.begin(), top.recs.end(), out.recs.begin());
         std::copy(top.aux.begin(), top.aux.end(), out.aux.begin());

@@ -88,7 +88,7 @@ static int check(unsigned ntris, unsigned nquads, unsigned width, unsigned leaf,
                 continue;
             }
             const uint32_t r = n.rec_base + j - ni;
-            if (r >= w.recs.size()) return fail("record out of range", ntris);
+            if (r + kWalkPadRecs >= w.recs.size()) return fail("record out of range", ntris);
             const PrimRec& p = w.recs[r];
             const WalkAux& x = w.aux[r];
             if (!(p.id_b & PR_FLAG)) return fail("record not last", ntris);

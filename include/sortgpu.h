@@ -229,9 +229,11 @@ int sortgpu_accel_errors(sortgpu_accel* accel, void* stream, uint32_t* flags);
  * leaf_min = a leaf-testing phase ends when fewer lanes hold a leaf (default 1, 1..64; transparent
  * shadows and trees without a walk tree only);
  * reorder = traversal order of sortgpu_trace_closest / _any / _attenuation / _multi and
- * sortgpu_pool_trace batches: 0 (default) sorts batches of at least 262,144 rays by origin cell
- * (128^3 grid over the scene box; pooled rays by scene, then by cell in their scene's box) before the
- * launch (stream-ordered device memory of 16 bytes per ray plus sort workspace, from a pool the
+ * sortgpu_pool_trace batches: 0 (default) sorts a batch by origin cell (128^3 grid over the scene box;
+ * pooled rays by scene, then by cell in their scene's box) before the launch where that pays: closest
+ * and any hit from 2,097,152 rays on trees of about 3.5M triangles or more, transparent shadows from
+ * 524,288 rays, probes from 1,048,576, trees without a second tree (sortgpu_accel_build) from 262,144
+ * (stream-ordered device memory of 16 bytes per ray plus sort workspace, from a pool the
  * context owns; a batch sharing one origin, such as camera rays, keeps its order and pays only the
  * sort), 1 = never, 2 = always; shade_order = order in which the path tracer shades each bounce's
  * hits: 0 (default) sorts them by position (a 16^3 grid over the scene box; by scene and an 8^3 grid

@@ -307,14 +307,14 @@ hipMemPool_t sortgpu::order_pool(sortgpu_ctx* ctx) {
 
 extern "C" {
 
-// Coherence order for a large batch on `s` (the tuning's reorder knob decides), or null for index
-// order. An order that cannot be had (no pool, no memory) only costs speed, so it is not an error.
+// Traversal order for a batch on `s`, or null for index order: as the tuning's reorder knob says, by
+// default where it pays. An order that cannot be had (no pool, no memory) only costs speed, so it is not an error.
 // Results never depend on it; `ro` is released on `s` after the launch that reads it.
-static const uint32_t* traversal_order(sortgpu_accel* acc, const sortgpu_ray* d_rays, uint32_t n, hipStream_t s,
-                                       RayOrder& ro) {
+static const uint32_t* traversal_order(sortgpu_accel* acc, const sortgpu_ray* d_rays, uint32_t n, bool pays,
+                                       hipStream_t s, RayOrder& ro) {
     sortgpu_ctx* ctx = acc->ctx;
     const uint32_t reorder = ctx->tuning.reorder;
-    if (reorder == 1 || (reorder != 2 && n < kReorderMinRays) || n > 0x7fffffffu) return nullptr;
+    if (reorder == 1 || (reorder != 2 && !pays) || n > 0x7fffffffu) return nullptr;
     hipMemPool_t pool = order_pool(ctx);
     if (pool && order_rays(pool, d_rays, n, acc->view.bbox, s, ro) == hipSuccess) return ro.order;
     (void)hipGetLastError();
@@ -361,7 +361,7 @@ static int trace_common(sortgpu_accel* acc, const sortgpu_ray* d_rays, uint32_t 
     }
     // traversal order (results do not depend on it; the counter launch keeps index order)
     RayOrder ro;
-    if (!stats) a.order = traversal_order(acc, d_rays, n, s, ro);
+    if (!stats) a.order = traversal_order(acc, d_rays, n, reorder_pays(n, walk_bytes(acc->host)), s, ro);
     hipError_t e = launch_trace(a, any, stats, s, ctx->num_cus);
     if (ro.order) release_order(ro, s);
     if (e != hipSuccess) return hip_fail(ctx, e, "trace launch");
@@ -418,7 +418,7 @@ int sortgpu_trace_closest_noalloc(sortgpu_accel* acc, const sortgpu_ray* d_rays,
     a.error = acc->d_error;
     apply_tuning(ctx, a);
     const uint32_t reorder = ctx->tuning.reorder;
-    if (reorder == 2 || (reorder != 1 && n >= kReorderMinRays)) {
+    if (reorder == 2 || (reorder != 1 && reorder_pays(n, walk_bytes(acc->host)))) {
         void* base = nullptr;
         hipError_t e = scratch_base(ctx->device, &base);
         if (e != hipSuccess) return hip_fail(ctx, e, "trace_closest_noalloc: scratch address");
@@ -561,7 +561,7 @@ int sortgpu_trace_attenuation(sortgpu_accel* acc, const sortgpu_ray* d_rays, uin
     apply_tuning(ctx, a);
     hipStream_t s = static_cast<hipStream_t>(stream);
     RayOrder ro;
-    a.order = traversal_order(acc, d_rays, n, s, ro);
+    a.order = traversal_order(acc, d_rays, n, n >= kReorderMinAttenuation, s, ro);
     hipError_t e = launch_attenuation(a, s, ctx->num_cus);
     if (ro.order) release_order(ro, s);
     if (e != hipSuccess) return hip_fail(ctx, e, "attenuation launch");
@@ -604,7 +604,7 @@ int sortgpu_trace_multi(sortgpu_accel* acc, const sortgpu_ray* d_rays, uint32_t 
     a.error = acc->d_error;
     hipStream_t s = static_cast<hipStream_t>(stream);
     RayOrder ro;
-    a.order = traversal_order(acc, d_rays, n, s, ro);
+    a.order = traversal_order(acc, d_rays, n, n >= kReorderMinMulti, s, ro);
     hipError_t e = launch_multi(a, s);
     if (ro.order) release_order(ro, s);
     if (e != hipSuccess) return hip_fail(ctx, e, "multi-hit launch");

@@ -68,9 +68,31 @@ int upload_accel(sortgpu_accel* acc);
 // Copies the context's tuning knobs into a launch.
 void apply_tuning(const sortgpu_ctx* ctx, struct TraceArgs& a);
 void free_accel_device(sortgpu_accel* acc);
-// Batches at least this large are traced in coherence order by default (smaller ones do not pay
-// for the sort).
+// Which batches are traced in traversal order by default (order.hip). Sorting costs 0.15 ms for 4M
+// rays, and a sorted batch reads its rays and writes its results scattered; what it saves is
+// traffic past the caches. Measured on rays in random order, sorted against index order:
+//   walk tree (closest, any): pays once the tree outgrows the caches and the batch is large. 4M rays
+//     through 1M triangles (57 MB of nodes and records) 1.76 against 1.52 ms, 4M triangles (230 MB)
+//     1.91 / 1.95, 8M 1.94 / 2.19, 16M 2.01 / 2.41; shadow segments 1M 1.79 / 1.69, 4M 1.93 / 2.34,
+//     16M 2.13 / 3.07; 2M rays: 4M triangles 1.16 / 1.11 (shadow 1.16 / 1.31), 16M 1.20 / 1.36;
+//     1M rays: 0.86 / 0.77 through 8M triangles; a pool of 64 scenes and 8M triangles, rays shuffled
+//     over the scenes, 4.63 / 6.83;
+//   transparent shadows: 300K rays 1.65 / 1.60, 600K 2.15 / 2.17, 4M 11.7 / 12.4 ms;
+//   multi-hit probes: 500K 0.54 / 0.48, 1M 0.82 / 0.91, 4M 3.49 / 4.66;
+//   Fast-BVH walk (trees without a walk tree): batches of 256K rays and more.
 constexpr uint32_t kReorderMinRays = 1u << 18;
+constexpr uint32_t kReorderMinWalkRays = 1u << 21;
+constexpr size_t kReorderMinWalkBytes = (size_t)192 << 20;
+constexpr uint32_t kReorderMinAttenuation = 1u << 19;
+constexpr uint32_t kReorderMinMulti = 1u << 20;
+// Bytes a walk reads of a tree's walk tree (0: it has none).
+inline size_t walk_bytes(const BuiltTree& t) {
+    return t.walk.nodes.size() * sizeof(WalkNode) + t.walk.recs.size() * sizeof(PrimRec);
+}
+// The default for closest- and any-hit batches on walk trees of `bytes` together (0: no walk tree).
+inline bool reorder_pays(uint32_t n, size_t bytes) {
+    return bytes ? n >= kReorderMinWalkRays && bytes >= kReorderMinWalkBytes : n >= kReorderMinRays;
+}
 // Waves of at least this many paths shade each bounce's hits in spatial order (tuning shade_order:
 // 0 = this default, 1 = never (0 returned), 2 = always).
 inline uint32_t shade_sort_min(const sortgpu_tuning& t) {

@@ -1,10 +1,10 @@
 // Traversal order of a ray batch.
 //
-// A traversal lane reads its own node and primitive records, and what a launch costs is the
-// number of such reads that the compute units serve. Lanes of one wave that walk the same nodes
-// at the same time share those reads. Incoherent batches (bounce rays from random surface points)
-// arrive in no useful order, so before the launch the batch is sorted (stably) by its origin's
-// cell on a 128^3 grid over the tree's box, in Morton order (a 21-bit key: the same three 8-bit
+// A traversal lane reads its own node and primitive records. Rays that walk the same part of a tree
+// at the same time find those records in the caches; incoherent batches (bounce rays from random
+// surface points) arrive in no useful order. So before a launch on a tree that outgrows the caches
+// (the rule and its figures: kReorderMinWalkRays and its neighbours) the batch is sorted (stably) by its
+// origin's cell on a 128^3 grid over the tree's box, in Morton order (a 21-bit key: the same three 8-bit
 // radix passes as a 64^3 grid, and an order that measured 0.6% faster on incoherent batches).
 // Direction cells or octants in the key were measured to cost camera batches 4-5% and gain bounce
 // batches under 1%, so the key has none: a batch sharing one origin keeps its order. The kernel takes rays in the sorted

@@ -20,7 +20,7 @@ struct sortgpu_pool {
     TreeView* d_views = nullptr;   // n tree views
     uint32_t* d_counters = nullptr;
     uint32_t* d_error = nullptr;
-    size_t bytes = 0;
+    size_t bytes = 0, walk_bytes = 0;
     std::atomic<uint32_t> slot{0};
 };
 
@@ -84,6 +84,7 @@ int sortgpu_pool_create(sortgpu_ctx* ctx, sortgpu_accel* const* accels, uint32_t
     p->width = width;
     p->max_stack = max_stack;
     p->walk_stack = walk_stack;
+    for (uint32_t i = 0; i < n && walk_stack; i++) p->walk_bytes += walk_bytes(accels[i]->host);
     hipError_t e;
     auto fail = [&](hipError_t err, const char* what) {
         int r = hip_fail(ctx, err, what);
@@ -209,7 +210,7 @@ int sortgpu_pool_trace(sortgpu_pool* p, const sortgpu_ray* d_rays, const uint32_
     // do not depend on it; an order that cannot be had only costs speed)
     RayOrder ro;
     const uint32_t reorder = p->ctx->tuning.reorder;
-    if (reorder == 2 || (reorder != 1 && n >= kReorderMinRays && n <= 0x7fffffffu)) {
+    if (reorder == 2 || (reorder != 1 && reorder_pays(n, p->walk_bytes) && n <= 0x7fffffffu)) {
         hipMemPool_t mp = order_pool(p->ctx);
         if (mp && order_rays_multi(mp, d_rays, d_ray_scene, n, p->d_views, p->n, s, ro) == hipSuccess)
             a.order = ro.order;

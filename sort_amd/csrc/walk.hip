@@ -31,6 +31,8 @@
 // more per ray on meshes. 8-wide nodes: 20.7 steps instead of 30.4, each with twice the arithmetic.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+
 #include "trace_launch.h"
 #include "traverse.h"
 
@@ -41,6 +43,8 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr uint32_t kNone = 0xffffffffu;
+constexpr uint32_t kDealtPerWave = 128;  // rays per wave from which part of a batch goes out through the counter
+constexpr uint32_t kQuadsPerWave = 28;   // rays per wave up to which four lanes take a ray together
 constexpr float kPad = 1.9073486328125e-6f;  // 2^-19
 
 // What the walk keeps of a ray besides the triangle test's constants: reciprocal directions (true
@@ -157,12 +161,16 @@ struct __attribute__((packed, aligned(4))) Float3 {
     float x, y, z;
 };
 
-// The value of the even lane of this lane's pair; the value of the pair's other lane.
-__device__ __forceinline__ uint32_t quad_even(uint32_t x) {
+// The value of the even lane of this lane's pair; of the pair's other lane; of another lane of its four.
+__device__ __forceinline__ uint32_t pair_even(uint32_t x) {
     return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xA0, 0xf, 0xf, true);  // quad_perm [0, 0, 2, 2]
 }
-__device__ __forceinline__ float quad_swap(float x) {
+__device__ __forceinline__ float pair_swap(float x) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, true));  // [1, 0, 3, 2]
+}
+template <int PERM>
+__device__ __forceinline__ uint32_t quad_rot(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, PERM, 0xf, 0xf, true);
 }
 
 struct Best {
@@ -245,116 +253,279 @@ __device__ __forceinline__ void exact_walk(const TreeView& tv, RayK& r, uint2* s
     }
 }
 
-template <bool ANY, bool MULTI, int LDS, int SPILL>
-// 4 waves per SIMD (128 VGPRs): 5 spilled in the rarely taken parts and gained nothing.
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_walk(TraceArgs a) {
-    __shared__ uint2 s_st[LDS * kBlock];  // (reference, entry distance), [entry][thread]
-    constexpr int CAP = LDS + SPILL;
-    uint2 sp_st[SPILL];  // deeper entries; also the stack of exact_walk, whose lane has none of its own left
-
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = __lane_id();
-    const uint32_t n_rays = a.n_dev ? *a.n_dev : a.n;
-    const uint32_t refill = a.refill ? a.refill : 16u;
-    const uint32_t leaf_batch = a.leaf_batch ? a.leaf_batch : 24u;
-    const WalkNode* __restrict__ nodes = a.tree.wnodes;
-    const PrimRec* __restrict__ recs = a.tree.wrecs;
-
+// A ray on its way through a walk tree.
+struct Walker {
     RayK r;
     Slabs s;
-    uint32_t cur = kNone;   // node to visit next (or the next leaf, while `leaf` is taken); kNone: pop the stack
-    uint32_t leaf = kNone;  // leaf waiting for the wave's leaf phase
-    uint32_t ray_id = kNone;
-    uint32_t hit = kNone;  // nearest candidate: record * 2 + (0: A or the quad, 1: B)
-    float bt = FLT_MAX, bu = 0.f, bv = 0.f;
-    float lim = FLT_MAX;     // search bound: the window's end, then bt and the slack above it
-    float second = FLT_MAX;  // second nearest distance met
-    float slack = 0.f;
-    int sp = 0;
-    bool more = true, overflow = false, open = false;  // open: exact_walk has to answer
+    const WalkNode* nodes;
+    const PrimRec* recs;
+    uint32_t cur;     // node to visit next (or the next leaf, while `leaf` is taken); kNone: pop the stack
+    uint32_t leaf;    // leaf waiting for the wave's leaf phase
+    uint32_t ray_id;  // kNone: no ray
+    uint32_t hit;     // nearest candidate: record * 2 + (0: A or the quad, 1: B)
+    float bt, bu, bv;
+    float lim;        // search bound: the window's end, then bt and the slack above it
+    float second;     // second nearest distance met
+    float slack;
+    int sp;
+    bool open;        // exact_walk has to answer
+
+    __device__ __forceinline__ bool idle() const { return cur == kNone && leaf == kNone && sp == 0; }
+    __device__ __forceinline__ bool walking() const { return (int32_t)cur >= 0 || (cur == kNone && sp > 0); }
+    __device__ __forceinline__ bool at_leaf() const { return cur != kNone && (int32_t)cur < 0; }
+};
+
+// Takes up ray `my`, or answers it where the scene's box already does.
+template <bool ANY, bool MULTI>
+__device__ __forceinline__ void start(const TraceArgs& a, uint32_t my, Walker& w) {
+    load_ray(a.rays, my, w.r);
+    w.bt = w.second = FLT_MAX;
+    w.lim = w.r.tmax;
+    w.bu = w.bv = 0.f;
+    w.hit = kNone;
+    w.open = false;
+    bool known = true;  // the scene id is one of the table's
+    const TreeView* tv = &a.tree;
+    if (MULTI) {
+        const uint32_t sid = a.ray_scene[my];
+        known = sid < a.n_trees;
+        if (!known) atomicOr(a.error, kFlagBadScene);
+        tv = a.trees + (known ? sid : 0u);
+        w.nodes = tv->wnodes;
+        w.recs = tv->wrecs;
+    }
+    const bool fits = slabs_setup(w.r, tv->bbox, w.s, w.slack);
+    shear_setup(w.r, w.s);
+    // a ray outside the bounds goes to the exact walk, with its root test
+    if (known && tv->valid && (!fits || root_test(w.r, w.s, tv->bbox))) {
+        w.ray_id = my;
+        if (fits) w.cur = 0;
+        else w.open = true;
+    } else if (!ANY) {
+        reinterpret_cast<float4*>(a.out)[my] = make_float4(FLT_MAX, __uint_as_float(kNone), 0.f, 0.f);
+    } else if (!a.occ_slot) {
+        static_cast<uint8_t*>(a.out)[my] = 0;
+    }
+}
+
+// Answers the walker's ray: shows that the Fast-BVH walk returns its candidate, or walks that tree.
+template <bool ANY, bool MULTI>
+__device__ __forceinline__ void settle(const TraceArgs& a, Walker& w, uint2* st) {
+    const Slabs& s = w.s;
+    RayK& r = w.r;
+    Best best{w.bt, w.bu, w.bv, kNone, false};
+    if (!w.open && w.hit != kNone) {
+        const TreeView& tv = MULTI ? a.trees[a.ray_scene[w.ray_id]] : a.tree;
+        const float4* xp = reinterpret_cast<const float4*>(tv.waux + (w.hit >> 1));
+        const float4 x0 = xp[0], x1 = xp[1];
+        best.any = true;
+        if (!ANY) {
+            const uint32_t* rw = reinterpret_cast<const uint32_t*>(tv.wrecs + (w.hit >> 1));
+            best.prim = rw[18 + (w.hit & 1u)] & PR_ID;
+        }
+        // the leaf box shrunk by the padding: if even that one is hit, the exact test passes too, with
+        // an entry distance no larger than this one
+        const bool px = s.rx >= 0.0f, py = s.ry >= 0.0f, pz = s.rz >= 0.0f;
+        float entry = fmaxf(fmaxf((px ? x0.x : x0.w) * s.rx + s.bx, (py ? x0.y : x1.x) * s.ry + s.by),
+                            fmaxf((pz ? x0.z : x1.y) * s.rz + s.bz, r.tmin));
+        const float exit = fminf(fminf((px ? x0.w : x0.x) * s.rx + s.ax, (py ? x1.x : x0.y) * s.ry + s.ay),
+                                 fminf((pz ? x1.y : x0.z) * s.rz + s.az, r.tmax));
+        // (beyond 1e5 the exact test steps along another line: it clamps the direction)
+        const bool clamped = fmaxf(fmaxf(fabsf(s.rx), fabsf(s.ry)), fabsf(s.rz)) > 1e5f;
+        const bool inside = entry <= exit && !clamped;
+        auto alone = [&](float e) { return ANY || e <= w.bt || (e < w.second && e <= w.lim); };
+        if (!(w.second > w.bt) && !ANY) {
+            w.open = true;  // a tie
+        } else if (!(inside && alone(entry))) {
+            load_ray(a.rays, w.ray_id, r);
+            ray_setup(r);
+            w.open = !box_test(r, x0.x, x0.w, x0.y, x1.x, x0.z, x1.y, entry) || !alone(entry);
+        }
+    }
+    if (w.open) {
+        const TreeView& tv = MULTI ? a.trees[a.ray_scene[w.ray_id]] : a.tree;
+        load_ray(a.rays, w.ray_id, r);
+        exact_walk<ANY>(tv, r, st, best);
+    }
+    if (!ANY) {
+        reinterpret_cast<float4*>(a.out)[w.ray_id] = make_float4(best.t, __uint_as_float(best.prim), best.u, best.v);
+    } else if (!a.occ_slot) {
+        static_cast<uint8_t*>(a.out)[w.ray_id] = best.any ? 1 : 0;
+    } else if (best.any) {  // the shadow ray's contribution is cleared here (w kept)
+        const uint32_t slot = a.occ_slot[w.ray_id];
+        float* c = reinterpret_cast<float*>(a.occ_rec + 4 * (size_t)(slot >> 1) + 2 + (slot & 1u));
+        c[0] = 0.f;
+        c[1] = 0.f;
+        c[2] = 0.f;
+    }
+}
+
+// A node record with the ray's near and far planes picked out, and where its children lie.
+struct NodeSlabs {
+    float gx, gy, gz, nx, ny, nz, fx, fy, fz;
+    uint32_t wnx, wfx, wny, wfy, wnz, wfz;
+    uint32_t ni, child_at, leaf_at;
+
+    __device__ __forceinline__ NodeSlabs(const WalkNode* nodes, uint32_t i, const Slabs& s) {
+        const uint4* np = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(nodes) + (((i << 1) + i) << 4));
+        const uint4 q0 = np[0], q1 = np[1], q2 = np[2];
+        const uint32_t meta = q0.w;
+        ni = (meta >> 24) & 15u;
+        gx = __uint_as_float((meta & 0xffu) << 23) * s.rx;
+        gy = __uint_as_float(((meta >> 8) & 0xffu) << 23) * s.ry;
+        gz = __uint_as_float(((meta >> 16) & 0xffu) << 23) * s.rz;
+        const float bx = __uint_as_float(q0.x) * s.rx, by = __uint_as_float(q0.y) * s.ry, bz = __uint_as_float(q0.z) * s.rz;
+        nx = bx + s.ax;
+        ny = by + s.ay;
+        nz = bz + s.az;
+        fx = bx + s.bx;
+        fy = by + s.by;
+        fz = bz + s.bz;
+        const bool px = s.rx >= 0.0f, py = s.ry >= 0.0f, pz = s.rz >= 0.0f;
+        wnx = px ? q1.z : q1.w;
+        wfx = px ? q1.w : q1.z;
+        wny = py ? q2.x : q2.y;
+        wfy = py ? q2.y : q2.x;
+        wnz = pz ? q2.z : q2.w;
+        wfz = pz ? q2.w : q2.z;
+        child_at = q1.x;
+        leaf_at = (q1.y | REF_LEAF) - ni;
+    }
+    // Sort key of slot j: kNone where the ray misses its box, else the entry distance (not negative,
+    // so that its bits order as it does) with the slot in the last two bits. `shift`: 8 j.
+    __device__ __forceinline__ uint32_t key(uint32_t j, uint32_t shift, float tmin, float lim) const {
+        auto q = [&](uint32_t x) { return (float)((x >> shift) & 0xffu); };
+        const float t0 = fmaxf(fmaxf(__builtin_fmaf(q(wnx), gx, nx), __builtin_fmaf(q(wny), gy, ny)),
+                               fmaxf(__builtin_fmaf(q(wnz), gz, nz), tmin));
+        const float t1 = fminf(fminf(__builtin_fmaf(q(wfx), gx, fx), __builtin_fmaf(q(wfy), gy, fy)),
+                               fminf(__builtin_fmaf(q(wfz), gz, fz), lim));
+        return t0 <= t1 ? ((__float_as_uint(t0) & ~3u) | j) : kNone;
+    }
+    __device__ __forceinline__ uint32_t ref(uint32_t key) const {
+        const uint32_t j = key & 3u;
+        return (j < ni ? child_at : leaf_at) + j;
+    }
+};
+
+// A triangle's or quad's hit in record `ri` (which: A or B).
+template <bool ANY, bool MULTI>
+__device__ __forceinline__ void found(const TraceArgs& a, Walker& w, uint32_t ri, float t, float u, float v, uint32_t which) {
+    // A tie of two triangles of one Fast-BVH leaf (a mesh with doubled faces has one at every hit): the
+    // one that comes first there wins. False: not such a tie.
+    auto same_leaf_order = [&]() {
+        const TreeView& tv = MULTI ? a.trees[a.ray_scene[w.ray_id]] : a.tree;
+        if ((w.recs[ri].id_a & PR_FLAG) || (w.recs[w.hit >> 1].id_a & PR_FLAG)) return false;
+        if (ri == w.hit >> 1) return true;  // the same record again
+        const WalkAux &x = tv.waux[ri], &y = tv.waux[w.hit >> 1];
+        const uint32_t px = (x.places >> (16u * which)) & 0xffffu, py = (y.places >> (16u * (w.hit & 1u))) & 0xffffu;
+        if (x.leaf != y.leaf || px == 0xffffu || py == 0xffffu) return false;
+        if (px < py) {
+            w.hit = 2 * ri + which;
+            w.bu = u;
+            w.bv = v;
+        }
+        return true;
+    };
+    if (t < w.bt) {
+        w.second = w.bt;
+        w.bt = t;
+        w.bu = u;
+        w.bv = v;
+        w.hit = 2 * ri + which;
+        w.lim = t + (w.slack + 4e-7f * t);
+    } else if (!ANY && !(t == w.bt && same_leaf_order())) {
+        w.second = fminf(w.second, t);
+    }
+}
+
+// The outcome of record `ri`: t, u, v of the nearer of A and B (`which`; A where they are equal), or
+// infinity, and the other one's distance; negative: the record is a quad.
+template <bool ANY, bool MULTI>
+__device__ __forceinline__ void leaf_outcome(const TraceArgs& a, Walker& w, uint32_t ri, float t, float u, float v,
+                                             float other, uint32_t which) {
+    if (other < 0.0f) {
+        const TreeView& tv = MULTI ? a.trees[a.ray_scene[w.ray_id]] : a.tree;
+        RayK q;
+        load_ray(a.rays, w.ray_id, q);
+        float qt;
+        if (quad_test(q, tv.quads[__float_as_uint(w.recs[ri].a.p0x)], FLT_MAX, qt))
+            found<ANY, MULTI>(a, w, ri, qt, 0.f, 0.f, 0u);
+    } else if (t < FLT_INF) {
+        found<ANY, MULTI>(a, w, ri, t, u, v, which);
+        w.second = fminf(w.second, other);
+    }
+    if (ANY && w.hit != kNone) {
+        w.sp = 0;
+        w.cur = w.leaf = kNone;
+    }
+}
+
+// Tests the triangle at `tp`; true: the record is a quad's (no triangle of a walk tree holds a NaN).
+__device__ __forceinline__ bool record_tri(RayK& r, const char* tp, float& t, float& u, float& v) {
+    r.kz = r.ky == 2 ? 0 : r.ky + 1;
+    r.kx = r.kz == 2 ? 0 : r.kz + 1;
+    const Float3* vp = reinterpret_cast<const Float3*>(tp);
+    const Float3 p0 = vp[0], p1 = vp[1], p2 = vp[2];
+    const Tri x{p0.x, p0.y, p0.z, p1.x, p1.y, p1.z, p2.x, p2.y, p2.z};
+    float tt, uu, vv;
+    if (tri_test(r, x, tt, uu, vv)) {
+        t = tt;
+        u = uu;
+        v = vv;
+    }
+    return __builtin_isnan(p1.x);
+}
+
+// One ray to a lane: batches that fill the chip.
+template <bool ANY, bool MULTI, int LDS, int SPILL>
+__device__ __forceinline__ void walk_lanes(const TraceArgs& a, uint32_t n_rays, uint2* s_st, uint32_t* s_next,
+                                           uint32_t* s_out) {
+    constexpr int CAP = LDS + SPILL;
+    uint2 sp_st[SPILL];  // deeper entries; also the stack of exact_walk, whose lane has none of its own left
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = __lane_id();
+    const uint32_t refill = a.refill ? a.refill : 16u;
+    const uint32_t leaf_batch = a.leaf_batch ? a.leaf_batch : 24u;
     // Handing out the rays. One atomic on the launch's counter takes about 8.5 ns of the whole chip's
     // time (measured: 4.19M rays, 16 at a time, spent 2.2 ms there), so every workgroup has a share of
     // its own that its waves take from through LDS. Of a large batch only three quarters are shares,
     // dealt 64 rays at a time so that all workgroups move through the order together (a contiguous
-    // share each has them all over the tree at once: 2.05 instead of 1.87 ms for 4.19M
-    // bounce rays); the rest goes out
-    // through the counter, in chunks that shrink with what is left, so that the workgroups end
-    // together. A batch with less than a full wave of rays for each wave spreads over all of them, on
-    // the first `seats` lanes of each.
+    // share each has them all over the tree at once: 2.05 instead of 1.87 ms for 4.19M sorted bounce
+    // rays); the rest goes out through the counter, in chunks that shrink with what is left, so that
+    // the workgroups end together. A batch with less than a full wave of rays for each wave spreads
+    // over all of them, on the first `seats` lanes of each.
     const uint32_t waves = gridDim.x * (kBlock / 64);
     const uint32_t seats = min((n_rays + waves - 1) / waves, 64u);
-    const bool dealt = n_rays >= 128u * waves;
+    const bool dealt = n_rays >= kDealtPerWave * waves;
     const uint32_t share = dealt ? (n_rays - n_rays / 4u) / (gridDim.x * 64u) * 64u : (n_rays + gridDim.x - 1) / gridDim.x;
     const uint32_t pooled = min(share * gridDim.x, n_rays);  // first ray that the counter hands out
-    __shared__ uint32_t s_next, s_out;  // rays of the share taken; whether the counter has run out
     if (tid == 0) {
-        s_next = 0;
-        s_out = pooled >= n_rays ? 1u : 0u;
+        *s_next = 0;                         // rays of the share taken
+        *s_out = pooled >= n_rays ? 1u : 0u;  // whether the counter has run out
     }
     __syncthreads();
-    bool sharing = true;             // the share may have rays left
-    uint32_t own = 0, own_end = 0;   // this wave's chunk of the rest
-    more = lane < seats;
-
+    bool sharing = true;            // the share may have rays left
+    uint32_t own = 0, own_end = 0;  // this wave's chunk of the rest
+    bool more = lane < seats, overflow = false;
+    Walker w;
+    w.nodes = a.tree.wnodes;
+    w.recs = a.tree.wrecs;
+    w.cur = w.leaf = w.ray_id = w.hit = kNone;
+    w.bt = w.lim = w.second = FLT_MAX;
+    w.bu = w.bv = w.slack = 0.f;
+    w.sp = 0;
+    w.open = false;
 
     while (true) {
-        const bool idle = cur == kNone && leaf == kNone && sp == 0;
-        const uint64_t want = __ballot(idle && (more || ray_id != kNone));
+        const bool idle = w.idle();
+        const uint64_t want = __ballot(idle && (more || w.ray_id != kNone));
         const uint64_t busy = __ballot(!idle);
         if (want == 0 && busy == 0) break;
         if (want != 0 && (busy == 0 || (uint32_t)__popcll(want) >= refill)) {
-            // ---- answer the rays that are through ----
-            if (idle && ray_id != kNone) {
-                Best best{bt, bu, bv, kNone, false};
-                {
-                    if (!open && hit != kNone) {
-                        const TreeView& tv = MULTI ? a.trees[a.ray_scene[ray_id]] : a.tree;
-                        const float4* xp = reinterpret_cast<const float4*>(tv.waux + (hit >> 1));
-                        const float4 x0 = xp[0], x1 = xp[1];
-                        best.any = true;
-                        if (!ANY) {
-                            const uint32_t* rw = reinterpret_cast<const uint32_t*>(tv.wrecs + (hit >> 1));
-                            best.prim = rw[18 + (hit & 1u)] & PR_ID;
-                        }
-                        // the leaf box shrunk by the padding: if even that one is hit, the exact test
-                        // passes too, with an entry distance no larger than this one
-                        const bool px = s.rx >= 0.0f, py = s.ry >= 0.0f, pz = s.rz >= 0.0f;
-                        float entry = fmaxf(fmaxf((px ? x0.x : x0.w) * s.rx + s.bx, (py ? x0.y : x1.x) * s.ry + s.by),
-                                            fmaxf((pz ? x0.z : x1.y) * s.rz + s.bz, r.tmin));
-                        const float exit = fminf(fminf((px ? x0.w : x0.x) * s.rx + s.ax, (py ? x1.x : x0.y) * s.ry + s.ay),
-                                                 fminf((pz ? x1.y : x0.z) * s.rz + s.az, r.tmax));
-                        // (beyond 1e5 the exact test steps along another line: it clamps the direction)
-                        const bool clamped = fmaxf(fmaxf(fabsf(s.rx), fabsf(s.ry)), fabsf(s.rz)) > 1e5f;
-                        const bool inside = entry <= exit && !clamped;
-                        auto alone = [&](float e) { return ANY || e <= bt || (e < second && e <= lim); };
-                        if (!(second > bt) && !ANY) {
-                            open = true;  // a tie
-                        } else if (!(inside && alone(entry))) {
-                            load_ray(a.rays, ray_id, r);
-                            ray_setup(r);
-                            open = !box_test(r, x0.x, x0.w, x0.y, x1.x, x0.z, x1.y, entry) || !alone(entry);
-                        }
-                    }
-                    if (open) {
-                        const TreeView& tv = MULTI ? a.trees[a.ray_scene[ray_id]] : a.tree;
-                        load_ray(a.rays, ray_id, r);
-                        exact_walk<ANY>(tv, r, sp_st, best);
-                    }
-                }
-                if (!ANY) {
-                    reinterpret_cast<float4*>(a.out)[ray_id] = make_float4(best.t, __uint_as_float(best.prim), best.u, best.v);
-                } else if (!a.occ_slot) {
-                    static_cast<uint8_t*>(a.out)[ray_id] = best.any ? 1 : 0;
-                } else if (best.any) {  // the shadow ray's contribution is cleared here (w kept)
-                    const uint32_t slot = a.occ_slot[ray_id];
-                    float* c = reinterpret_cast<float*>(a.occ_rec + 4 * (size_t)(slot >> 1) + 2 + (slot & 1u));
-                    c[0] = 0.f;
-                    c[1] = 0.f;
-                    c[2] = 0.f;
-                }
-                ray_id = kNone;
+            if (idle && w.ray_id != kNone) {
+                settle<ANY, MULTI>(a, w, sp_st);
+                w.ray_id = kNone;
             }
-            // ---- take new ones ----
             const uint64_t take = __ballot(idle && more);
             if (take != 0) {
                 const uint32_t cnt = (uint32_t)__popcll(take);
@@ -363,7 +534,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                 bool given = false, out = false;  // a lane without a ray waits for the next refill; out: there is none
                 if (sharing) {
                     uint32_t v = 0;
-                    if (lane == 0) v = atomicAdd(&s_next, cnt);
+                    if (lane == 0) v = atomicAdd(s_next, cnt);
                     v = __builtin_amdgcn_readfirstlane(v);
                     sharing = v + cnt < share;
                     v += rank;
@@ -372,7 +543,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                 } else {
                     if (own == own_end) {
                         uint32_t done = 0;
-                        if (lane == 0) done = __hip_atomic_load(&s_out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        if (lane == 0) done = __hip_atomic_load(s_out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                         out = __builtin_amdgcn_readfirstlane(done) != 0;
                         if (!out) {
                             const uint32_t rest = n_rays - max(own_end, pooled);
@@ -382,7 +553,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                             own_end = min(own + chunk, n_rays);
                             out = own >= n_rays;
                             if (out && lane == 0)
-                                __hip_atomic_store(&s_out, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                                __hip_atomic_store(s_out, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                         }
                     }
                     k = own + rank;
@@ -390,39 +561,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                     own = min(own + cnt, own_end);
                 }
                 if (out) more = false;
-                if (idle && more) {
-                    if (given) {
-                        const uint32_t my = a.order ? a.order[k] : k;
-                        load_ray(a.rays, my, r);
-                        bt = second = FLT_MAX;
-                        lim = r.tmax;
-                        bu = bv = 0.f;
-                        hit = kNone;
-                        open = false;
-                        bool known = true;  // the scene id is one of the table's
-                        const TreeView* tv = &a.tree;
-                        if (MULTI) {
-                            const uint32_t sid = a.ray_scene[my];
-                            known = sid < a.n_trees;
-                            if (!known) atomicOr(a.error, kFlagBadScene);
-                            tv = a.trees + (known ? sid : 0u);
-                            nodes = tv->wnodes;
-                            recs = tv->wrecs;
-                        }
-                        const bool fits = slabs_setup(r, tv->bbox, s, slack);
-                        shear_setup(r, s);
-                        // a ray outside the bounds goes to the exact walk, with its root test
-                        if (known && tv->valid && (!fits || root_test(r, s, tv->bbox))) {
-                            ray_id = my;
-                            if (fits) cur = 0;
-                            else open = true;
-                        } else if (!ANY) {
-                            reinterpret_cast<float4*>(a.out)[my] = make_float4(FLT_MAX, __uint_as_float(kNone), 0.f, 0.f);
-                        } else if (!a.occ_slot) {
-                            static_cast<uint8_t*>(a.out)[my] = 0;
-                        }
-                    }
-                }
+                if (idle && more && given) start<ANY, MULTI>(a, a.order ? a.order[k] : k, w);
             }
             continue;
         }
@@ -433,56 +572,29 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         // bounce rays, 0.47 -> 0.44 for 2.07M camera rays)
         const uint32_t batch = (leaf_batch * (uint32_t)__popcll(busy) + 63u) / 64u;
         while (true) {
-            const bool walk = (int32_t)cur >= 0 || (cur == kNone && sp > 0);
-            if (__ballot(walk) == 0 || (uint32_t)__popcll(__ballot(leaf != kNone)) >= batch) break;
-            const bool pop = walk && cur == kNone;
+            const bool walk = w.walking();
+            if (__ballot(walk) == 0 || (uint32_t)__popcll(__ballot(w.leaf != kNone)) >= batch) break;
+            const bool pop = walk && w.cur == kNone;
             // Stack accesses are LDS ones unless some lane of the wave is past the entries there: a
             // choice per lane would make every access a generic one.
-            if (__ballot(pop && sp > LDS) == 0) {
+            if (__ballot(pop && w.sp > LDS) == 0) {
                 if (pop) {
-                    --sp;
-                    const uint2 e = s_st[sp * kBlock + tid];
-                    if (__uint_as_float(e.y) <= lim) cur = e.x;
+                    --w.sp;
+                    const uint2 e = s_st[w.sp * kBlock + tid];
+                    if (__uint_as_float(e.y) <= w.lim) w.cur = e.x;
                 }
             } else if (pop) {
-                --sp;
+                --w.sp;
                 uint2 e;
-                if (sp < LDS) e = s_st[sp * kBlock + tid];
-                else e = sp_st[min(sp - LDS, SPILL - 1)];
-                if (__uint_as_float(e.y) <= lim) cur = e.x;
+                if (w.sp < LDS) e = s_st[w.sp * kBlock + tid];
+                else e = sp_st[min(w.sp - LDS, SPILL - 1)];
+                if (__uint_as_float(e.y) <= w.lim) w.cur = e.x;
             }
-            if (walk && (int32_t)cur >= 0) {
-                const uint4* np = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(nodes) + (((cur << 1) + cur) << 4));
-                const uint4 q0 = np[0], q1 = np[1], q2 = np[2];
-                const uint32_t meta = q0.w;
-                const uint32_t ni = (meta >> 24) & 15u;
-                const float gx = __uint_as_float((meta & 0xffu) << 23) * s.rx;
-                const float gy = __uint_as_float(((meta >> 8) & 0xffu) << 23) * s.ry;
-                const float gz = __uint_as_float(((meta >> 16) & 0xffu) << 23) * s.rz;
-                const float bx = __uint_as_float(q0.x) * s.rx, by = __uint_as_float(q0.y) * s.ry,
-                            bz = __uint_as_float(q0.z) * s.rz;
-                const float nx = bx + s.ax, ny = by + s.ay, nz = bz + s.az;
-                const float fx = bx + s.bx, fy = by + s.by, fz = bz + s.bz;
-                const bool px = s.rx >= 0.0f, py = s.ry >= 0.0f, pz = s.rz >= 0.0f;
-                const uint32_t wnx = px ? q1.z : q1.w, wfx = px ? q1.w : q1.z;
-                const uint32_t wny = py ? q2.x : q2.y, wfy = py ? q2.y : q2.x;
-                const uint32_t wnz = pz ? q2.z : q2.w, wfz = pz ? q2.w : q2.z;
+            if (walk && (int32_t)w.cur >= 0) {
+                const NodeSlabs n(w.nodes, w.cur, w.s);
                 uint32_t key[4];
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    auto q = [&](uint32_t w) { return (float)((w >> (8 * j)) & 0xffu); };
-                    const float t0 = fmaxf(fmaxf(__builtin_fmaf(q(wnx), gx, nx), __builtin_fmaf(q(wny), gy, ny)),
-                                           fmaxf(__builtin_fmaf(q(wnz), gz, nz), r.tmin));
-                    const float t1 = fminf(fminf(__builtin_fmaf(q(wfx), gx, fx), __builtin_fmaf(q(wfy), gy, fy)),
-                                           fminf(__builtin_fmaf(q(wfz), gz, fz), lim));
-                    // distances are not negative: their bits order as they do; the slot rides in the last two
-                    key[j] = t0 <= t1 ? ((__float_as_uint(t0) & ~3u) | (uint32_t)j) : kNone;
-                }
-                const uint32_t leaf_at = (q1.y | REF_LEAF) - ni;
-                auto ref = [&](uint32_t k) {
-                    const uint32_t j = k & 3u;
-                    return (j < ni ? q1.x : leaf_at) + j;
-                };
+                for (uint32_t j = 0; j < 4; j++) key[j] = n.key(j, 8 * j, w.r.tmin, w.lim);
                 auto order = [&](uint32_t& x, uint32_t& y) {
                     const uint32_t lo = min(x, y), up = max(x, y);
                     x = lo;
@@ -495,80 +607,66 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                 order(key[1], key[2]);
                 // Farthest first. An entry that is no hit is written as well and then written over:
                 // the slot above the top is free.
-                if (__ballot(sp + 3 > LDS) == 0) {
+                if (__ballot(w.sp + 3 > LDS) == 0) {
 #pragma unroll
                     for (int i = 3; i >= 1; i--) {
-                        s_st[sp * kBlock + tid] = make_uint2(ref(key[i]), key[i]);
-                        sp += key[i] != kNone ? 1 : 0;
+                        s_st[w.sp * kBlock + tid] = make_uint2(n.ref(key[i]), key[i]);
+                        w.sp += key[i] != kNone ? 1 : 0;
                     }
                 } else {
 #pragma unroll
                     for (int i = 3; i >= 1; i--) {
                         if (key[i] == kNone) continue;
-                        const uint2 e = make_uint2(ref(key[i]), key[i]);
-                        if (sp < LDS) s_st[sp * kBlock + tid] = e;
-                        else if (sp < CAP) sp_st[sp - LDS] = e;
+                        const uint2 e = make_uint2(n.ref(key[i]), key[i]);
+                        if (w.sp < LDS) s_st[w.sp * kBlock + tid] = e;
+                        else if (w.sp < CAP) sp_st[w.sp - LDS] = e;
                         // not reached: the host sizes the stack for the tree
-                        if (sp < CAP) sp++;
+                        if (w.sp < CAP) w.sp++;
                         else overflow = true;
                     }
                 }
-                cur = key[0] != kNone ? ref(key[0]) : kNone;
+                w.cur = key[0] != kNone ? n.ref(key[0]) : kNone;
             }
-            if (cur != kNone && (int32_t)cur < 0 && leaf == kNone) {
-                leaf = cur;
-                cur = kNone;
+            if (w.at_leaf() && w.leaf == kNone) {
+                w.leaf = w.cur;
+                w.cur = kNone;
             }
         }
         // ---- leaf phase: the waiting leaves' triangles, one to a lane ----
         // Leaf number i of the wave has its A tested by lane 2i and its B by lane 2i + 1, with the ray
         // fetched from the lane that owns it: twenty leaves keep forty lanes busy for one triangle's
         // time, where their owners would take two. At most 32 leaves a round; others wait.
-        const uint64_t holders = __ballot(leaf != kNone);
+        const uint64_t holders = __ballot(w.leaf != kNone);
         if (holders == 0) continue;
         const uint32_t rank = (uint32_t)__popcll(holders & ((1ull << lane) - 1ull));
-        const bool mine = leaf != kNone && rank < 32u;
+        const bool mine = w.leaf != kNone && rank < 32u;
         // lane 2i learns which lane owns leaf i; lane 2i + 1 has it from its neighbour
         int owner = __builtin_amdgcn_ds_permute((int)((mine ? 2u * rank : 63u) << 2), mine ? (int)lane : -1);
-        owner = (int)quad_even((uint32_t)owner);
+        owner = (int)pair_even((uint32_t)owner);
         const bool tester = (lane >> 1) < (uint32_t)__popcll(holders);
         const int from = owner << 2;
         auto fetch = [&](float x) { return __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(x))); };
-        RayK w;
-        w.okx = fetch(r.okx); w.oky = fetch(r.oky); w.okz = fetch(r.okz);
-        w.sx = fetch(r.sx); w.sy = fetch(r.sy); w.sz = fetch(r.sz);
-        w.tmin = fetch(r.tmin);
-        w.tmax = fetch(r.tmax);
-        w.ky = __builtin_amdgcn_ds_bpermute(from, r.ky);
-        const uint32_t ri = leaf & ~REF_LEAF;
+        RayK r;
+        r.okx = fetch(w.r.okx); r.oky = fetch(w.r.oky); r.okz = fetch(w.r.okz);
+        r.sx = fetch(w.r.sx); r.sy = fetch(w.r.sy); r.sz = fetch(w.r.sz);
+        r.tmin = fetch(w.r.tmin);
+        r.tmax = fetch(w.r.tmax);
+        r.ky = __builtin_amdgcn_ds_bpermute(from, w.r.ky);
+        const uint32_t ri = w.leaf & ~REF_LEAF;
         const char* tp = nullptr;
         if (MULTI) {
-            const uint64_t at = reinterpret_cast<uint64_t>(recs + ri);
+            const uint64_t at = reinterpret_cast<uint64_t>(w.recs + ri);
             const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)(uint32_t)at);
             const uint32_t up = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)(uint32_t)(at >> 32));
             tp = reinterpret_cast<const char*>(((uint64_t)up << 32) | lo);
         } else {
             const uint32_t at = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)(ri * (uint32_t)sizeof(PrimRec)));
-            tp = reinterpret_cast<const char*>(recs) + at;
+            tp = reinterpret_cast<const char*>(w.recs) + at;
         }
         float t = FLT_INF, u = 0.f, v = 0.f;
         bool quad = false;
-        if (tester) {
-            w.kz = w.ky == 2 ? 0 : w.ky + 1;
-            w.kx = w.kz == 2 ? 0 : w.kz + 1;
-            const Float3* vp = reinterpret_cast<const Float3*>(tp + (lane & 1u) * sizeof(Tri));
-            const Float3 p0 = vp[0], p1 = vp[1], p2 = vp[2];
-            const Tri x{p0.x, p0.y, p0.z, p1.x, p1.y, p1.z, p2.x, p2.y, p2.z};
-            quad = __builtin_isnan(p1.x);  // a quad's record (no triangle of a walk tree holds a NaN)
-            float tt, uu, vv;
-            if (tri_test(w, x, tt, uu, vv)) {
-                t = tt;
-                u = uu;
-                v = vv;
-            }
-        }
-        // the nearer of A and B (A where they are equal), and the other one's distance
-        const float to = quad_swap(t), uo = quad_swap(u), vo = quad_swap(v);
+        if (tester) quad = record_tri(r, tp + (lane & 1u) * sizeof(Tri), t, u, v);
+        const float to = pair_swap(t), uo = pair_swap(u), vo = pair_swap(v);
         const bool take_b = to < t;  // as lane 2i sees it
         float other = take_b ? t : (to == t ? FLT_INF : to);
         if (quad) other = -1.0f;
@@ -578,56 +676,136 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         const float ro = result(other);
         const bool rb = __builtin_amdgcn_ds_bpermute(back, take_b ? 1 : 0) != 0;
         if (mine) {
-            leaf = kNone;
-            if (cur != kNone && (int32_t)cur < 0) {
-                leaf = cur;
-                cur = kNone;
+            w.leaf = kNone;
+            if (w.at_leaf()) {
+                w.leaf = w.cur;
+                w.cur = kNone;
             }
-            // A tie of two triangles of one Fast-BVH leaf (a mesh with doubled faces has one at every
-            // hit): the one that comes first there wins. False: not such a tie.
-            auto same_leaf_order = [&](uint32_t which, float tie_u, float tie_v) {
-                const TreeView& tv = MULTI ? a.trees[a.ray_scene[ray_id]] : a.tree;
-                if ((recs[ri].id_a & PR_FLAG) || (recs[hit >> 1].id_a & PR_FLAG)) return false;
-                if (ri == hit >> 1) return true;  // the same record again
-                const WalkAux &x = tv.waux[ri], &y = tv.waux[hit >> 1];
-                const uint32_t px = (x.places >> (16u * which)) & 0xffffu, py = (y.places >> (16u * (hit & 1u))) & 0xffffu;
-                if (x.leaf != y.leaf || px == 0xffffu || py == 0xffffu) return false;
-                if (px < py) {
-                    hit = 2 * ri + which;
-                    bu = tie_u;
-                    bv = tie_v;
-                }
-                return true;
-            };
-            auto found = [&](float ft, float fu, float fv, uint32_t which) {
-                if (ft < bt) {
-                    second = bt;
-                    bt = ft;
-                    bu = fu;
-                    bv = fv;
-                    hit = 2 * ri + which;
-                    lim = ft + (slack + 4e-7f * ft);
-                } else if (!ANY && !(ft == bt && same_leaf_order(which, fu, fv))) {
-                    second = fminf(second, ft);
-                }
-            };
-            if (ro < 0.0f) {
-                const TreeView& tv = MULTI ? a.trees[a.ray_scene[ray_id]] : a.tree;
-                RayK q;
-                load_ray(a.rays, ray_id, q);
-                float ft;
-                if (quad_test(q, tv.quads[__float_as_uint(recs[ri].a.p0x)], FLT_MAX, ft)) found(ft, 0.f, 0.f, 0u);
-            } else if (rt < FLT_INF) {
-                found(rt, ru, rv, rb ? 1u : 0u);
-                second = fminf(second, ro);
-            }
-            if (ANY && hit != kNone) {
-                sp = 0;
-                cur = leaf = kNone;
-            }
+            leaf_outcome<ANY, MULTI>(a, w, ri, rt, ru, rv, ro, rb ? 1u : 0u);
         }
     }
     if (overflow) atomicOr(a.error, kFlagStackOverflow);
+}
+
+// One ray to four lanes (a child of its node each, a triangle to every other one): batches too small
+// to fill the chip, where the time is that of the longest rays' chains of steps. A step has half
+// the instructions of walk_lanes', and a wave's 16 rays wait less for one another.
+// All four lanes hold the same walker. The stack has kQuadStack entries in LDS, [entry][ray].
+// Against walk_lanes: 1,000 rays in the Cornell room 41 -> 29 us, 64 rays through 50K triangles 132 -> 89,
+// 65K 165 -> 131, 100K 182 -> 156; at 32 rays a wave (131K) it takes 182 -> 183, the Cornell room
+// 78 -> 94, at 49 (200K) 193 -> 239: four rays' worth of lanes for one stops paying once the chip is full.
+constexpr int kQuadStack = 64;
+template <bool ANY, bool MULTI, int SPILL>
+__device__ __forceinline__ void walk_quads(const TraceArgs& a, uint32_t n_rays, uint2* s_st, uint32_t* s_next) {
+    uint2 exact_st[SPILL];
+    const uint32_t lane = __lane_id();
+    const uint32_t sub = lane & 3u;
+    const uint32_t waves = gridDim.x * (kBlock / 64);
+    const uint32_t seats = min((n_rays + waves - 1) / waves, 16u);
+    const uint32_t share = (n_rays + gridDim.x - 1) / gridDim.x;
+    if (threadIdx.x == 0) *s_next = 0;
+    __syncthreads();
+    uint2* st = s_st + (threadIdx.x >> 6) * (kQuadStack * 16) + (lane >> 2);
+    bool more = (lane >> 2) < seats, overflow = false;
+    Walker w;
+    w.nodes = a.tree.wnodes;
+    w.recs = a.tree.wrecs;
+    w.cur = w.leaf = w.ray_id = w.hit = kNone;
+    w.bt = w.lim = w.second = FLT_MAX;
+    w.bu = w.bv = w.slack = 0.f;
+    w.sp = 0;
+    w.open = false;
+    while (true) {
+        const bool idle = w.idle();
+        const uint64_t want = __ballot(idle && (more || w.ray_id != kNone));
+        const uint64_t busy = __ballot(!idle);
+        if (want == 0 && busy == 0) break;
+        if (want != 0 && (busy == 0 || (uint32_t)__popcll(want) >= 16u)) {
+            if (idle && w.ray_id != kNone) {
+                if (sub == 0) settle<ANY, MULTI>(a, w, exact_st);
+                w.ray_id = kNone;
+            }
+            const uint64_t take = __ballot(idle && more && sub == 0);
+            if (take != 0) {
+                uint32_t v = 0;
+                if (lane == 0) v = atomicAdd(s_next, (uint32_t)__popcll(take));
+                v = __builtin_amdgcn_readfirstlane(v) + (uint32_t)__popcll(take & ((1ull << (lane & ~3u)) - 1ull));
+                const uint32_t k = blockIdx.x * share + v;
+                if (idle && more) {
+                    if (v < share && k < n_rays) start<ANY, MULTI>(a, a.order ? a.order[k] : k, w);
+                    else more = false;
+                }
+            }
+            continue;
+        }
+        const uint32_t batch = ((uint32_t)__popcll(busy) + 3u) / 4u;
+        while (true) {
+            const bool walk = w.walking();
+            if (__ballot(walk) == 0 || (uint32_t)__popcll(__ballot(w.leaf != kNone)) >= batch) break;
+            if (walk && w.cur == kNone) {
+                --w.sp;
+                const uint2 e = st[w.sp * 16];
+                if (__uint_as_float(e.y) <= w.lim) w.cur = e.x;
+            }
+            if (walk && (int32_t)w.cur >= 0) {
+                const NodeSlabs n(w.nodes, w.cur, w.s);
+                const uint32_t key = n.key(sub, 8 * sub, w.r.tmin, w.lim);
+                const uint32_t k1 = quad_rot<0x39>(key), k2 = quad_rot<0x4E>(key), k3 = quad_rot<0x93>(key);
+                const uint32_t nearest = min(min(key, k1), min(k2, k3));
+                // place of this lane's child: hits farther than it lie below
+                const int below = (k1 != kNone && k1 > key ? 1 : 0) + (k2 != kNone && k2 > key ? 1 : 0) +
+                                  (k3 != kNone && k3 > key ? 1 : 0);
+                const int hits = (key != kNone ? 1 : 0) + (k1 != kNone ? 1 : 0) + (k2 != kNone ? 1 : 0) +
+                                 (k3 != kNone ? 1 : 0);
+                if (key != kNone && key != nearest) {
+                    // always: the host takes this form for trees whose stack fits
+                    if (w.sp + below < kQuadStack) st[(w.sp + below) * 16] = make_uint2(n.ref(key), key);
+                    else overflow = true;
+                }
+                w.sp = min(w.sp + max(hits - 1, 0), kQuadStack);
+                w.cur = nearest != kNone ? n.ref(nearest) : kNone;
+            }
+            if (w.at_leaf() && w.leaf == kNone) {
+                w.leaf = w.cur;
+                w.cur = kNone;
+            }
+        }
+        if (w.leaf != kNone) {
+            const uint32_t ri = w.leaf & ~REF_LEAF;
+            w.leaf = kNone;
+            if (w.at_leaf()) {
+                w.leaf = w.cur;
+                w.cur = kNone;
+            }
+            float t = FLT_INF, u = 0.f, v = 0.f;
+            const bool quad = record_tri(w.r, reinterpret_cast<const char*>(w.recs + ri) + (sub & 1u) * sizeof(Tri), t, u, v);
+            const float to = pair_swap(t), uo = pair_swap(u), vo = pair_swap(v);
+            // (every lane takes part in the exchange: a lane left out would hand its neighbour a zero)
+            const float quad_there = pair_swap(quad ? 1.0f : 0.0f);
+            const bool quad_any = quad | (quad_there != 0.0f);
+            const bool odd = (sub & 1u) != 0;
+            const float ta = odd ? to : t, tb = odd ? t : to;
+            const bool take_b = tb < ta;
+            const bool own = take_b == odd;  // this lane tested the nearer one
+            leaf_outcome<ANY, MULTI>(a, w, ri, take_b ? tb : ta, own ? u : uo, own ? v : vo,
+                                     quad_any ? -1.0f : take_b ? ta : (ta == tb ? FLT_INF : tb), take_b ? 1u : 0u);
+        }
+    }
+    if (overflow) atomicOr(a.error, kFlagStackOverflow);
+}
+
+// 4 waves per SIMD (128 VGPRs): 5 spilled in the rarely taken parts and gained nothing.
+template <bool ANY, bool MULTI, int LDS, int SPILL>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_walk(TraceArgs a) {
+    __shared__ uint2 s_st[LDS * kBlock];  // stacks: (reference, entry distance)
+    __shared__ uint32_t s_next, s_out;
+    static_assert(LDS < 16 || LDS * kBlock >= kQuadStack * 16 * (kBlock / 64), "the quads' stacks fit");
+    const uint32_t n_rays = a.n_dev ? *a.n_dev : a.n;
+    const uint32_t stack = MULTI ? a.walk_stack : a.tree.walk_stack;
+    if (LDS >= 16 && stack <= (uint32_t)kQuadStack && n_rays <= kQuadsPerWave * gridDim.x * (kBlock / 64))
+        walk_quads<ANY, MULTI, SPILL>(a, n_rays, s_st, &s_next);
+    else
+        walk_lanes<ANY, MULTI, LDS, SPILL>(a, n_rays, s_st, &s_next, &s_out);
 }
 
 __global__ void k_walk_reset(uint32_t* counter) {
@@ -637,17 +815,24 @@ __global__ void k_walk_reset(uint32_t* counter) {
 template <bool ANY, bool MULTI, int LDS, int SPILL>
 hipError_t launch(const TraceArgs& a, hipStream_t stream, int num_cus) {
     auto kern = k_walk<ANY, MULTI, LDS, SPILL>;
-    int per_cu = 0;
-    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kBlock, 0);
-    if (e != hipSuccess) return e;
-    if (per_cu < 1) per_cu = 1;
+    // asked once: the answer is the kernel's and the architecture's
+    static std::atomic<int> resident{0};
+    int per_cu = resident.load(std::memory_order_relaxed);
+    if (per_cu < 1) {
+        hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kBlock, 0);
+        if (e != hipSuccess) return e;
+        if (per_cu < 1) per_cu = 1;
+        resident.store(per_cu, std::memory_order_relaxed);
+    }
     if (a.blocks_per_cu && (int)a.blocks_per_cu < per_cu) per_cu = (int)a.blocks_per_cu;
-    // as many waves as run at once, down to four rays each
-    const uint64_t want = ((uint64_t)a.n + 15) / 16;
+    // as many waves as run at once, down to one ray each
+    const uint64_t want = ((uint64_t)a.n + 3) / 4;
     uint64_t grid = (uint64_t)num_cus * (uint64_t)per_cu;
     if (want < grid) grid = want;
     if (grid < 1) grid = 1;
-    hipLaunchKernelGGL(k_walk_reset, dim3(1), dim3(64), 0, stream, a.counter);
+    // a batch that the workgroups' shares cover never asks the counter (saves a launch, about 5 us)
+    if (a.n >= kDealtPerWave * (kBlock / 64) * grid)
+        hipLaunchKernelGGL(k_walk_reset, dim3(1), dim3(64), 0, stream, a.counter);
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kBlock), 0, stream, a);
     return hipGetLastError();
 }

@@ -86,6 +86,11 @@ __host__ __device__ __forceinline__ Rng4 rng4(uint32_t seed, uint32_t pixel, uin
     const U4 r = philox4x32_10(U4{sample, bounce, call, 0u}, seed, pixel);
     return Rng4{u01(r.x), u01(r.y), u01(r.z), u01(r.w)};
 }
+// Four draws, computed when asked for.
+struct Draw {
+    uint32_t seed, pixel, sample, bounce, call;
+    __device__ __forceinline__ Rng4 operator()() const { return rng4(seed, pixel, sample, bounce, call); }
+};
 // Draw assignment per vertex (bounce b): call 0 = light pick, light u, light v, NEE bxdf pick;
 // call 1 = NEE bsdf (t, u, v), continuation bxdf pick; call 2 = continuation bsdf (t, u, v), RR;
 // call 3 / 4 = fresh samples drawn inside the NEE / continuation BSDF sampling (dielectric,
@@ -525,7 +530,10 @@ __device__ __forceinline__ float mat_pdf(const MatRec& m, V3 wo, V3 wi) {
     }
 }
 // bs = (t, u, v) of the BsdfSample; fr = 4 fresh draws (dielectric: t,u,v; Disney: r,u,v).
-__device__ __forceinline__ BsdfSampleOut mat_sample(const MatRec& m, V3 wo, float bs_u, float bs_v, Rng4 fr) {
+// `fresh` names the draws of the materials that take fresh ones; the others do not compute them.
+__device__ __forceinline__ BsdfSampleOut mat_sample(const MatRec& m, V3 wo, float bs_u, float bs_v, const Draw& fresh) {
+    Rng4 fr = {0.f, 0.f, 0.f, 0.f};
+    if (m.type != MAT_LAMBERT && m.type != MAT_GGX && m.type != MAT_TRANSPARENT) fr = fresh();
     switch (m.type) {
         case MAT_LAMBERT: {
             BsdfSampleOut o;

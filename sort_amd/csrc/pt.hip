@@ -46,22 +46,23 @@ __device__ __forceinline__ int sample_discrete(const float* cdf, uint32_t count,
     return (int)off;
 }
 
-// Where a workgroup's threads append to two queues: one atomic per queue and workgroup. Every thread of
-// the workgroup calls it, `turn` counting the calls. A thread adds up to one entry to the first
-// queue and two to the second, in thread order within its wave (its first entry of the second queue
-// before the wave's second ones).
+// Where a workgroup's threads append to two queues whose counts lie side by side: one 64-bit atomic per
+// workgroup. Every thread of the workgroup calls it, `turn` counting the calls. A thread adds up to
+// one entry to the first queue and two to the second, in thread order within its wave (the wave's
+// first entries of the second queue before its second ones).
 // An atomic on one address takes about 8.5 ns of the whole chip's time, so three atomics per wave bound
 // the shading of a million paths at 0.4 ms a bounce, whatever it computed. A 256 x 256 Cornell frame of
-// 16 samples, depth 5: 3.57 ms with those, 2.66 with two atomics per workgroup; 640 x 480 and 24 samples of
-// 512,002 triangles of spheres, depth 8: 8.60 and 7.07 ms.
+// 16 samples, depth 5: 3.57 ms with those, 2.66 with two atomics per workgroup, 2.59 with one; 640 x 480
+// and 24 samples of 512,002 triangles of spheres, depth 8: 8.60, 7.07 and 7.02 ms.
 struct AppendSlots {
     uint32_t a, b0, b1;
 };
 struct AppendShared {
-    uint32_t cnt[2][2][kPtBlock / 64], base[2];
+    uint32_t cnt[2][2][kPtBlock / 64];
+    unsigned long long base;
 };
 __device__ __forceinline__ AppendSlots block_append(AppendShared& sh, uint32_t turn, bool a, bool b0, bool b1,
-                                                    uint32_t* count_a, uint32_t* count_b) {
+                                                    uint32_t* counts) {
     const uint32_t lane = __lane_id(), wave = threadIdx.x / 64;
     const uint64_t ma = __ballot(a), m0 = __ballot(b0), m1 = __ballot(b1);
     const uint64_t below = (1ull << lane) - 1ull;
@@ -83,13 +84,14 @@ __device__ __forceinline__ AppendSlots block_append(AppendShared& sh, uint32_t t
             all[k] += c;
         }
     }
-    if (threadIdx.x == 0 && all[0]) sh.base[0] = atomicAdd(count_a, all[0]);
-    if (threadIdx.x == 64 && all[1]) sh.base[1] = atomicAdd(count_b, all[1]);
+    if (threadIdx.x == 0 && (all[0] | all[1]))
+        sh.base = atomicAdd(reinterpret_cast<unsigned long long*>(counts), all[0] | (unsigned long long)all[1] << 32);
     __syncthreads();
     AppendSlots s;
-    s.a = sh.base[0] + before[0] + (uint32_t)__popcll(ma & below);
-    s.b0 = sh.base[1] + before[1] + (uint32_t)__popcll(m0 & below);
-    s.b1 = sh.base[1] + before[1] + (uint32_t)(__popcll(m0) + __popcll(m1 & below));
+    const uint32_t base_a = (uint32_t)sh.base, base_b = (uint32_t)(sh.base >> 32);
+    s.a = base_a + before[0] + (uint32_t)__popcll(ma & below);
+    s.b0 = base_b + before[1] + (uint32_t)__popcll(m0 & below);
+    s.b1 = base_b + before[1] + (uint32_t)(__popcll(m0) + __popcll(m1 & below));
     return s;
 }
 
@@ -118,10 +120,14 @@ __device__ __forceinline__ void init_path(PathState ps, uint32_t p, uint32_t pix
 // Camera rays of every chunk (PerspectiveCamera::GenerateRay in closed form: raster -> camera
 // through the inverse of Scale(W,H,1) Scale(.5,-.5,1) Translate(1,-1,0) Perspective(xs, ys),
 // then the orthonormal ViewLookat basis).
+__device__ __forceinline__ void init_counts(uint32_t* count, uint32_t paths) {
+    count[0] = paths;
+    for (int k = 1; k < 6; k++) count[k] = 0;
+}
 __global__ __launch_bounds__(kPtBlock) void k_raygen(const WaveDesc* __restrict__ w, PathState ps, Queues q) {
     const ChunkTable& ct = w->ct;
     const uint32_t p = blockIdx.x * kPtBlock + threadIdx.x;
-    if (p == 0) q.count[0] = ct.total_paths;
+    if (p == 0) init_counts(q.count, ct.total_paths);
     if (p >= ct.total_paths) return;
     const ChunkDev& c = ct.c[chunk_of_path(ct, p)];
     const ReqDev& R = w->reqs[c.req];
@@ -147,7 +153,7 @@ __global__ __launch_bounds__(kPtBlock) void k_raygen(const WaveDesc* __restrict_
 __global__ __launch_bounds__(kPtBlock) void k_raygen_rays(const float4* rays, const uint32_t* keys, uint32_t n,
                                                           const ReqDev* __restrict__ reqs, PathState ps, Queues q) {
     const uint32_t p = blockIdx.x * kPtBlock + threadIdx.x;
-    if (p == 0) q.count[0] = n;
+    if (p == 0) init_counts(q.count, n);
     if (p >= n) return;
     q.ray[0][2 * p] = rays[2 * p];
     q.ray[0][2 * p + 1] = rays[2 * p + 1];
@@ -156,17 +162,10 @@ __global__ __launch_bounds__(kPtBlock) void k_raygen_rays(const float4* rays, co
     init_path(ps, p, keys[2 * p], keys[2 * p + 1], 0u);
 }
 
-__global__ void k_zero_counts(uint32_t* count, int which) {
-    if (threadIdx.x == 0) {
-        count[which] = 0;
-        count[2] = 0;
-    }
-}
-
 // Records the extension rays of the current queue and their hits into the ray dump (paths of
 // pixels in the dump's range only).
 __global__ __launch_bounds__(kPtBlock) void k_dump(uint32_t bounce, int cur, PathState ps, Queues q, RayDumpDev d) {
-    const uint32_t n = q.count[cur];
+    const uint32_t n = q.count[2 * cur];
     for (uint32_t i = blockIdx.x * kPtBlock + threadIdx.x; i < n; i += gridDim.x * kPtBlock) {
         const uint32_t p = q.pid[cur][i];
         const float4* pr = ps.rec + 4 * (size_t)p;
@@ -180,10 +179,13 @@ __global__ __launch_bounds__(kPtBlock) void k_dump(uint32_t bounce, int cur, Pat
     }
 }
 
-__global__ void k_add_totals(const uint32_t* count, int ext_slot, unsigned long long* totals) {
+// Ends a bounce: its rays join the totals, and the next bounce's counts and the work counters of its
+// two traversals start from 0. One launch for what were four, at about 5 us each.
+__global__ void k_end_bounce(uint32_t* count, int cur, unsigned long long* totals) {
     if (threadIdx.x == 0) {
-        totals[0] += count[ext_slot];
-        totals[1] += count[2];
+        totals[0] += count[2 * cur];
+        totals[1] += count[2 * (cur ^ 1) + 1];
+        count[2 * cur] = count[2 * cur + 1] = count[4] = count[5] = 0;
     }
 }
 
@@ -294,7 +296,7 @@ __global__ __launch_bounds__(256) void k_sort_count(int cur, const TreeView* tre
     __shared__ uint32_t h[kSortBuckets];
     for (uint32_t j = threadIdx.x; j < kSortBuckets; j += 256) h[j] = 0;
     __syncthreads();
-    const uint32_t n = q.count[cur];
+    const uint32_t n = q.count[2 * cur];
     const uint32_t chunk = (n + kSortBlocks - 1) / kSortBlocks;
     const uint32_t lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
     for (uint32_t i = lo + threadIdx.x; i < hi; i += 256) {
@@ -365,7 +367,7 @@ __global__ __launch_bounds__(256) void k_sort_scatter(int cur, Queues q) {
     for (uint32_t j = threadIdx.x; j < kSortBuckets; j += 256)
         off[j] = q.sbase[j] + q.shist[blockIdx.x * kSortBuckets + j];
     __syncthreads();
-    const uint32_t n = q.count[cur];
+    const uint32_t n = q.count[2 * cur];
     const uint32_t chunk = (n + kSortBlocks - 1) / kSortBlocks;
     const uint32_t lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
     for (uint32_t i = lo + threadIdx.x; i < hi; i += 256) q.sperm[atomicAdd(&off[q.skey[i]], 1u)] = i;
@@ -373,11 +375,14 @@ __global__ __launch_bounds__(256) void k_sort_scatter(int cur, Queues q) {
 
 // ---- shade -------------------------------------------------------------------------------------
 // `order` (or null): the queue entries in the order to shade them.
-__global__ __launch_bounds__(kPtBlock) void k_shade(const SceneDev* __restrict__ scenes,
+// Gathers of vertices, materials and path records bound it: 4 waves per SIMD (128 VGPRs, 32 bytes of
+// scratch) instead of the 3 of 138 VGPRs take the Cornell frame above from 2.59 to 2.56 ms, the spheres
+// from 7.02 to 6.98.
+__global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_shade(const SceneDev* __restrict__ scenes,
                                                     const ReqDev* __restrict__ reqs, uint32_t bounce, int cur,
                                                     PathState ps, Queues q, const uint32_t* __restrict__ order) {
     __shared__ AppendShared append;
-    const uint32_t n = q.count[cur];
+    const uint32_t n = q.count[2 * cur];
     const int nxt = cur ^ 1;
     uint32_t turn = 0;
     for (uint32_t base = blockIdx.x * kPtBlock; base < n; base += gridDim.x * kPtBlock) {
@@ -517,7 +522,7 @@ __global__ __launch_bounds__(kPtBlock) void k_shade(const SceneDev* __restrict__
             pr[3] = c1;
         }
         // compaction of survivors and shadow rays
-        const AppendSlots slot = block_append(append, turn++, cont, sh0, sh1, &q.count[nxt], &q.count[2]);
+        const AppendSlots slot = block_append(append, turn++, cont, sh0, sh1, &q.count[2 * nxt]);
         if (cont) {
             const uint32_t ci = slot.a;
             put_ray(q.ray[nxt], ci, ro, 0.0001f, rd, FLT_MAX);
@@ -544,8 +549,9 @@ __global__ __launch_bounds__(kPtBlock) void k_shade(const SceneDev* __restrict__
 // first half of its ray record; a black one clears its contribution slot, any other scales it
 // (EvaluateDirect's attenuation factor, integratormethod.cpp:134-142 and 181-185; applied here to
 // the finished contribution instead of first in the product, which moves float rounding only).
-__global__ __launch_bounds__(kPtBlock) void k_resolve_att(PathState ps, Queues q) {
-    const uint32_t n = q.count[2];
+__global__ __launch_bounds__(kPtBlock) void k_resolve_att(PathState ps, Queues q,
+                                                          const uint32_t* __restrict__ n_shadow) {
+    const uint32_t n = *n_shadow;
     for (uint32_t i = blockIdx.x * kPtBlock + threadIdx.x; i < n; i += gridDim.x * kPtBlock) {
         const float4 a = q.sray[2 * (size_t)i];
         float4* c = ps.rec + path_slot(q.ssid[i]);
@@ -636,7 +642,7 @@ hipError_t pt_bounces(const PtLaunch& L, uint32_t npaths, hipStream_t s) {
     const unsigned shade_blocks = std::min<unsigned>(blocks_for(npaths), (unsigned)L.num_cus * 8u);
     hipError_t e;
     for (uint32_t b = 0; b < L.max_depth; b++) {
-        const int cur = (int)(b & 1u), nxt = cur ^ 1;
+        const int cur = (int)(b & 1u);
         hipEvent_t* tev = nullptr;  // this bounce's six stage events, when timed
         if (L.stage_ev && *L.stage_used + 6 <= L.stage_cap) {
             tev = L.stage_ev + *L.stage_used;
@@ -646,8 +652,10 @@ hipError_t pt_bounces(const PtLaunch& L, uint32_t npaths, hipStream_t s) {
         TraceArgs ta = L.trace;
         ta.rays = L.q.ray[cur];
         ta.n = npaths;
-        ta.n_dev = &L.q.count[cur];
+        ta.n_dev = &L.q.count[2 * cur];
         ta.out = L.q.hit;
+        ta.counter = L.q.count + 4;
+        ta.counter_clear = true;
         if (L.trees) {
             ta.trees = L.trees;
             ta.ray_scene = L.q.rsc[cur];
@@ -660,7 +668,6 @@ hipError_t pt_bounces(const PtLaunch& L, uint32_t npaths, hipStream_t s) {
             (e = mark(1)) != hipSuccess)
             return e;
         if (L.dump.rays) hipLaunchKernelGGL(k_dump, dim3(shade_blocks), dim3(kPtBlock), 0, s, b, cur, L.ps, L.q, L.dump);
-        hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, s, L.q.count, nxt);
         const uint32_t* order = nullptr;
         if (L.sort_min && npaths >= L.sort_min && L.q.sperm) {
             SortBox box;
@@ -682,8 +689,9 @@ hipError_t pt_bounces(const PtLaunch& L, uint32_t npaths, hipStream_t s) {
             return e;
         TraceArgs sa = ta;
         sa.rays = L.q.sray;
+        sa.counter = L.q.count + 5;
         sa.n = 2 * npaths;
-        sa.n_dev = &L.q.count[2];
+        sa.n_dev = &L.q.count[2 * (cur ^ 1) + 1];
         if (L.trees ? L.transps != nullptr : L.transp != nullptr) {
             // Visibility::GetAttenuation: each walk's result overwrites its own ray's first half
             // (a lane reads its ray before it writes the result, and no other lane reads it)
@@ -696,7 +704,8 @@ hipError_t pt_bounces(const PtLaunch& L, uint32_t npaths, hipStream_t s) {
                 sa.transp = L.transp;
             }
             if ((e = launch_attenuation(sa, s, L.num_cus)) != hipSuccess) return e;
-            hipLaunchKernelGGL(k_resolve_att, dim3(shade_blocks), dim3(kPtBlock), 0, s, L.ps, L.q);
+            hipLaunchKernelGGL(k_resolve_att, dim3(shade_blocks), dim3(kPtBlock), 0, s, L.ps, L.q,
+                               sa.n_dev);
         } else {
             // occluded shadow rays clear their contribution slots inside the any-hit launch
             sa.out = nullptr;
@@ -706,7 +715,7 @@ hipError_t pt_bounces(const PtLaunch& L, uint32_t npaths, hipStream_t s) {
             if ((e = launch_trace(sa, true, false, s, L.num_cus)) != hipSuccess) return e;
         }
         if ((e = mark(5)) != hipSuccess) return e;
-        hipLaunchKernelGGL(k_add_totals, dim3(1), dim3(64), 0, s, L.q.count, cur, L.q.totals);
+        hipLaunchKernelGGL(k_end_bounce, dim3(1), dim3(64), 0, s, L.q.count, cur, L.q.totals);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     return hipSuccess;

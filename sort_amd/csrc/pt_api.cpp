@@ -72,8 +72,6 @@ PtLaunch make_launch(sortgpu_scene* sc, const WaveDesc* d_wave, uint32_t max_dep
     std::memset(&L, 0, sizeof(L));
     sortgpu_accel* acc = sc->accel;
     L.trace.tree = acc->view;
-    const uint32_t slot = acc->slot.fetch_add(1) % kCounterSlots;
-    L.trace.counter = acc->d_counters + slot * kCounterStride;
     L.trace.error = acc->d_error;
     L.trace.stats = nullptr;
     apply_tuning(acc->ctx, L.trace);

@@ -18,7 +18,7 @@ struct RayDumpDev {
 };
 
 struct PtLaunch {
-    TraceArgs trace;            // counter / error slots and tuning; the single tree when trees == null
+    TraceArgs trace;            // error slot and tuning; the single tree when trees == null
     const SceneDev* scenes;     // device scene table
     const WaveDesc* wave;       // device wave descriptor (chunks + request table)
     const TreeView* trees;      // device tree table for multi-scene waves, or null

@@ -87,7 +87,8 @@ struct Queues {
     float4* sray;       // shadow rays
     uint32_t* ssid;     // shadow slot: 2 * path + k
     uint32_t* ssc;      // scene of each shadow entry
-    uint32_t* count;    // [0],[1] extension queue counts, [2] shadow count
+    uint32_t* count;    // [2c] length of extension queue c, [2c + 1] shadow rays of the shading that filled it;
+                        // [4],[5] work counters of the extension and the shadow traversal
     unsigned long long* totals;  // [0] extension rays, [1] shadow rays
     // spatial order of a bounce's hits (bucket sort): bucket per entry, the order, per-block bucket
     // counts (kSortBlocks x kSortBuckets) and bucket bases (kSortBuckets)

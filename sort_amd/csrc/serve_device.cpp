@@ -68,7 +68,6 @@ class HipDevice : public Device {
             return (err = hip_msg("hipEventCreate", e), hip_rc(e));
         if ((rc = ring_.init(ctx_))) return (err = "request ring allocation failed", rc);
         const size_t sb = (size_t)max_scenes_ * sizeof(SceneDev), tb = (size_t)max_scenes_ * sizeof(TreeView);
-        const size_t cb = (size_t)kCounterSlots * kCounterStride * sizeof(uint32_t);
         void* p = nullptr;
         if ((e = hipMalloc(&p, sb)) != hipSuccess) return (err = hip_msg("hipMalloc(scene table)", e), hip_rc(e));
         d_scenes_ = static_cast<SceneDev*>(p);
@@ -77,9 +76,8 @@ class HipDevice : public Device {
         const size_t pb = (size_t)max_scenes_ * sizeof(const float*);
         if ((e = hipMalloc(&p, pb)) != hipSuccess) return (err = hip_msg("hipMalloc(transparency table)", e), hip_rc(e));
         d_transps_ = static_cast<const float**>(p);
-        if ((e = hipMalloc(&p, cb + 256)) != hipSuccess) return (err = hip_msg("hipMalloc(counters)", e), hip_rc(e));
-        d_counters_ = static_cast<uint32_t*>(p);
-        d_error_ = d_counters_ + cb / sizeof(uint32_t);
+        if ((e = hipMalloc(&p, 256)) != hipSuccess) return (err = hip_msg("hipMalloc(error)", e), hip_rc(e));
+        d_error_ = static_cast<uint32_t*>(p);
         if ((e = hipHostMalloc(&p, sb, hipHostMallocDefault)) != hipSuccess)
             return (err = hip_msg("hipHostMalloc(scene table)", e), hip_rc(e));
         h_scenes_ = static_cast<SceneDev*>(p);
@@ -95,13 +93,13 @@ class HipDevice : public Device {
         if ((e = hipMemcpy(d_scenes_, h_scenes_, sb, hipMemcpyHostToDevice)) != hipSuccess ||
             (e = hipMemcpy(d_trees_, h_trees_, tb, hipMemcpyHostToDevice)) != hipSuccess ||
             (e = hipMemcpy(d_transps_, h_transps_, pb, hipMemcpyHostToDevice)) != hipSuccess ||
-            (e = hipMemset(d_counters_, 0, cb + 256)) != hipSuccess)
+            (e = hipMemset(d_error_, 0, 256)) != hipSuccess)
             return (err = hip_msg("table initialisation", e), hip_rc(e));
         for (uint32_t i = 0; i < ns_; i++)
             if ((e = pt_zero_f4(reinterpret_cast<float4*>(ws_[i].q.totals), 1, s_[i])) != hipSuccess ||
                 (e = hipStreamSynchronize(s_[i])) != hipSuccess)
                 return (err = hip_msg("workspace initialisation", e), hip_rc(e));
-        fixed_ = sb + tb + pb + cb + 256 + (size_t)ReqRing::kSlots * sizeof(WaveDesc);
+        fixed_ = sb + tb + pb + 256 + (size_t)ReqRing::kSlots * sizeof(WaveDesc);
         for (uint32_t i = 0; i < ns_; i++) fixed_ += ws_[i].mem.bytes + sizeof(WaveDesc);
         return SORTGPU_OK;
     }
@@ -121,7 +119,7 @@ class HipDevice : public Device {
         for (uint32_t i = 0; i < ns_; i++) ws_[i].release();
         if (d_scenes_) hipFree(d_scenes_);
         if (d_trees_) hipFree(d_trees_);
-        if (d_counters_) hipFree(d_counters_);
+        if (d_error_) hipFree(d_error_);
         if (h_scenes_) hipHostFree(h_scenes_);
         if (h_trees_) hipHostFree(h_trees_);
         if (d_transps_) hipFree(d_transps_);
@@ -387,12 +385,11 @@ class HipDevice : public Device {
         hipEvent_t a, b;
     };
 
-    // Launch parameters of the waves of stream k: its workspace, its descriptor and its own work
-    // counter (waves of one stream run one after another).
+    // Launch parameters of the waves of stream k: its workspace and its descriptor (waves of one stream
+    // run one after another).
     PtLaunch wave_launch(uint32_t k, uint32_t depth, bool att, bool walk) const {
         PtLaunch L;
         std::memset(&L, 0, sizeof(L));
-        L.trace.counter = d_counters_ + k * kCounterStride;
         L.trace.error = d_error_;
         apply_tuning(ctx_, L.trace);
         L.scenes = d_scenes_;
@@ -502,7 +499,6 @@ class HipDevice : public Device {
     TreeView* h_trees_ = nullptr;
     const float** d_transps_ = nullptr;  // per scene: its transparency table on the device, or null
     const float** h_transps_ = nullptr;
-    uint32_t* d_counters_ = nullptr;
     uint32_t* d_error_ = nullptr;
     uint32_t slot_ = 0;
     std::vector<SceneHost> scenes_;

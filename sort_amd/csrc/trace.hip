@@ -441,7 +441,7 @@ static hipError_t launch_one(const TraceArgs& a, hipStream_t stream, int num_cus
     uint64_t grid = (uint64_t)num_cus * (uint64_t)per_cu;
     if (want < grid) grid = want;
     if (grid < 1) grid = 1;
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, stream, a.counter);
+    if (!a.counter_clear) hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, stream, a.counter);
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kBlock), 0, stream, a);
     return hipGetLastError();
 }

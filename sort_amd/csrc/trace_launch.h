@@ -13,7 +13,7 @@ struct TraceArgs {
     uint32_t n;                    // ray count, or the capacity when n_dev is set
     const uint32_t* n_dev;         // optional device-side ray count (read at kernel start)
     void* out;                     // closest: n x 16 B hits; any: n x u8 (device)
-    uint32_t* counter;             // work counter (device), reset by the launch
+    uint32_t* counter;             // work counter (device), reset by the launch unless counter_clear
     uint32_t* error;               // error flags (device): kFlag* bits
     unsigned long long* stats;     // 5 counters (device), only with stats
     // multi-scene form: trees != null selects it
@@ -29,6 +29,7 @@ struct TraceArgs {
     uint32_t blocks_per_cu;        // cap on resident workgroups per CU (default: occupancy limit)
     uint32_t leaf_batch;           // lanes holding a leaf that end a node phase (default 32)
     uint32_t leaf_min;             // a leaf phase ends below this many lanes holding a leaf (default 1)
+    bool counter_clear = false;    // the work before this launch on its stream leaves the counter at 0
     // optional traversal order: the k-th ray taken from the work counter is rays[order[k]] (a
     // permutation of 0..n-1, device), its result goes to out[order[k]]; null = index order.
     const uint32_t* order = nullptr;

@@ -831,7 +831,7 @@ hipError_t launch(const TraceArgs& a, hipStream_t stream, int num_cus) {
     if (want < grid) grid = want;
     if (grid < 1) grid = 1;
     // a batch that the workgroups' shares cover never asks the counter (saves a launch, about 5 us)
-    if (a.n >= kDealtPerWave * (kBlock / 64) * grid)
+    if (!a.counter_clear && a.n >= kDealtPerWave * (kBlock / 64) * grid)
         hipLaunchKernelGGL(k_walk_reset, dim3(1), dim3(64), 0, stream, a.counter);
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kBlock), 0, stream, a);
     return hipGetLastError();

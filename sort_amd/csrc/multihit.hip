@@ -2,9 +2,12 @@
 // reference's record update (Fbvh::GetIntersect with BSSRDFIntersections, fast_bvh.hpp:656-752;
 // intersectTriangleMulti_SIMD, simd_triangle.h:412-452; BSSRDFIntersections, bssrdf.h:32-56).
 //
-// One ray per lane with its own stack (private memory): subsurface probe rays are a small share of
-// a frame's rays and end after a few leaves, so this kernel keeps the closest-hit kernel's slab
-// and triangle arithmetic and push order, without its wave-level refill and leaf batching.
+// One ray per lane: subsurface probe rays are a small share of a frame's rays and end after a few leaves,
+// so this kernel keeps the Fast-BVH walk's slab and triangle arithmetic and push order (trace.hip),
+// without its refill. What bounds it are the loads of nodes and records, with few lanes at work in each.
+// 500,009 probes into 200,003 triangles, 0.465 ms with every stack in scratch memory and a wave doing a
+// node step and a whole leaf in each turn: the top 16 stack entries in LDS take it to 0.436, a node
+// phase until three quarters of the lanes at work hold a leaf to 0.360 (a half: 0.375).
 #include <hip/hip_runtime.h>
 
 #include "trace_launch.h"
@@ -14,9 +17,11 @@ namespace sortgpu {
 namespace {
 
 constexpr int kMultiBlock = 256;
+constexpr int kMultiLds = 16;
 
 template <int W, int STACK>
 __global__ __launch_bounds__(kMultiBlock) void k_multi(MultiArgs a) {
+    __shared__ uint2 s_st[kMultiLds * kMultiBlock];  // the top entries of every lane's stack
     const uint64_t slot_k = (uint64_t)blockIdx.x * kMultiBlock + threadIdx.x;
     if (slot_k >= a.n) return;
     // the k-th probe of the traversal order (a permutation of 0..n-1), results at its own index
@@ -39,22 +44,76 @@ __global__ __launch_bounds__(kMultiBlock) void k_multi(MultiArgs a) {
     uint32_t cnt = 0;
     float maxt = FLT_MAX;  // resolved only when a record is replaced (bssrdf.h:50-55)
 
-    uint2 st[STACK];
+    uint2 deep[STACK - kMultiLds];
     int sp = 0;
     bool overflow = false;
+    auto push = [&](int e, uint32_t ref, float t) {
+        const uint2 v = make_uint2(ref, __float_as_uint(t));
+        if (e < kMultiLds) s_st[e * kMultiBlock + threadIdx.x] = v;
+        else deep[min(e - kMultiLds, STACK - kMultiLds - 1)] = v;
+    };
     if (a.tree.valid) {
         const float rmin = root_slab(r, a.tree.bbox);
-        if (rmin >= 0.0f) st[sp++] = make_uint2(a.tree.root, __float_as_uint(rmin));
+        if (rmin >= 0.0f) push(sp++, a.tree.root, rmin);
     }
-    while (sp > 0) {
-        const uint2 e = st[--sp];
-        const uint32_t ref = e.x;
-        if (maxt < __uint_as_float(e.y)) continue;
-        if (ref & REF_LEAF) {
+    uint32_t li = 0xffffffffu;  // the leaf that the lane holds
+    while (true) {
+        // Node phase: until no lane can walk or three quarters of those at work hold a leaf. The leaf phase
+        // then ends every leaf held, so each round takes some lane on.
+        const uint32_t busy = (uint32_t)__popcll(__ballot(sp > 0 || li != 0xffffffffu));
+        if (busy == 0) break;
+        while (true) {
+            const bool walk = li == 0xffffffffu && sp > 0;
+            if (__ballot(walk) == 0 || 4u * (uint32_t)__popcll(__ballot(li != 0xffffffffu)) >= 3u * busy) break;
+            if (walk) {
+                --sp;
+                // the LDS read is unconditional (clamped index) so that it stays an LDS access
+                uint2 e = s_st[min(sp, kMultiLds - 1) * kMultiBlock + threadIdx.x];
+                if (sp >= kMultiLds) e = deep[min(sp - kMultiLds, STACK - kMultiLds - 1)];
+                const bool live = !(maxt < __uint_as_float(e.y));
+                if (live && (e.x & REF_LEAF)) {
+                    li = e.x & ~REF_LEAF;
+                } else if (live) {
+                    float f[W];
+                    uint32_t ch[W];
+                    const uint32_t m = node_test<W>(r, nodes, e.x, f, ch);
+                    uint32_t elig = m;
+                    if (__popc(m) >= 3) {
+                        // repeated argmax over f > -1 (fast_bvh.hpp:725-740)
+#pragma unroll
+                        for (int j = 0; j < W; j++)
+                            if (!(f[j] > -1.0f)) elig &= ~(1u << j);
+                    }
+                    // farther first, ties lower lane first (the hit children's distances are not NaN)
+                    uint32_t rank[W];
+#pragma unroll
+                    for (int j = 0; j < W; j++) rank[j] = 0;
+#pragma unroll
+                    for (int j = 1; j < W; j++) {
+#pragma unroll
+                        for (int k = 0; k < j; k++) {
+                            const bool kfirst = f[k] >= f[j];
+                            rank[j] += kfirst ? ((elig >> k) & 1u) : 0u;
+                            rank[k] += kfirst ? 0u : ((elig >> j) & 1u);
+                        }
+                    }
+                    const int n = __popc(elig);
+                    if (sp + n > STACK) {  // cannot happen for a tree the host accepted (max_stack <= STACK)
+                        overflow = true;
+                        sp = 0;
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < W; j++)
+                            if (elig & (1u << j)) push(sp + (int)rank[j], ch[j], f[j]);
+                        sp += n;
+                    }
+                }
+            }
+        }
+        if (li != 0xffffffffu) {
             // triangle groups of W (PR_GEND ends one): every hit of a group is judged against maxt
             // as it was before the group; quads are not tested. The leaf's next record loads while
             // the current one is tested.
-            uint32_t li = ref & ~REF_LEAF;
             bool gstart = true;
             float gmaxt = maxt;
             auto tri = [&](const Tri& x, uint32_t id) {
@@ -99,40 +158,8 @@ __global__ __launch_bounds__(kMultiBlock) void k_multi(MultiArgs a) {
                 pr = nxt;
                 ++li;
             }
-            continue;
+            li = 0xffffffffu;
         }
-        float f[W];
-        uint32_t ch[W];
-        const uint32_t m = node_test<W>(r, nodes, ref, f, ch);
-        uint32_t elig = m;
-        if (__popc(m) >= 3) {
-            // repeated argmax over f > -1 (fast_bvh.hpp:725-740)
-#pragma unroll
-            for (int j = 0; j < W; j++)
-                if (!(f[j] > -1.0f)) elig &= ~(1u << j);
-        }
-        // farther first, ties lower lane first (the hit children's distances are not NaN)
-        uint32_t rank[W];
-#pragma unroll
-        for (int j = 0; j < W; j++) rank[j] = 0;
-#pragma unroll
-        for (int j = 1; j < W; j++) {
-#pragma unroll
-            for (int k = 0; k < j; k++) {
-                const bool kfirst = f[k] >= f[j];
-                rank[j] += kfirst ? ((elig >> k) & 1u) : 0u;
-                rank[k] += kfirst ? 0u : ((elig >> j) & 1u);
-            }
-        }
-        const int n = __popc(elig);
-        if (sp + n > STACK) {  // cannot happen for a tree the host accepted (max_stack <= STACK)
-            overflow = true;
-            break;
-        }
-#pragma unroll
-        for (int j = 0; j < W; j++)
-            if (elig & (1u << j)) st[sp + (int)rank[j]] = make_uint2(ch[j], __float_as_uint(f[j]));
-        sp += n;
     }
     if (overflow) atomicOr(a.error, kFlagStackOverflow);
     float4* out = reinterpret_cast<float4*>(a.hits) + 4 * i;

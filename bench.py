@@ -12,7 +12,9 @@ are timed the same way and reported beside it.
 roofline: HBM-bound. Algorithmic bytes per ray = 32 (ray) + 16 (hit) + 224 * inner nodes
 visited + 36 * triangles tested, with the visit counts from the traversal's own counters (equal
 to the oracle's on these rays); achieved = bytes per launch / mean launch time (HIP events on
-the launch stream). roofline.memory_pipeline adds the ceiling the kernel actually meets: lanes
+the launch stream). Those are the bytes of the Fast-BVH walk, which defines the query's results; the
+kernel finds them through a smaller tree (walk.hip), so this fraction and the next may pass 1.
+roofline.memory_pipeline adds the ceiling that the Fast-BVH walk meets: lanes
 read their own records, so compute units return 16-byte chunks at a bounded rate; a probe kernel
 measures that rate for the traversal's two access patterns and gives the launch time it allows.
 
@@ -75,7 +77,7 @@ def log(msg):
     print(msg, file=sys.stderr, flush=True)
 
 
-TRAFFIC_PROFILE = "profiles/k_trace_obvh_1m_soup_incoherent.md"
+TRAFFIC_PROFILE = "profiles/k_walk_1m_soup_incoherent.md"
 
 
 def profiled_traffic(a):

@@ -78,6 +78,12 @@ def _check(acc, ob, rays, label):
     bad = np.nonzero(np.any(hits.view(np.uint32) != ref.view(np.uint32), axis=1))[0]
     assert bad.size == 0, f"{label}: {bad.size} closest differ, ray {rays[bad[0]]}: {hits[bad[0]]} {ref[bad[0]]}"
     assert np.array_equal(occ, ref_occ), label
+    try:  # small batches give four lanes to a ray; with 8 LDS entries every ray has one
+        batch.set_tuning(acc.ctx, lds_entries=8)
+        lanes, lanes_occ = acc.get_intersect(d).cpu().numpy(), acc.is_occluded(d).cpu().numpy()
+    finally:
+        batch.set_tuning(acc.ctx)
+    assert np.array_equal(lanes.view(np.uint32), hits.view(np.uint32)) and np.array_equal(lanes_occ, occ), label
     acc.check_errors()
     return hits
 
@@ -158,6 +164,7 @@ def test_windows_directions_and_pool(gpu_ctx, lds):
     try:
         batch.set_tuning(gpu_ctx, lds_entries=lds)
         hits = _check(acc, ob, r, f"windows lds {lds}")
+        batch.set_tuning(gpu_ctx, lds_entries=lds)
         accs = [acc] + [Obvh(gpu_ctx).build(*scenes.soup(n, seed=n)) for n in (700, 40)]
         pool = batch.Pool(gpu_ctx, accs)
         sid = (k % 3).astype(np.int32)

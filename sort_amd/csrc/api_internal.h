@@ -77,8 +77,10 @@ void free_accel_device(sortgpu_accel* acc);
 //     16M 2.13 / 3.07; 2M rays: 4M triangles 1.16 / 1.11 (shadow 1.16 / 1.31), 16M 1.20 / 1.36;
 //     1M rays: 0.86 / 0.77 through 8M triangles; a pool of 64 scenes and 8M triangles, rays shuffled
 //     over the scenes, 4.63 / 6.83;
-//   transparent shadows: 300K rays 1.65 / 1.60, 600K 2.15 / 2.17, 4M 11.7 / 12.4 ms;
-//   multi-hit probes: 500K 0.54 / 0.48, 1M 0.82 / 0.91, 4M 3.49 / 4.66;
+//   transparent shadows: 524K rays through 200K triangles 1.99 / 1.90 ms, through 1M 2.63 / 2.75; 1M
+//     rays 2.96 / 2.97 and 3.80 / 4.10; 2M 4.94 / 5.11 and 6.38 / 6.82;
+//   multi-hit probes: 524K into 200K triangles 0.45 / 0.38, into 1M 0.56 / 0.51; 1M 0.62 / 0.69 and
+//     0.84 / 0.95; 4M 1.80 / 2.58 and 2.62 / 3.50;
 //   Fast-BVH walk (trees without a walk tree): batches of 256K rays and more.
 constexpr uint32_t kReorderMinRays = 1u << 18;
 constexpr uint32_t kReorderMinWalkRays = 1u << 21;

@@ -449,7 +449,7 @@ __device__ __forceinline__ void leaf_outcome(const TraceArgs& a, Walker& w, uint
         RayK q;
         load_ray(a.rays, w.ray_id, q);
         float qt;
-        if (quad_test(q, tv.quads[__float_as_uint(w.recs[ri].a.p0x)], FLT_MAX, qt))
+        if ((w.recs[ri].id_a & PR_FLAG) && quad_test(q, tv.quads[__float_as_uint(w.recs[ri].a.p0x)], FLT_MAX, qt))
             found<ANY, MULTI>(a, w, ri, qt, 0.f, 0.f, 0u);
     } else if (t < FLT_INF) {
         found<ANY, MULTI>(a, w, ri, t, u, v, which);
@@ -461,7 +461,8 @@ __device__ __forceinline__ void leaf_outcome(const TraceArgs& a, Walker& w, uint
     }
 }
 
-// Tests the triangle at `tp`; true: the record is a quad's (no triangle of a walk tree holds a NaN).
+// Tests the triangle at `tp`; true: the record is a quad's (it has a NaN where no triangle of a walk tree
+// has one: the builder leaves such triangles out).
 __device__ __forceinline__ bool record_tri(RayK& r, const char* tp, float& t, float& u, float& v) {
     r.kz = r.ky == 2 ? 0 : r.ky + 1;
     r.kx = r.kz == 2 ? 0 : r.kz + 1;

@@ -253,6 +253,10 @@ struct Builder {
         const float* a = in.pos + 3 * (size_t)v[0];
         const float* b = in.pos + 3 * (size_t)v[1];
         const float* c = in.pos + 3 * (size_t)v[2];
+        // A triangle with a NaN coordinate passes no test; its record holds three equal corners, which pass
+        // none either. (Its box bounds the other coordinates, so it reaches this tree; an infinite one does not.)
+        for (int k = 0; k < 3; k++)
+            if (!std::isfinite(a[k]) || !std::isfinite(b[k]) || !std::isfinite(c[k])) return;
         t.p0x = a[0]; t.p0y = a[1]; t.p0z = a[2];
         t.p1x = b[0]; t.p1y = b[1]; t.p1z = b[2];
         t.p2x = c[0]; t.p2y = c[1]; t.p2z = c[2];
@@ -461,7 +465,7 @@ void build_walk_tree(const BuildInput& in, const std::vector<BuildPrim>& prims, 
         far = std::max(far, std::max(std::fabs(bbox[k]), std::fabs(bbox[3 + k])));
         ext = std::max(ext, bbox[3 + k] - bbox[k]);
     }
-    for (const BuildPrim& p : prims)  // NaN vertices leave a box that bounds nothing
+    for (const BuildPrim& p : prims)  // an axis on which every coordinate is NaN has a box that bounds nothing
         for (int k = 0; k < 3; k++)
             if (!(p.mn[k] <= p.mx[k]) || !(p.mn[k] >= bbox[k] && p.mx[k] <= bbox[3 + k])) return;
     if (far > 1e12f || far > 4096.0f * ext) return;

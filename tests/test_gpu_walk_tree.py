@@ -177,3 +177,20 @@ def test_windows_directions_and_pool(gpu_ctx, lds):
         one = accs[i].get_intersect(torch.from_numpy(r).cuda()).cpu().numpy()
         assert np.array_equal(got[sid == i].view(np.uint32), one[sid == i].view(np.uint32))
     pool.close()
+
+
+@pytest.mark.parametrize("quads", [False, True])
+@pytest.mark.parametrize("width", [8, 4])
+def test_vertices_with_a_nan_coordinate(gpu_ctx, width, quads):
+    """Such a triangle is never hit; its neighbours in the tree are, as if it were not there."""
+    g = np.random.default_rng(11)
+    t = g.uniform(0.0, 1.0, (3000, 1, 3)) + g.normal(0.0, 0.03, (3000, 3, 3))
+    t = t.astype(np.float32)
+    bad = np.arange(0, len(t), 4)
+    rays = _rays(g, 12000, (t.reshape(-1, 3), None))
+    t[bad, bad // 4 % 3, bad // 12 % 3] = np.nan
+    mesh = scenes.tris_to_mesh(list(t))
+    acc, ob = _build(gpu_ctx, width, mesh, [scenes.translate_quad((0.5, 1.2, 0.5), 0.5)] if quads else None)
+    hits = _check(acc, ob, scenes.make_rays(*rays, 0.0, FLT_MAX), f"nan quads={quads}")
+    prim = hits[:, 1].view(np.uint32)
+    assert np.mean(prim != MISS) > 0.1 and not np.isin(prim, bad).any()

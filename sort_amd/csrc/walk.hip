@@ -361,6 +361,10 @@ __device__ __forceinline__ void settle(const TraceArgs& a, Walker& w, uint2* st)
     }
 }
 
+// The entry distance in a stack entry's key, without the slot in its last two bits (which would put a box
+// that starts at the search bound past it).
+__device__ __forceinline__ float key_distance(uint32_t key) { return __uint_as_float(key & ~3u); }
+
 // A node record with the ray's near and far planes picked out, and where its children lie.
 struct NodeSlabs {
     float gx, gy, gz, nx, ny, nz, fx, fy, fz;
@@ -583,14 +587,14 @@ __device__ __forceinline__ void walk_lanes(const TraceArgs& a, uint32_t n_rays, 
                 if (pop) {
                     --w.sp;
                     const uint2 e = s_st[w.sp * kBlock + tid];
-                    if (__uint_as_float(e.y) <= w.lim) w.cur = e.x;
+                    if (key_distance(e.y) <= w.lim) w.cur = e.x;
                 }
             } else if (pop) {
                 --w.sp;
                 uint2 e;
                 if (w.sp < LDS) e = s_st[w.sp * kBlock + tid];
                 else e = sp_st[min(w.sp - LDS, SPILL - 1)];
-                if (__uint_as_float(e.y) <= w.lim) w.cur = e.x;
+                if (key_distance(e.y) <= w.lim) w.cur = e.x;
             }
             if (walk && (int32_t)w.cur >= 0) {
                 const NodeSlabs n(w.nodes, w.cur, w.s);
@@ -747,7 +751,7 @@ __device__ __forceinline__ void walk_quads(const TraceArgs& a, uint32_t n_rays, 
             if (walk && w.cur == kNone) {
                 --w.sp;
                 const uint2 e = st[w.sp * 16];
-                if (__uint_as_float(e.y) <= w.lim) w.cur = e.x;
+                if (key_distance(e.y) <= w.lim) w.cur = e.x;
             }
             if (walk && (int32_t)w.cur >= 0) {
                 const NodeSlabs n(w.nodes, w.cur, w.s);

@@ -194,3 +194,22 @@ def test_vertices_with_a_nan_coordinate(gpu_ctx, width, quads):
     hits = _check(acc, ob, scenes.make_rays(*rays, 0.0, FLT_MAX), f"nan quads={quads}")
     prim = hits[:, 1].view(np.uint32)
     assert np.mean(prim != MISS) > 0.1 and not np.isin(prim, bad).any()
+
+
+@pytest.mark.parametrize("n", [700, 40000])
+def test_windows_of_one_float(gpu_ctx, n):
+    """Windows that hold a known hit's distance and no other number: the boxes on the way to it start at tmin,
+    and a stack entry, whose last two bits name its slot, may not be taken for one past tmax."""
+    g = np.random.default_rng(n)
+    t = g.uniform(0.0, 1.0, (n, 1, 3)) + g.normal(0.0, 0.5 * n ** (-1 / 3), (n, 3, 3))
+    mesh = scenes.tris_to_mesh(list(t.astype(np.float32)))
+    acc, ob = _build(gpu_ctx, 8, mesh, None)
+    o, d = _rays(g, 20000, mesh)
+    hits = ob.closest(scenes.make_rays(o, d, 0.0, FLT_MAX), threads=16)
+    at = hits[:, 0][hits[:, 1].view(np.uint32) != MISS]
+    o, d = o[hits[:, 1].view(np.uint32) != MISS], d[hits[:, 1].view(np.uint32) != MISS]
+    for ulps in (1, 2, 3):
+        lo = (at.view(np.uint32) - np.uint32(ulps)).view(np.float32)
+        rays = scenes.make_rays(o, d, lo, at)
+        found = _check(acc, ob, rays, f"{ulps} ulps, {n} triangles")
+        assert np.mean(found[:, 1].view(np.uint32) != MISS) > 0.5

@@ -10,8 +10,8 @@ namespace sortgpu {
 void free_accel_device(sortgpu_accel* acc) {
     if (!acc || !acc->ctx || acc->ctx->host_only) return;
     ctx_bind(acc->ctx);
-    void* ptrs[] = {acc->d_nodes,  acc->d_prims, acc->d_quads, acc->d_wnodes, acc->d_wrecs,
-                    acc->d_waux,   acc->d_counters, acc->d_error, acc->d_stats};
+    void* ptrs[] = {acc->d_nodes, acc->d_prims,  acc->d_quads,    acc->d_wnodes, acc->d_wrecs,
+                    acc->d_waux,  acc->d_wgates, acc->d_counters, acc->d_error,  acc->d_stats};
     for (void* p : ptrs)
         if (p) hipFree(p);
     acc->d_nodes = nullptr;
@@ -20,6 +20,7 @@ void free_accel_device(sortgpu_accel* acc) {
     acc->d_wnodes = nullptr;
     acc->d_wrecs = nullptr;
     acc->d_waux = nullptr;
+    acc->d_wgates = nullptr;
     acc->d_counters = nullptr;
     acc->d_error = nullptr;
     acc->d_stats = nullptr;
@@ -46,7 +47,8 @@ int upload_accel(sortgpu_accel* acc) {
     const BuiltTree& h = acc->host;
     const size_t nb = h.node_bytes.size(), pb = h.prims.size() * sizeof(PrimRec),
                  qb = h.quads.size() * sizeof(QuadRec), wb = h.walk.nodes.size() * sizeof(WalkNode),
-                 rb = h.walk.recs.size() * sizeof(PrimRec), xb = h.walk.aux.size() * sizeof(WalkAux);
+                 rb = h.walk.recs.size() * sizeof(PrimRec), xb = h.walk.aux.size() * sizeof(WalkAux),
+                 gb = h.walk.gates.size() * sizeof(uint32_t);
     if ((rc = dev_alloc_copy(ctx, &acc->d_nodes, nb ? h.node_bytes.data() : nullptr, nb, "hipMalloc(nodes)")) ||
         (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_prims), h.prims.data(), pb, "hipMalloc(prims)")) ||
         (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_quads), qb ? h.quads.data() : nullptr, qb,
@@ -56,7 +58,9 @@ int upload_accel(sortgpu_accel* acc) {
                 (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_wrecs), h.walk.recs.data(), rb,
                                      "hipMalloc(walk records)")) ||
                 (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_waux), h.walk.aux.data(), xb,
-                                     "hipMalloc(walk leaf boxes)")))) ||
+                                     "hipMalloc(walk leaf boxes)")) ||
+                (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_wgates), h.walk.gates.data(), gb,
+                                     "hipMalloc(walk gates)")))) ||
         (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_counters), nullptr,
                              kCounterSlots * kCounterStride * sizeof(uint32_t), "hipMalloc(counters)")) ||
         (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_error), nullptr, 16, "hipMalloc(error)")) ||
@@ -64,14 +68,16 @@ int upload_accel(sortgpu_accel* acc) {
         free_accel_device(acc);
         return rc;
     }
-    acc->device_bytes = nb + pb + qb + wb + rb + xb;
+    acc->device_bytes = nb + pb + qb + wb + rb + xb + gb;
     acc->view.nodes = acc->d_nodes;
     acc->view.prims = acc->d_prims;
     acc->view.quads = acc->d_quads;
     acc->view.wnodes = acc->d_wnodes;
     acc->view.wrecs = acc->d_wrecs;
     acc->view.waux = acc->d_waux;
+    acc->view.wgates = acc->d_wgates;
     acc->view.walk_stack = h.walk.stack;
+    acc->view.walk_pad = h.walk.pad;
     return 0;
 }
 

@@ -46,6 +46,7 @@ struct sortgpu_accel {
     sortgpu::WalkNode* d_wnodes = nullptr;
     sortgpu::PrimRec* d_wrecs = nullptr;
     sortgpu::WalkAux* d_waux = nullptr;
+    uint32_t* d_wgates = nullptr;
     uint32_t* d_counters = nullptr;
     uint32_t* d_error = nullptr;
     unsigned long long* d_stats = nullptr;

@@ -91,6 +91,16 @@ struct alignas(16) WalkAux {
 };
 static_assert(sizeof(WalkAux) == 32, "WalkAux must be 32 B");
 
+// Gates (walk.hip says what they are for): two words a record, for A and B (a record of one triangle or of a
+// quad repeats its own). Bytes 0 to 2: the unit normal in 127ths, or zeros to let every ray through. Byte 3
+// of a gated node's first word: how many records its Fast-BVH leaf takes, from the node's rec_base on; of its
+// second word: the leaf's widest reach in 1,024ths. A gated node is the root of such a leaf's part of the walk
+// tree, and the last bit of its base[0] is set.
+constexpr uint32_t kGateRecs = 8;         // records that the kernel reads the words of at a time
+constexpr uint32_t kGatePad = 2 * kGateRecs;
+constexpr uint32_t kGateShut = 0x7f7f7fu; // for what needs no gate; it lets a few rays through, in vain
+constexpr float kWalkWiden = 1.0f / 256;  // a triangle's box is widened by this part of its longest edge
+
 // Everything a traversal kernel needs about one tree.
 struct TreeView {
     const void* nodes;      // NodeRec<W>*
@@ -99,13 +109,14 @@ struct TreeView {
     const WalkNode* wnodes; // walk tree (null: none)
     const PrimRec* wrecs;
     const WalkAux* waux;
+    const uint32_t* wgates;
     uint32_t root;          // child reference of the root (leaf when the tree is one leaf)
     uint32_t valid;         // 0: every query misses
     uint32_t max_stack;     // (W-1)*(depth-1)+1
     uint32_t width;
     float bbox[6];          // enlarged scene box (root slab test)
     uint32_t walk_stack;    // most stack entries a walk-tree traversal holds; 0: no walk tree
-    uint32_t pad;
+    float walk_pad;         // padding of the walk's boxes, as a part of the largest coordinate in play
 };
 
 }  // namespace sortgpu

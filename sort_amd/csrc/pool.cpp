@@ -66,7 +66,7 @@ int sortgpu_pool_create(sortgpu_ctx* ctx, sortgpu_accel* const* accels, uint32_t
     for (uint32_t i = 0; i < n && walk_stack; i++) {
         const WalkTree& w = accels[i]->host.walk;
         total += align256(w.nodes.size() * sizeof(WalkNode)) + align256(w.recs.size() * sizeof(PrimRec)) +
-                 align256(w.aux.size() * sizeof(WalkAux));
+                 align256(w.aux.size() * sizeof(WalkAux)) + align256(w.gates.size() * sizeof(uint32_t));
     }
     if (!width) width = 8;
     if (max_stack > trace_max_stack_supported()) {
@@ -131,8 +131,10 @@ int sortgpu_pool_create(sortgpu_ctx* ctx, sortgpu_accel* const* accels, uint32_t
             v.wnodes = static_cast<const WalkNode*>(put(h.walk.nodes.data(), h.walk.nodes.size() * sizeof(WalkNode)));
             v.wrecs = static_cast<const PrimRec*>(put(h.walk.recs.data(), h.walk.recs.size() * sizeof(PrimRec)));
             v.waux = static_cast<const WalkAux*>(put(h.walk.aux.data(), h.walk.aux.size() * sizeof(WalkAux)));
+            v.wgates = static_cast<const uint32_t*>(put(h.walk.gates.data(), h.walk.gates.size() * sizeof(uint32_t)));
             if (e != hipSuccess) return fail(e, "hipMemcpy(pool walk tree)");
             v.walk_stack = h.walk.stack;
+            v.walk_pad = h.walk.pad;
         }
         v.root = h.root_ref;
         v.valid = h.valid ? 1u : 0u;

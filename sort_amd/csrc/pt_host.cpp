@@ -190,7 +190,9 @@ int prepare_scene(sortgpu_ctx* ctx, const sortgpu_accel* acc, const sortgpu_scen
         im.tree.wnodes = nullptr;
         im.tree.wrecs = nullptr;
         im.tree.waux = nullptr;
+        im.tree.wgates = nullptr;
         im.tree.walk_stack = with_tree ? acc->host.walk.stack : 0;
+        im.tree.walk_pad = acc->host.walk.pad;
         if (with_tree) {
             im.nodes = acc->host.node_bytes;
             im.prims = acc->host.prims;
@@ -320,6 +322,7 @@ void for_each_array(const SceneImage& im, bool lean, SceneDev& d, F f) {
         f(im.walk.nodes.data(), vbytes(im.walk.nodes), reinterpret_cast<const void**>(&d.tree.wnodes));
         f(im.walk.recs.data(), vbytes(im.walk.recs), reinterpret_cast<const void**>(&d.tree.wrecs));
         f(im.walk.aux.data(), vbytes(im.walk.aux), reinterpret_cast<const void**>(&d.tree.waux));
+        f(im.walk.gates.data(), vbytes(im.walk.gates), reinterpret_cast<const void**>(&d.tree.wgates));
     }
     f(im.idx.data(), vbytes(im.idx), reinterpret_cast<const void**>(&d.idx));
     f(im.pos.data(), vbytes(im.pos), reinterpret_cast<const void**>(&d.pos));

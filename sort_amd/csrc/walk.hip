@@ -5,10 +5,7 @@
 // go to the one met first. This kernel finds candidates in a tree of its own (4-wide nodes of 48
 // bytes, at most two triangles to a leaf) and then shows that the walk would have returned the same:
 //
-//   * The candidates are complete. A walk node's boxes are quantised outwards, and every slab is
-//     widened by kPad = 2^-19 of the largest coordinate in play, more than the rounding of the slab
-//     distances (4 units of 2^-24 of it) and of the triangle test (18 units) put together. So a
-//     triangle that the triangle test accepts is always reached, unless its t is past the pruning bound.
+//   * The candidates are complete: below.
 //   * Slab distances grow monotonically from a box to a box inside it, in floating point too (each
 //     is one product and one sum), and a Fast-BVH node's box holds its children's exactly. So the
 //     walk may take hits from a leaf when the leaf's own box passes, and the leaf is pruned only by
@@ -19,23 +16,55 @@
 //     max(t, e) and e does not lie past lim, the walk returns this candidate.
 //
 // A ray for which this cannot be shown (a tie across leaves, a leaf box missed by rounding), or whose
-// numbers leave the bounds above (NaN, infinities, a negative tmin, an origin very far out), is walked
+// numbers leave the bounds below (NaN, infinities, a negative tmin, an origin very far out), is walked
 // again through the Fast-BVH by its lane, in `exact_walk`. Any hit needs less: the first candidate
 // whose leaf box passes.
 //
-// What it saves: on the benchmark's 4,194,304 bounce rays through 2^20 triangles a ray of the
-// Fast-BVH walk tests 14.8 nodes and 81.5 triangles, reading 391 chunks of 16 bytes; here it tests 30.4
-// nodes and 11.6 triangles, reading 123 chunks, with about half the arithmetic. That alone took the call from
-// 4.35 to 2.09 ms (1.56 with what is measured further down); 1.5M shadow segments through 300K triangles
-// from 1.79 to 0.97 (0.68), 2M camera rays on 768K triangles of spheres from 0.80 to 0.70 (0.31).
-// Leaves of one triangle instead of two: 2 to 3 steps more per ray on meshes. 8-wide nodes: 20.7 steps
-// instead of 30.4, each with twice the arithmetic.
+// Why the candidates are complete. Let u = 2^-24, M the largest coordinate of origin and scene, D that of a
+// vertex relative to the origin. Take a triangle with longest edge L and height H over it, in a leaf whose box
+// the exact test passes, at R at most across (times sqrt(3), for the shear), and accepted by the triangle test
+// at t. The test sees its corners projected along the ray, wrong by e = 5.7 u D + u R; it takes the signs of the
+// three products of two corners, and a sign is right unless the ray sees the two within an angle of u (or
+// pi - u). So either the ray passes within rounding of the triangle, or it sees all of it within 2 u, however
+// far beside it: a flat sheet edge-on, a needle, a triangle of the rounding's own size. The Fast-BVH has such
+// hits all over the leaf's box (at up to 16 triangles to a leaf), where no box of the triangle's reaches.
+//   - Beside: all three corners lie within u R + e of one plane through the ray, so the ray's direction lies
+//     within 2.83 (u R + e) / H of the triangle's plane. Within 8 e / H of it, too, rounding may take half of the
+//     projected area. Such triangles are the gates' matter: each Fast-BVH leaf's part of the walk tree starts
+//     at a node of its own (a gated node) with all its triangles' normals in four bytes each, and a ray that
+//     comes there is tested against each triangle whose plane it is that near to, whatever its box says
+//     (kGateReach, kGateLeaf; normals in 127ths add 0.0137).
+//   - Otherwise t is a mean of the corners' distances with weights that are off by 6 u R R over the projected
+//     area, so that the ray's point at t lies within 36 u L L / (H s) + e of the triangle where its direction is
+//     more than s off the plane. What of this is more than L / 256, by which a triangle's box is widened, is again
+//     the gates' matter (kGateShape). The rest, with the rounding of the slab distances (10 u M, the Fast-BVH's own
+//     4 among them) and of t (8 u M), is below the 32 u M that every slab is widened by.
+//   - So a leaf's boxes are met where they matter, and the node at its top wherever the exact test passes the
+//     leaf's box. That test steps along a direction with no component below 1e-5: slabs of smaller ones are
+//     widened by what that strays. And a gate's hit may lie before its leaf's entry, so that no box is left out
+//     for its entry distance but only where it starts past `lim` on the ray's main axis: t is a mean of
+//     distances on that axis.
+// Scenes below 1e-8 have no walk tree: products would be lost to underflow. A quad is tested in its own space:
+// its rounding there, and what its two matrices disagree by, are in the tree's padding (walk_tree.cpp).
+// tests/native/walk_complete_check.cpp looks for counterexamples with this arithmetic on the CPU.
+//
+// What it costs and saves: on the benchmark's 4,194,304 bounce rays through 2^20 triangles a ray of the
+// Fast-BVH walk tests 14.8 nodes and 81.5 triangles, reading 391 chunks of 16 bytes; here it tests 35.7
+// nodes, the boxed triangles of 6.2 records, 46 records' normals at 7.6 gates and two triangles behind them.
+// The call takes 2.19 instead of 4.35 ms; 1.5M shadow segments through 300K triangles 0.91 instead of 1.79, 2M camera
+// rays on 768K triangles of spheres 0.36 instead of 0.80. Without the gates and with boxes left out for their
+// entry distances, and other answers for the rays above, it was 1.57, 0.69 and 0.30. Gates seen to by each ray's
+// own lane in the node step took 3.04, 1.23 and 0.40: one node in five has one. (The figures beside the choices
+// further down are from before the gates.)
+// Leaves of one triangle instead of two: 2 to 3 steps more per ray on meshes. 8-wide nodes: a third of the steps
+// less, each with twice the arithmetic.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
 
 #include "trace_launch.h"
 #include "traverse.h"
+#include "walk_step.h"
 
 #pragma clang fp contract(off)
 
@@ -43,110 +72,8 @@ namespace sortgpu {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr uint32_t kNone = 0xffffffffu;
 constexpr uint32_t kDealtPerWave = 128;  // rays per wave from which part of a batch goes out through the counter
 constexpr uint32_t kQuadsPerWave = 28;   // rays per wave up to which four lanes take a ray together
-constexpr float kPad = 1.9073486328125e-6f;  // 2^-19
-
-// What the walk keeps of a ray besides the triangle test's constants: reciprocal directions (true
-// ones, at most 1e18) and plane offsets widened outwards (near: a, far: b).
-struct Slabs {
-    float rx, ry, rz, ax, ay, az, bx, by, bz;
-};
-
-__device__ __forceinline__ float recip(float d) {
-    const float a = fmaxf(fabsf(d), 1e-18f);
-    return copysignf(1.0f / a, d);
-}
-
-// ray_setup's shear constants and traverse.h's root test, from the reciprocals above: 1 / d is the
-// same number wherever |d| >= 1e-18. (The Fast-BVH's own slab constants are not set.)
-__device__ __forceinline__ void shear_setup(RayK& r, const Slabs& s) {
-    const float ax = fabsf(r.dx), ay = fabsf(r.dy), az = fabsf(r.dz);
-    int ky;
-    if (ax > ay && ax > az) ky = 0;
-    else ky = ay > az ? 1 : 2;
-    const int kz = ky == 2 ? 0 : ky + 1;
-    const int kx = kz == 2 ? 0 : kz + 1;
-    r.kx = kx; r.ky = ky; r.kz = kz;
-    const float px = sel3(r.dx, r.dy, r.dz, kx);
-    const float py = sel3(r.dx, r.dy, r.dz, ky);
-    const float pz = sel3(r.dx, r.dy, r.dz, kz);
-    r.sx = -px / py;
-    r.sz = -pz / py;
-    r.sy = sel3(s.rx, s.ry, s.rz, ky);
-    r.okx = sel3(r.ox, r.oy, r.oz, kx);
-    r.oky = sel3(r.ox, r.oy, r.oz, ky);
-    r.okz = sel3(r.ox, r.oy, r.oz, kz);
-}
-__device__ __forceinline__ bool root_test(const RayK& r, const Slabs& s, const float* bb) {
-    float tmax = r.tmax, tmin = r.tmin;
-    const float o[3] = {r.ox, r.oy, r.oz};
-    const float d[3] = {r.dx, r.dy, r.dz};
-    const float q[3] = {s.rx, s.ry, s.rz};
-    bool ok = true;
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        if (d[a] < 0.00001f && d[a] > -0.00001f) {
-            ok &= !(o[a] > bb[3 + a] || o[a] < bb[a]);
-        } else {
-            const float t1 = (bb[3 + a] - o[a]) * q[a], t2 = (bb[a] - o[a]) * q[a];
-            const bool swap = t1 > t2;
-            tmin = smax(swap ? t2 : t1, tmin);
-            tmax = smin(swap ? t1 : t2, tmax);
-            ok &= !(tmin > tmax);
-        }
-    }
-    return ok && tmin >= 0.0f;
-}
-
-// Whether the error bounds above hold for this ray; fills `s` and the search slack.
-__device__ __forceinline__ bool slabs_setup(const RayK& r, const float* bb, Slabs& s, float& slack) {
-    const float mo = fmaxf(fmaxf(fabsf(r.ox), fabsf(r.oy)), fabsf(r.oz));
-    const float md = fmaxf(fmaxf(fabsf(r.dx), fabsf(r.dy)), fabsf(r.dz));
-    float mb = 0.0f, ext = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        mb = fmaxf(mb, fmaxf(fabsf(bb[k]), fabsf(bb[3 + k])));
-        ext = fmaxf(ext, bb[3 + k] - bb[k]);
-    }
-    const float pad = kPad * (mo + mb);
-    s.rx = recip(r.dx);
-    s.ry = recip(r.dy);
-    s.rz = recip(r.dz);
-    const float ox = -r.ox * s.rx, oy = -r.oy * s.ry, oz = -r.oz * s.rz;
-    const float px = pad * fabsf(s.rx), py = pad * fabsf(s.ry), pz = pad * fabsf(s.rz);
-    s.ax = ox - px;
-    s.ay = oy - py;
-    s.az = oz - pz;
-    s.bx = ox + px;
-    s.by = oy + py;
-    s.bz = oz + pz;
-    slack = 2.0f * pad * fminf(fminf(fabsf(s.rx), fabsf(s.ry)), fabsf(s.rz));
-    // comparisons with a NaN are false; fmaxf drops one, so every component is tested
-    return __builtin_isfinite(r.ox) & __builtin_isfinite(r.oy) & __builtin_isfinite(r.oz) &
-           __builtin_isfinite(r.dx) & __builtin_isfinite(r.dy) & __builtin_isfinite(r.dz) & (r.tmin >= 0.0f) &
-           !__builtin_isnan(r.tmax) & (mo <= 1e12f) & (mo <= 4096.0f * ext) & (md >= 1e-12f) & (md <= 1e12f);
-}
-
-// The Fast-BVH's slab test of one box in the x86-select form (traverse.h node_test).
-__device__ __forceinline__ bool box_test(const RayK& r, float lx, float hx, float ly, float hy, float lz, float hz,
-                                         float& entry) {
-    float fmn = r.tmin, fmx = r.tmax;
-    float t1 = r.odx + r.rcx * hx, t2 = r.odx + r.rcx * lx;
-    fmn = xmax(fmn, xmin(t1, t2));
-    fmx = xmin(fmx, xmax(t1, t2));
-    t1 = r.ody + r.rcy * hy;
-    t2 = r.ody + r.rcy * ly;
-    fmn = xmax(fmn, xmin(t1, t2));
-    fmx = xmin(fmx, xmax(t1, t2));
-    t1 = r.odz + r.rcz * hz;
-    t2 = r.odz + r.rcz * lz;
-    fmn = xmax(fmn, xmin(t1, t2));
-    fmx = xmin(fmx, xmax(t1, t2));
-    entry = fmn;
-    return fmn <= fmx;
-}
 
 __device__ __forceinline__ void load_ray(const void* rays, uint32_t i, RayK& r) {
     const float4* rp = reinterpret_cast<const float4*>(rays) + 2 * (size_t)i;
@@ -173,6 +100,32 @@ template <int PERM>
 __device__ __forceinline__ uint32_t quad_rot(uint32_t x) {
     return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, PERM, 0xf, 0xf, true);
 }
+template <int PERM>
+__device__ __forceinline__ float quad_rot_f(float x) { return __uint_as_float(quad_rot<PERM>(__float_as_uint(x))); }
+
+// How many lanes below this one are in `m`.
+__device__ __forceinline__ uint32_t rank_in(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+// Another lane's value.
+__device__ __forceinline__ uint32_t of_lane(uint32_t lane, uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(lane << 2), (int)x);
+}
+__device__ __forceinline__ float of_lane(uint32_t lane, float x) { return __uint_as_float(of_lane(lane, __float_as_uint(x))); }
+template <class T>
+__device__ __forceinline__ const T* of_lane(uint32_t lane, const T* x) {
+    const uint64_t at = reinterpret_cast<uint64_t>(x);
+    return reinterpret_cast<const T*>((uint64_t)of_lane(lane, (uint32_t)(at >> 32)) << 32 | of_lane(lane, (uint32_t)at));
+}
+
+// The gate words of two records, and which of their triangles they let a ray through to.
+struct __attribute__((aligned(8))) GateWords {
+    uint32_t a, b, c, d;
+    __device__ __forceinline__ uint32_t open(uint32_t dir, uint32_t bound) const {
+        return (gate_open(a, dir, bound) ? 1u : 0u) | (gate_open(b, dir, bound) ? 2u : 0u) |
+               (gate_open(c, dir, bound) ? 4u : 0u) | (gate_open(d, dir, bound) ? 8u : 0u);
+    }
+};
 
 struct Best {
     float t, u, v;
@@ -267,7 +220,6 @@ struct Walker {
     float bt, bu, bv;
     float lim;        // search bound: the window's end, then bt and the slack above it
     float second;     // second nearest distance met
-    float slack;
     int sp;
     bool open;        // exact_walk has to answer
 
@@ -278,7 +230,7 @@ struct Walker {
 
 // Takes up ray `my`, or answers it where the scene's box already does.
 template <bool ANY, bool MULTI>
-__device__ __forceinline__ void start(const TraceArgs& a, uint32_t my, Walker& w) {
+__device__ __forceinline__ void start(const TraceArgs& a, uint32_t my, Walker& w, float& slack, uint32_t& gate) {
     load_ray(a.rays, my, w.r);
     w.bt = w.second = FLT_MAX;
     w.lim = w.r.tmax;
@@ -295,7 +247,7 @@ __device__ __forceinline__ void start(const TraceArgs& a, uint32_t my, Walker& w
         w.nodes = tv->wnodes;
         w.recs = tv->wrecs;
     }
-    const bool fits = slabs_setup(w.r, tv->bbox, w.s, w.slack);
+    const bool fits = slabs_setup(w.r, tv->bbox, tv->walk_pad, w.s, slack, gate);
     shear_setup(w.r, w.s);
     // a ray outside the bounds goes to the exact walk, with its root test
     if (known && tv->valid && (!fits || root_test(w.r, w.s, tv->bbox))) {
@@ -361,66 +313,22 @@ __device__ __forceinline__ void settle(const TraceArgs& a, Walker& w, uint2* st)
     }
 }
 
-// The entry distance in a stack entry's key, without the slot in its last two bits (which would put a box
-// that starts at the search bound past it).
-__device__ __forceinline__ float key_distance(uint32_t key) { return __uint_as_float(key & ~3u); }
-
-// A node record with the ray's near and far planes picked out, and where its children lie.
-struct NodeSlabs {
-    float gx, gy, gz, nx, ny, nz, fx, fy, fz;
-    uint32_t wnx, wfx, wny, wfy, wnz, wfz;
-    uint32_t ni, child_at, leaf_at;
-
-    __device__ __forceinline__ NodeSlabs(const WalkNode* nodes, uint32_t i, const Slabs& s) {
-        const uint4* np = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(nodes) + (((i << 1) + i) << 4));
-        const uint4 q0 = np[0], q1 = np[1], q2 = np[2];
-        const uint32_t meta = q0.w;
-        ni = (meta >> 24) & 15u;
-        gx = __uint_as_float((meta & 0xffu) << 23) * s.rx;
-        gy = __uint_as_float(((meta >> 8) & 0xffu) << 23) * s.ry;
-        gz = __uint_as_float(((meta >> 16) & 0xffu) << 23) * s.rz;
-        const float bx = __uint_as_float(q0.x) * s.rx, by = __uint_as_float(q0.y) * s.ry, bz = __uint_as_float(q0.z) * s.rz;
-        nx = bx + s.ax;
-        ny = by + s.ay;
-        nz = bz + s.az;
-        fx = bx + s.bx;
-        fy = by + s.by;
-        fz = bz + s.bz;
-        const bool px = s.rx >= 0.0f, py = s.ry >= 0.0f, pz = s.rz >= 0.0f;
-        wnx = px ? q1.z : q1.w;
-        wfx = px ? q1.w : q1.z;
-        wny = py ? q2.x : q2.y;
-        wfy = py ? q2.y : q2.x;
-        wnz = pz ? q2.z : q2.w;
-        wfz = pz ? q2.w : q2.z;
-        child_at = q1.x;
-        leaf_at = (q1.y | REF_LEAF) - ni;
-    }
-    // Sort key of slot j: kNone where the ray misses its box, else the entry distance (not negative,
-    // so that its bits order as it does) with the slot in the last two bits. `shift`: 8 j.
-    __device__ __forceinline__ uint32_t key(uint32_t j, uint32_t shift, float tmin, float lim) const {
-        auto q = [&](uint32_t x) { return (float)((x >> shift) & 0xffu); };
-        const float t0 = fmaxf(fmaxf(__builtin_fmaf(q(wnx), gx, nx), __builtin_fmaf(q(wny), gy, ny)),
-                               fmaxf(__builtin_fmaf(q(wnz), gz, nz), tmin));
-        const float t1 = fminf(fminf(__builtin_fmaf(q(wfx), gx, fx), __builtin_fmaf(q(wfy), gy, fy)),
-                               fminf(__builtin_fmaf(q(wfz), gz, fz), lim));
-        return t0 <= t1 ? ((__float_as_uint(t0) & ~3u) | j) : kNone;
-    }
-    __device__ __forceinline__ uint32_t ref(uint32_t key) const {
-        const uint32_t j = key & 3u;
-        return (j < ni ? child_at : leaf_at) + j;
-    }
-};
-
 // A triangle's or quad's hit in record `ri` (which: A or B).
 template <bool ANY, bool MULTI>
-__device__ __forceinline__ void found(const TraceArgs& a, Walker& w, uint32_t ri, float t, float u, float v, uint32_t which) {
+__device__ __forceinline__ void found(const TraceArgs& a, Walker& w, float slack, uint32_t ri, float t, float u, float v, uint32_t which) {
     // A tie of two triangles of one Fast-BVH leaf (a mesh with doubled faces has one at every hit): the
     // one that comes first there wins. False: not such a tie.
     auto same_leaf_order = [&]() {
         const TreeView& tv = MULTI ? a.trees[a.ray_scene[w.ray_id]] : a.tree;
         if ((w.recs[ri].id_a & PR_FLAG) || (w.recs[w.hit >> 1].id_a & PR_FLAG)) return false;
-        if (ri == w.hit >> 1) return true;  // the same record again
+        if (ri == w.hit >> 1) {  // the same record again: A before B
+            if (which < (w.hit & 1u)) {
+                w.hit = 2 * ri + which;
+                w.bu = u;
+                w.bv = v;
+            }
+            return true;
+        }
         const WalkAux &x = tv.waux[ri], &y = tv.waux[w.hit >> 1];
         const uint32_t px = (x.places >> (16u * which)) & 0xffffu, py = (y.places >> (16u * (w.hit & 1u))) & 0xffffu;
         if (x.leaf != y.leaf || px == 0xffffu || py == 0xffffu) return false;
@@ -437,8 +345,8 @@ __device__ __forceinline__ void found(const TraceArgs& a, Walker& w, uint32_t ri
         w.bu = u;
         w.bv = v;
         w.hit = 2 * ri + which;
-        w.lim = t + (w.slack + 4e-7f * t);
-    } else if (!ANY && !(t == w.bt && same_leaf_order())) {
+        w.lim = t + (slack + 4e-7f * t);
+    } else if (!ANY && !(t == w.bt && w.hit != kNone && same_leaf_order())) {
         w.second = fminf(w.second, t);
     }
 }
@@ -446,7 +354,7 @@ __device__ __forceinline__ void found(const TraceArgs& a, Walker& w, uint32_t ri
 // The outcome of record `ri`: t, u, v of the nearer of A and B (`which`; A where they are equal), or
 // infinity, and the other one's distance; negative: the record is a quad.
 template <bool ANY, bool MULTI>
-__device__ __forceinline__ void leaf_outcome(const TraceArgs& a, Walker& w, uint32_t ri, float t, float u, float v,
+__device__ __forceinline__ void leaf_outcome(const TraceArgs& a, Walker& w, float slack, uint32_t ri, float t, float u, float v,
                                              float other, uint32_t which) {
     if (other < 0.0f) {
         const TreeView& tv = MULTI ? a.trees[a.ray_scene[w.ray_id]] : a.tree;
@@ -454,9 +362,9 @@ __device__ __forceinline__ void leaf_outcome(const TraceArgs& a, Walker& w, uint
         load_ray(a.rays, w.ray_id, q);
         float qt;
         if ((w.recs[ri].id_a & PR_FLAG) && quad_test(q, tv.quads[__float_as_uint(w.recs[ri].a.p0x)], FLT_MAX, qt))
-            found<ANY, MULTI>(a, w, ri, qt, 0.f, 0.f, 0u);
+            found<ANY, MULTI>(a, w, slack, ri, qt, 0.f, 0.f, 0u);
     } else if (t < FLT_INF) {
-        found<ANY, MULTI>(a, w, ri, t, u, v, which);
+        found<ANY, MULTI>(a, w, slack, ri, t, u, v, which);
         w.second = fminf(w.second, other);
     }
     if (ANY && w.hit != kNone) {
@@ -482,10 +390,125 @@ __device__ __forceinline__ bool record_tri(RayK& r, const char* tp, float& t, fl
     return __builtin_isnan(p1.x);
 }
 
+// The gates that a wave's rays have come to, and the triangles that these let them through to. Both wait until
+// there is one for every lane, or until a ray is to be answered: a lane takes a gate or a triangle of any ray
+// of the wave, with the ray fetched from its owner.
+struct GateShared {
+    uint32_t gate[127];  // first record << 6 | owner
+    uint2 tri[127];      // record * 2 + (0: A, 1: B), owner
+    uint32_t ray[64];    // each lane's gate_ray()
+    float slack[64];     // and its search slack (both are wanted seldom, and registers are short)
+};
+struct Gates {
+    GateShared& sh;
+    uint32_t n_gate = 0, n_tri = 0;
+
+    __device__ __forceinline__ explicit Gates(GateShared& s) : sh(s) {}
+    __device__ __forceinline__ bool full() const { return n_gate >= 64u; }
+    __device__ __forceinline__ bool waiting() const { return (n_gate | n_tri) != 0; }
+
+    // Notes the gate from record `first` on for this lane's ray, where `at`. (Called by the whole wave.)
+    __device__ __forceinline__ void put(bool at, uint32_t first, uint32_t lane) {
+        const uint64_t m = __ballot(at);
+        if (m == 0) return;
+        if (at) sh.gate[n_gate + rank_in(m)] = first << 6 | lane;
+        n_gate += (uint32_t)__popcll(m);
+    }
+
+    // Takes the last of the gates, one to a lane, and tests the triangles behind them by 64; `all`: the last
+    // few too. GROUP: lanes that hold one ray.
+    template <bool ANY, bool MULTI, uint32_t GROUP>
+    __device__ __forceinline__ void pass(const TraceArgs& a, Walker& w, bool all) {
+        const uint32_t lane = __lane_id();
+        const uint32_t n = min(n_gate, 64u);
+        n_gate -= n;
+        __builtin_amdgcn_wave_barrier();
+        uint32_t count = 0, bound = 0, ray = 0, owner = 0, first = 0;
+        const GateWords* gp = nullptr;
+        if (lane < n) {
+            const uint32_t e = sh.gate[n_gate + lane];
+            owner = e & 63u;
+            first = e >> 6;
+            ray = sh.ray[owner];
+            count = 1;
+        }
+        const uint32_t* words = a.tree.wgates;
+        if (MULTI) {
+            const uint32_t id = of_lane(owner, w.ray_id);
+            if (lane < n) words = a.trees[a.ray_scene[id]].wgates;
+        }
+        gp = reinterpret_cast<const GateWords*>(words + 2 * (size_t)first);
+        uint32_t open = 0, at = 0;
+        while (true) {
+            uint64_t m = __ballot(open != 0);
+            if (m == 0 && __ballot(at < count) != 0) {  // the next eight records' words
+                if (at < count) {
+                    const GateWords g[4] = {gp[0], gp[1], gp[2], gp[3]};
+                    if (at == 0) {
+                        count = g[0].a >> 24;
+                        bound = gate_bound(ray, g[0].b >> 24);
+                    }
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; i++) open |= g[i].open(ray & 0xffffffu, bound) << (4 * i);
+                    open &= (1u << (2u * min(count - at, kGateRecs))) - 1u;
+                    gp += kGateRecs / 2;
+                }
+                at += kGateRecs;
+                m = __ballot(open != 0);
+            }
+            const bool done = m == 0 && __ballot(at < count) == 0;
+            if (m != 0) {
+                if (open != 0)
+                    sh.tri[n_tri + rank_in(m)] =
+                        make_uint2(2 * (first + at - kGateRecs) + (uint32_t)__ffs((int)open) - 1u, owner);
+                open &= open - 1u;
+                n_tri += (uint32_t)__popcll(m);
+            }
+            if (n_tri >= 64u || (done && all && n_tri != 0)) test<ANY, MULTI, GROUP>(a, w);
+            if (done) break;
+        }
+    }
+
+    // Tests the last of the triangles, one to a lane.
+    template <bool ANY, bool MULTI, uint32_t GROUP>
+    __device__ __forceinline__ void test(const TraceArgs& a, Walker& w) {
+        const uint32_t lane = __lane_id();
+        const uint32_t n = min(n_tri, 64u);
+        n_tri -= n;
+        __builtin_amdgcn_wave_barrier();
+        const uint2 e = sh.tri[n_tri + min(lane, n - 1u)];
+        const uint32_t owner = e.y;
+        RayK r;
+        r.okx = of_lane(owner, w.r.okx); r.oky = of_lane(owner, w.r.oky); r.okz = of_lane(owner, w.r.okz);
+        r.sx = of_lane(owner, w.r.sx); r.sy = of_lane(owner, w.r.sy); r.sz = of_lane(owner, w.r.sz);
+        r.tmin = of_lane(owner, w.r.tmin);
+        r.tmax = fminf(of_lane(owner, w.r.tmax), of_lane(owner, w.lim));
+        r.ky = (int)of_lane(owner, (uint32_t)w.r.ky);
+        const PrimRec* recs = MULTI ? of_lane(owner, w.recs) : w.recs;
+        float t = FLT_INF, u = 0.f, v = 0.f;
+        if (lane < n) record_tri(r, reinterpret_cast<const char*>(recs + (e.x >> 1)) + (e.x & 1u) * sizeof(Tri), t, u, v);
+        // almost never: a hit of an edge-on triangle, to its ray
+        for (uint64_t m = __ballot(t < FLT_INF); m != 0; m &= m - 1) {
+            const uint32_t l = (uint32_t)__ffsll((unsigned long long)m) - 1u;
+            const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)owner, (int)l);
+            const uint32_t x = (uint32_t)__builtin_amdgcn_readlane((int)e.x, (int)l);
+            auto bits = [&](float f) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), (int)l)); };
+            const float ht = bits(t), hu = bits(u), hv = bits(v);
+            if (lane / GROUP == to / GROUP) {
+                found<ANY, MULTI>(a, w, sh.slack[lane], x >> 1, ht, hu, hv, x & 1u);
+                if (ANY) {
+                    w.sp = 0;
+                    w.cur = w.leaf = kNone;
+                }
+            }
+        }
+    }
+};
+
 // One ray to a lane: batches that fill the chip.
 template <bool ANY, bool MULTI, int LDS, int SPILL>
-__device__ __forceinline__ void walk_lanes(const TraceArgs& a, uint32_t n_rays, uint2* s_st, uint32_t* s_next,
-                                           uint32_t* s_out) {
+__device__ __forceinline__ void walk_lanes(const TraceArgs& a, uint32_t n_rays, uint2* s_st, GateShared& s_gate,
+                                           uint32_t* s_next, uint32_t* s_out) {
     constexpr int CAP = LDS + SPILL;
     uint2 sp_st[SPILL];  // deeper entries; also the stack of exact_walk, whose lane has none of its own left
     const uint32_t tid = threadIdx.x;
@@ -518,16 +541,19 @@ __device__ __forceinline__ void walk_lanes(const TraceArgs& a, uint32_t n_rays, 
     w.recs = a.tree.wrecs;
     w.cur = w.leaf = w.ray_id = w.hit = kNone;
     w.bt = w.lim = w.second = FLT_MAX;
-    w.bu = w.bv = w.slack = 0.f;
+    w.bu = w.bv = 0.f;
     w.sp = 0;
     w.open = false;
+    Gates gates(s_gate);
 
     while (true) {
         const bool idle = w.idle();
         const uint64_t want = __ballot(idle && (more || w.ray_id != kNone));
         const uint64_t busy = __ballot(!idle);
         if (want == 0 && busy == 0) break;
-        if (want != 0 && (busy == 0 || (uint32_t)__popcll(want) >= refill)) {
+        const bool answer = want != 0 && (busy == 0 || (uint32_t)__popcll(want) >= refill);
+        if (answer) {
+            while (gates.waiting()) gates.pass<ANY, MULTI, 1>(a, w, gates.n_gate <= 64u);
             if (idle && w.ray_id != kNone) {
                 settle<ANY, MULTI>(a, w, sp_st);
                 w.ray_id = kNone;
@@ -567,7 +593,7 @@ __device__ __forceinline__ void walk_lanes(const TraceArgs& a, uint32_t n_rays, 
                     own = min(own + cnt, own_end);
                 }
                 if (out) more = false;
-                if (idle && more && given) start<ANY, MULTI>(a, a.order ? a.order[k] : k, w);
+                if (idle && more && given) start<ANY, MULTI>(a, a.order ? a.order[k] : k, w, s_gate.slack[lane], s_gate.ray[lane]);
             }
             continue;
         }
@@ -587,20 +613,25 @@ __device__ __forceinline__ void walk_lanes(const TraceArgs& a, uint32_t n_rays, 
                 if (pop) {
                     --w.sp;
                     const uint2 e = s_st[w.sp * kBlock + tid];
-                    if (key_distance(e.y) <= w.lim) w.cur = e.x;
+                    if (__uint_as_float(e.y) <= w.lim) w.cur = e.x;
                 }
             } else if (pop) {
                 --w.sp;
                 uint2 e;
                 if (w.sp < LDS) e = s_st[w.sp * kBlock + tid];
                 else e = sp_st[min(w.sp - LDS, SPILL - 1)];
-                if (key_distance(e.y) <= w.lim) w.cur = e.x;
+                if (__uint_as_float(e.y) <= w.lim) w.cur = e.x;
             }
+            bool gated = false;
+            uint32_t first = 0;
             if (walk && (int32_t)w.cur >= 0) {
                 const NodeSlabs n(w.nodes, w.cur, w.s);
                 uint32_t key[4];
+                float near[4];
 #pragma unroll
-                for (uint32_t j = 0; j < 4; j++) key[j] = n.key(j, 8 * j, w.r.tmin, w.lim);
+                for (uint32_t j = 0; j < 4; j++) key[j] = n.key(j, 8 * j, w.r, w.lim, near[j]);
+                // one bound for the four: a choice by slot would cost more than the visits it saves
+                const uint32_t ahead = __float_as_uint(fminf(fminf(near[0], near[1]), fminf(near[2], near[3])));
                 auto order = [&](uint32_t& x, uint32_t& y) {
                     const uint32_t lo = min(x, y), up = max(x, y);
                     x = lo;
@@ -616,14 +647,14 @@ __device__ __forceinline__ void walk_lanes(const TraceArgs& a, uint32_t n_rays, 
                 if (__ballot(w.sp + 3 > LDS) == 0) {
 #pragma unroll
                     for (int i = 3; i >= 1; i--) {
-                        s_st[w.sp * kBlock + tid] = make_uint2(n.ref(key[i]), key[i]);
+                        s_st[w.sp * kBlock + tid] = make_uint2(n.ref(key[i]), ahead);
                         w.sp += key[i] != kNone ? 1 : 0;
                     }
                 } else {
 #pragma unroll
                     for (int i = 3; i >= 1; i--) {
                         if (key[i] == kNone) continue;
-                        const uint2 e = make_uint2(n.ref(key[i]), key[i]);
+                        const uint2 e = make_uint2(n.ref(key[i]), ahead);
                         if (w.sp < LDS) s_st[w.sp * kBlock + tid] = e;
                         else if (w.sp < CAP) sp_st[w.sp - LDS] = e;
                         // not reached: the host sizes the stack for the tree
@@ -631,8 +662,12 @@ __device__ __forceinline__ void walk_lanes(const TraceArgs& a, uint32_t n_rays, 
                         else overflow = true;
                     }
                 }
+                gated = n.gated;
+                first = n.first_record();
                 w.cur = key[0] != kNone ? n.ref(key[0]) : kNone;
             }
+            gates.put(gated, first, lane);
+            if (gates.full()) gates.pass<ANY, MULTI, 1>(a, w, false);
             if (w.at_leaf() && w.leaf == kNone) {
                 w.leaf = w.cur;
                 w.cur = kNone;
@@ -687,7 +722,7 @@ __device__ __forceinline__ void walk_lanes(const TraceArgs& a, uint32_t n_rays, 
                 w.leaf = w.cur;
                 w.cur = kNone;
             }
-            leaf_outcome<ANY, MULTI>(a, w, ri, rt, ru, rv, ro, rb ? 1u : 0u);
+            leaf_outcome<ANY, MULTI>(a, w, s_gate.slack[lane], ri, rt, ru, rv, ro, rb ? 1u : 0u);
         }
     }
     if (overflow) atomicOr(a.error, kFlagStackOverflow);
@@ -702,7 +737,8 @@ __device__ __forceinline__ void walk_lanes(const TraceArgs& a, uint32_t n_rays, 
 // 78 -> 94, at 49 (200K) 193 -> 239: four rays' worth of lanes for one stops paying once the chip is full.
 constexpr int kQuadStack = 64;
 template <bool ANY, bool MULTI, int SPILL>
-__device__ __forceinline__ void walk_quads(const TraceArgs& a, uint32_t n_rays, uint2* s_st, uint32_t* s_next) {
+__device__ __forceinline__ void walk_quads(const TraceArgs& a, uint32_t n_rays, uint2* s_st, GateShared& s_gate,
+                                           uint32_t* s_next) {
     uint2 exact_st[SPILL];
     const uint32_t lane = __lane_id();
     const uint32_t sub = lane & 3u;
@@ -718,15 +754,18 @@ __device__ __forceinline__ void walk_quads(const TraceArgs& a, uint32_t n_rays, 
     w.recs = a.tree.wrecs;
     w.cur = w.leaf = w.ray_id = w.hit = kNone;
     w.bt = w.lim = w.second = FLT_MAX;
-    w.bu = w.bv = w.slack = 0.f;
+    w.bu = w.bv = 0.f;
     w.sp = 0;
     w.open = false;
+    Gates gates(s_gate);
     while (true) {
         const bool idle = w.idle();
         const uint64_t want = __ballot(idle && (more || w.ray_id != kNone));
         const uint64_t busy = __ballot(!idle);
         if (want == 0 && busy == 0) break;
-        if (want != 0 && (busy == 0 || (uint32_t)__popcll(want) >= 16u)) {
+        const bool answer = want != 0 && (busy == 0 || (uint32_t)__popcll(want) >= 16u);
+        if (answer) {
+            while (gates.waiting()) gates.pass<ANY, MULTI, 4>(a, w, gates.n_gate <= 64u);
             if (idle && w.ray_id != kNone) {
                 if (sub == 0) settle<ANY, MULTI>(a, w, exact_st);
                 w.ray_id = kNone;
@@ -738,7 +777,7 @@ __device__ __forceinline__ void walk_quads(const TraceArgs& a, uint32_t n_rays, 
                 v = __builtin_amdgcn_readfirstlane(v) + (uint32_t)__popcll(take & ((1ull << (lane & ~3u)) - 1ull));
                 const uint32_t k = blockIdx.x * share + v;
                 if (idle && more) {
-                    if (v < share && k < n_rays) start<ANY, MULTI>(a, a.order ? a.order[k] : k, w);
+                    if (v < share && k < n_rays) start<ANY, MULTI>(a, a.order ? a.order[k] : k, w, s_gate.slack[lane], s_gate.ray[lane]);
                     else more = false;
                 }
             }
@@ -751,11 +790,16 @@ __device__ __forceinline__ void walk_quads(const TraceArgs& a, uint32_t n_rays, 
             if (walk && w.cur == kNone) {
                 --w.sp;
                 const uint2 e = st[w.sp * 16];
-                if (key_distance(e.y) <= w.lim) w.cur = e.x;
+                if (__uint_as_float(e.y) <= w.lim) w.cur = e.x;
             }
+            bool gated = false;
+            uint32_t first = 0;
             if (walk && (int32_t)w.cur >= 0) {
                 const NodeSlabs n(w.nodes, w.cur, w.s);
-                const uint32_t key = n.key(sub, 8 * sub, w.r.tmin, w.lim);
+                float near;
+                const uint32_t key = n.key(sub, 8 * sub, w.r, w.lim, near);
+                const float ahead_2 = fminf(near, quad_rot_f<0xB1>(near));
+                const float ahead = fminf(ahead_2, quad_rot_f<0x4E>(ahead_2));
                 const uint32_t k1 = quad_rot<0x39>(key), k2 = quad_rot<0x4E>(key), k3 = quad_rot<0x93>(key);
                 const uint32_t nearest = min(min(key, k1), min(k2, k3));
                 // place of this lane's child: hits farther than it lie below
@@ -765,12 +809,16 @@ __device__ __forceinline__ void walk_quads(const TraceArgs& a, uint32_t n_rays, 
                                  (k3 != kNone ? 1 : 0);
                 if (key != kNone && key != nearest) {
                     // always: the host takes this form for trees whose stack fits
-                    if (w.sp + below < kQuadStack) st[(w.sp + below) * 16] = make_uint2(n.ref(key), key);
+                    if (w.sp + below < kQuadStack) st[(w.sp + below) * 16] = make_uint2(n.ref(key), __float_as_uint(ahead));
                     else overflow = true;
                 }
                 w.sp = min(w.sp + max(hits - 1, 0), kQuadStack);
+                gated = n.gated && sub == 0;
+                first = n.first_record();
                 w.cur = nearest != kNone ? n.ref(nearest) : kNone;
             }
+            gates.put(gated, first, lane);
+            if (gates.full()) gates.pass<ANY, MULTI, 4>(a, w, false);
             if (w.at_leaf() && w.leaf == kNone) {
                 w.leaf = w.cur;
                 w.cur = kNone;
@@ -793,7 +841,7 @@ __device__ __forceinline__ void walk_quads(const TraceArgs& a, uint32_t n_rays, 
             const float ta = odd ? to : t, tb = odd ? t : to;
             const bool take_b = tb < ta;
             const bool own = take_b == odd;  // this lane tested the nearer one
-            leaf_outcome<ANY, MULTI>(a, w, ri, take_b ? tb : ta, own ? u : uo, own ? v : vo,
+            leaf_outcome<ANY, MULTI>(a, w, s_gate.slack[lane], ri, take_b ? tb : ta, own ? u : uo, own ? v : vo,
                                      quad_any ? -1.0f : take_b ? ta : (ta == tb ? FLT_INF : tb), take_b ? 1u : 0u);
         }
     }
@@ -804,14 +852,15 @@ __device__ __forceinline__ void walk_quads(const TraceArgs& a, uint32_t n_rays, 
 template <bool ANY, bool MULTI, int LDS, int SPILL>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_walk(TraceArgs a) {
     __shared__ uint2 s_st[LDS * kBlock];  // stacks: (reference, entry distance)
+    __shared__ GateShared s_gate[kBlock / 64];
     __shared__ uint32_t s_next, s_out;
     static_assert(LDS < 16 || LDS * kBlock >= kQuadStack * 16 * (kBlock / 64), "the quads' stacks fit");
     const uint32_t n_rays = a.n_dev ? *a.n_dev : a.n;
     const uint32_t stack = MULTI ? a.walk_stack : a.tree.walk_stack;
     if (LDS >= 16 && stack <= (uint32_t)kQuadStack && n_rays <= kQuadsPerWave * gridDim.x * (kBlock / 64))
-        walk_quads<ANY, MULTI, SPILL>(a, n_rays, s_st, &s_next);
+        walk_quads<ANY, MULTI, SPILL>(a, n_rays, s_st, s_gate[threadIdx.x / 64], &s_next);
     else
-        walk_lanes<ANY, MULTI, LDS, SPILL>(a, n_rays, s_st, &s_next, &s_out);
+        walk_lanes<ANY, MULTI, LDS, SPILL>(a, n_rays, s_st, s_gate[threadIdx.x / 64], &s_next, &s_out);
 }
 
 __global__ void k_walk_reset(uint32_t* counter) {

@@ -71,6 +71,12 @@ void parallel_for(uint32_t n, uint32_t grain, unsigned threads, F f) {
     for (auto& t : th) t.join();
 }
 
+uint32_t float_bits(float f) {
+    uint32_t u;
+    std::memcpy(&u, &f, sizeof(u));
+    return u;
+}
+
 struct Builder {
     const BuildInput& in;
     const std::vector<BuildPrim>& P;
@@ -79,9 +85,13 @@ struct Builder {
     RawVec<uint32_t> ord;            // primitive places, grouped as the walk records take them
     RawVec<uint32_t> place_leaf;     // Fast-BVH leaf (SrcNode index) of each primitive place
     std::vector<uint32_t> root;      // binary root of each SrcNode
-    RawVec<float> sbox;              // 6 per SrcNode
+    RawVec<float> sbox;              // 6 per SrcNode leaf: its box, as the Fast-BVH has it
+    RawVec<float> wbox;              // 6 per SrcNode: the box of what lies below it in this tree
+    const float* bbox;               // the scene's box, and its largest extent
+    float extent;
 
-    Builder(const BuildInput& i, const std::vector<BuildPrim>& p, const std::vector<SrcNode>& s) : in(i), P(p), S(s) {}
+    Builder(const BuildInput& i, const std::vector<BuildPrim>& p, const std::vector<SrcNode>& s, const float* bb, float ext)
+        : in(i), P(p), S(s), bbox(bb), extent(ext) {}
 
     // Arranges it[0..n) as a binary tree: bin nodes from bins[at], the root first. `unit`: the split
     // falls on whole groups of so many items, and a group is a leaf of the primitives it holds
@@ -171,9 +181,9 @@ struct Builder {
         return id;
     }
 
-    // Binary tree over one Fast-BVH leaf: triangles two to a leaf, then the quads one to a leaf. A quad
-    // stands with its Fast-BVH leaf's box: its own corners come from another matrix (light to world)
-    // than its test (world to light), and nothing makes the two agree.
+    // Binary tree over one Fast-BVH leaf: triangles two to a leaf, then the quads one to a leaf. A triangle
+    // stands with its box widened by kWalkWiden of its longest edge (walk.hip), a quad with its Fast-BVH
+    // leaf's box: its own corners come from another matrix (light to world) than its test (world to light).
     void leaf_tree(uint32_t s, uint32_t at, std::vector<Item>& it) {
         const SrcNode& n = S[s];
         it.clear();
@@ -184,6 +194,14 @@ struct Builder {
                 Item x;
                 std::memcpy(x.mn, pass ? &sbox[6 * (size_t)s] : P[i].mn, sizeof(x.mn));
                 std::memcpy(x.mx, pass ? &sbox[6 * (size_t)s + 3] : P[i].mx, sizeof(x.mx));
+                if (!pass) {  // (the box's diagonal is no shorter than the longest edge)
+                    const float e[3] = {x.mx[0] - x.mn[0], x.mx[1] - x.mn[1], x.mx[2] - x.mn[2]};
+                    const float by = kWalkWiden * 1.001f * std::sqrt(e[0] * e[0] + e[1] * e[1] + e[2] * e[2]);
+                    for (int k = 0; k < 3; k++) {
+                        x.mn[k] -= by;
+                        x.mx[k] += by;
+                    }
+                }
                 std::memcpy(x.c, P[i].c, sizeof(x.c));
                 x.ref = i;
                 x.weight = 1;
@@ -195,8 +213,10 @@ struct Builder {
             const uint32_t id = at++;
             const uint32_t l = arrange(it.data(), tris, n.off, 2, at);
             const uint32_t r = arrange(it.data() + tris, nq, n.off + tris, 1, at);
-            std::memcpy(bins[id].mn, &sbox[6 * (size_t)s], 12);
-            std::memcpy(bins[id].mx, &sbox[6 * (size_t)s + 3], 12);
+            for (int k = 0; k < 3; k++) {
+                bins[id].mn[k] = std::min(bins[l].mn[k], bins[r].mn[k]);
+                bins[id].mx[k] = std::max(bins[l].mx[k], bins[r].mx[k]);
+            }
             bins[id].l = (int32_t)l;
             bins[id].r = (int32_t)r;
         } else {
@@ -209,8 +229,8 @@ struct Builder {
         Item it[8];
         for (uint32_t j = 0; j < n.nchild; j++) {
             const uint32_t c = n.first + j;
-            std::memcpy(it[j].mn, &sbox[6 * (size_t)c], 12);
-            std::memcpy(it[j].mx, &sbox[6 * (size_t)c + 3], 12);
+            std::memcpy(it[j].mn, &wbox[6 * (size_t)c], 12);
+            std::memcpy(it[j].mx, &wbox[6 * (size_t)c + 3], 12);
             for (int k = 0; k < 3; k++) it[j].c[k] = (it[j].mn[k] + it[j].mx[k]) * 0.5f;
             it[j].ref = root[c];
             it[j].weight = (S[c].cnt + 1) / 2;
@@ -218,7 +238,14 @@ struct Builder {
         arrange(it, n.nchild, 0, 0, at);
     }
 
-    // The children of the wide node over binary node `b`.
+    // Whether binary node `b` lies in a Fast-BVH leaf (its root or below), and whether it is the root of one
+    // that takes more than one record.
+    bool in_leaf(uint32_t b) const { return b < 2 * (uint32_t)P.size(); }
+    bool gated(uint32_t b) const {
+        return in_leaf(b) && !bins[b].leaf() && 2 * S[place_leaf[b / 2]].off == b;
+    }
+
+    // The children of the wide node over binary node `b`. A gated node below it stays whole.
     uint32_t fold(uint32_t b, uint32_t out[4]) const {
         uint32_t n = 1;
         out[0] = b;
@@ -227,7 +254,7 @@ struct Builder {
             float ba = -1.0f;
             for (uint32_t i = 0; i < n; i++) {
                 const Bin& x = bins[out[i]];
-                if (x.leaf()) continue;
+                if (x.leaf() || (out[i] != b && gated(out[i]))) continue;
                 const float a = x.area();
                 if (a > ba) {
                     ba = a;
@@ -262,7 +289,37 @@ struct Builder {
         t.p2x = c[0]; t.p2y = c[1]; t.p2z = c[2];
     }
 
-    void record(const Bin& b, PrimRec& r, WalkAux& x) const {
+    // The gate word of triangle `id` (layout.h): its normal in 127ths, and how near to its plane's direction a
+    // ray has to run to be let through, in 1,024ths; a triangle so narrow that this says little lets every ray
+    // through (a normal of zeros).
+    uint32_t gate_word(uint32_t id, uint32_t leaf) const {
+        const float* b = &sbox[6 * (size_t)leaf];
+        double across = 0.0;  // the leaf box's diagonal, squared
+        for (int k = 0; k < 3; k++) across += ((double)b[3 + k] - b[k]) * ((double)b[3 + k] - b[k]);
+        const uint32_t* v = in.idx + 3 * (size_t)id;
+        double e[3][3], len[3];  // the edges, and their lengths squared
+        for (int i = 0; i < 3; i++) {
+            len[i] = 0.0;
+            for (int k = 0; k < 3; k++) {
+                e[i][k] = (double)in.pos[3 * (size_t)v[(i + 1) % 3] + k] - (double)in.pos[3 * (size_t)v[i] + k];
+                len[i] += e[i][k] * e[i][k];
+            }
+        }
+        if (len[0] == 0.0 || len[1] == 0.0 || len[2] == 0.0) return kGateShut;  // two equal corners: never hit
+        double n[3];
+        for (int k = 0; k < 3; k++) n[k] = e[0][(k + 1) % 3] * e[1][(k + 2) % 3] - e[0][(k + 2) % 3] * e[1][(k + 1) % 3];
+        const double area = std::sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);  // twice the triangle's
+        const double longest = std::sqrt(std::max(len[0], std::max(len[1], len[2])));
+        const double height = area / longest;
+        const double s = std::max(kGateReach * extent + kGateLeaf * std::sqrt(across), kGateShape * longest) / height;
+        if (!(s <= 1.0 / 16.0)) return 0;
+        uint32_t word = (uint32_t)std::ceil(s * 1024.0) << 24;
+        for (int k = 0; k < 3; k++) word |= ((uint32_t)(int)std::lrint(127.0 * n[k] / area) & 0xffu) << (8 * k);
+        return word;
+    }
+
+    // Fills record `r`, its `x` and its two gate words from the leaf `b`.
+    void record(const Bin& b, PrimRec& r, WalkAux& x, uint32_t* gate) const {
         std::memset(&r, 0, sizeof(r));
         uint32_t place[2] = {ord[~b.l], b.r > 1 ? ord[~b.l + 1] : 0u};
         if (b.r > 1 && place[1] < place[0]) std::swap(place[0], place[1]);  // A before B in build order
@@ -274,10 +331,13 @@ struct Builder {
             std::memcpy(&r.a.p0x, &q, sizeof(q));
             r.a.p1x = std::numeric_limits<float>::quiet_NaN();  // never hit as a triangle
             r.id_a = id | PR_FLAG;
+            gate[0] = gate[1] = kGateShut;
         } else {
             put_tri(r.a, id);
             r.id_a = id;
+            gate[0] = gate[1] = gate_word(id, leaf);
             if (b.r > 1) {
+                gate[1] = gate_word(P[place[1]].id, leaf);
                 put_tri(r.b, P[place[1]].id);
                 r.id_b = P[place[1]].id | PR_FLAG;
             }
@@ -300,11 +360,16 @@ struct Builder {
         RawVec<WalkNode> nodes;
         RawVec<PrimRec> recs;
         RawVec<WalkAux> aux;
+        RawVec<uint32_t> gates;
         uint32_t stack = 0;
     };
     struct Todo {
         uint32_t bin, slot, held;  // held: stack entries below this node on the way to it
     };
+
+    uint32_t records_below(uint32_t b) const {
+        return bins[b].leaf() ? 1u : records_below((uint32_t)bins[b].l) + records_below((uint32_t)bins[b].r);
+    }
 
     // Fills the wide node of `t` in `p`; its inner children are appended to p.nodes and to `more`.
     void wide(const Todo& t, Part& p, std::vector<Todo>& more) const {
@@ -320,10 +385,13 @@ struct Builder {
         w.rec_base = (uint32_t)p.recs.size();
         uint8_t* lo[3] = {w.lo_x, w.lo_y, w.lo_z};
         uint8_t* hi[3] = {w.hi_x, w.hi_y, w.hi_z};
+        const bool gate = gated(t.bin);
         for (int k = 0; k < 3; k++) {
             w.base[k] = b.mn[k];
+            // the last bit of base[0] says whether the node has a gate
+            while (k == 0 && (float_bits(w.base[0]) & 1u) != (gate ? 1u : 0u)) w.base[0] = std::nextafter(w.base[0], -FLT_MAX);
             // smallest power-of-two step with which 255 of them reach the far plane
-            const double ext = (double)b.mx[k] - (double)b.mn[k];
+            const double ext = (double)b.mx[k] - (double)w.base[k];
             int e = 1;
             if (ext > 0.0) {
                 (void)std::frexp(ext / 255.0, &e);  // ext / 255 = m * 2^e, m in [0.5, 1)
@@ -343,7 +411,8 @@ struct Builder {
             }
         }
         const uint32_t held = t.held + n;
-        p.stack = std::max(p.stack, held);
+        // a gate counts its records in a byte
+        p.stack = std::max(p.stack, gate && records_below(t.bin) > 255u ? kWalkMaxStack + 1 : held);
         for (uint32_t j = 0; j < n; j++) {
             if (j < ni) {
                 more.push_back({c[j], (uint32_t)p.nodes.size(), held - 1});
@@ -351,15 +420,44 @@ struct Builder {
             } else {
                 p.recs.emplace_back();
                 p.aux.emplace_back();
-                record(bins[c[j]], p.recs.back(), p.aux.back());
+                p.gates.resize(p.gates.size() + 2);
+                record(bins[c[j]], p.recs.back(), p.aux.back(), &p.gates[p.gates.size() - 2]);
             }
         }
         p.nodes[t.slot] = w;
     }
 
+    // Fills every wide node from `t` down, depth first: the records of a gated node follow one another.
+    void subtree(const Todo& t, Part& p) const {
+        std::vector<Todo> st = {t};
+        while (!st.empty()) {
+            const Todo x = st.back();
+            st.pop_back();
+            const size_t first = p.recs.size();
+            if (gated(x.bin)) {
+                std::vector<Todo> in_leaf;
+                wide(x, p, in_leaf);
+                while (!in_leaf.empty()) {
+                    const Todo y = in_leaf.back();
+                    in_leaf.pop_back();
+                    wide(y, p, in_leaf);
+                }
+                // the first two words carry what the whole gate needs: its records and its widest reach
+                uint32_t s = 0;
+                for (size_t i = 2 * first; i < p.gates.size(); i++) s = std::max(s, p.gates[i] >> 24);
+                uint32_t* g = &p.gates[2 * first];
+                g[0] = (g[0] & 0xffffffu) | (uint32_t)(p.recs.size() - first) << 24;
+                g[1] = (g[1] & 0xffffffu) | s << 24;
+            } else {
+                wide(x, p, st);
+            }
+        }
+    }
+
     void run(unsigned threads, WalkTree& out) {
         const uint32_t n = (uint32_t)P.size(), ns = (uint32_t)S.size();
         sbox.resize(6 * (size_t)ns);
+        wbox.resize(6 * (size_t)ns);
         root.resize(ns);
         ord.resize(n);
         place_leaf.resize(n);
@@ -380,14 +478,24 @@ struct Builder {
             }
             static thread_local std::vector<Item> it;
             leaf_tree(leaves[i], root[leaves[i]], it);
+            const Bin& r = bins[root[leaves[i]]];
+            float* w = &wbox[6 * (size_t)leaves[i]];
+            std::memcpy(w, r.mn, 12);
+            std::memcpy(w + 3, r.mx, 12);
         });
         for (uint32_t i = (uint32_t)inner.size(); i-- > 0;) {  // children follow their parents
             const SrcNode& s = S[inner[i]];
-            float* b = &sbox[6 * (size_t)inner[i]];
+            float* b = &wbox[6 * (size_t)inner[i]];
             empty_box(b, b + 3);
-            for (uint32_t j = 0; j < s.nchild; j++) grow(b, b + 3, &sbox[6 * (size_t)(s.first + j)], &sbox[6 * (size_t)(s.first + j) + 3]);
+            for (uint32_t j = 0; j < s.nchild; j++) grow(b, b + 3, &wbox[6 * (size_t)(s.first + j)], &wbox[6 * (size_t)(s.first + j) + 3]);
         }
         parallel_for((uint32_t)inner.size(), 256, threads, [&](uint32_t i) { inner_tree(inner[i], root[inner[i]]); });
+
+        // a tree of one record: nothing bounds it but the scene's box
+        if (S[0].nchild == 0 && bins[root[0]].leaf()) {
+            std::memcpy(bins[root[0]].mn, bbox, 12);
+            std::memcpy(bins[root[0]].mx, bbox + 3, 12);
+        }
 
         // fold: the upper nodes one after another, then one part per subtree
         Part top;
@@ -397,21 +505,18 @@ struct Builder {
         const size_t parts_wanted = n < 16384 ? SIZE_MAX : 512;
         while (head < queue.size() && queue.size() - head < parts_wanted) {
             const Todo t = queue[head++];
-            wide(t, top, queue);
+            if (gated(t.bin)) subtree(t, top);
+            else wide(t, top, queue);
         }
         const uint32_t np = (uint32_t)(queue.size() - head);
         std::vector<Part> parts(np);
         parallel_for(np, 1, threads, [&](uint32_t i) {
-            std::vector<Todo> st = {{queue[head + i].bin, 0, queue[head + i].held}};
             parts[i].nodes.reserve(n / np);
             parts[i].recs.reserve(n / np);
             parts[i].aux.reserve(n / np);
+            parts[i].gates.reserve(2 * (n / np));
             parts[i].nodes.emplace_back();
-            while (!st.empty()) {
-                const Todo t = st.back();
-                st.pop_back();
-                wide(t, parts[i], st);
-            }
+            subtree({queue[head + i].bin, 0, queue[head + i].held}, parts[i]);
         });
         // a part's node 0 takes the slot its parent kept; the others follow the nodes before them
         std::vector<uint64_t> nbase(np + 1), rbase(np + 1);
@@ -430,6 +535,7 @@ struct Builder {
         out.nodes.resize(nbase[np]);
         out.recs.resize(rbase[np] + kWalkPadRecs);
         out.aux.resize(rbase[np] + kWalkPadRecs);
+        out.gates.resize(2 * rbase[np] + kGatePad);
         PrimRec none;  // a triangle of three equal corners is never hit
         std::memset(&none, 0, sizeof(none));
         none.id_b = PR_NONE | PR_FLAG;
@@ -438,6 +544,8 @@ struct Builder {
         std::copy(top.nodes.begin(), top.nodes.end(), out.nodes.begin());
         std::copy(top.recs.begin(), top.recs.end(), out.recs.begin());
         std::copy(top.aux.begin(), top.aux.end(), out.aux.begin());
+        std::fill(out.gates.end() - kGatePad, out.gates.end(), 0u);
+        std::copy(top.gates.begin(), top.gates.end(), out.gates.begin());
         parallel_for(np, 1, threads, [&](uint32_t i) {
             const Part& p = parts[i];
             for (size_t k = 0; k < p.nodes.size(); k++) {
@@ -448,6 +556,7 @@ struct Builder {
             }
             std::copy(p.recs.begin(), p.recs.end(), out.recs.begin() + rbase[i]);
             std::copy(p.aux.begin(), p.aux.end(), out.aux.begin() + rbase[i]);
+            std::copy(p.gates.begin(), p.gates.end(), out.gates.begin() + 2 * rbase[i]);
         });
         out.stack = stack;
     }
@@ -468,11 +577,36 @@ void build_walk_tree(const BuildInput& in, const std::vector<BuildPrim>& prims, 
     for (const BuildPrim& p : prims)  // an axis on which every coordinate is NaN has a box that bounds nothing
         for (int k = 0; k < 3; k++)
             if (!(p.mn[k] <= p.mx[k]) || !(p.mn[k] >= bbox[k] && p.mx[k] <= bbox[3 + k])) return;
-    if (far > 1e12f || far > 4096.0f * ext) return;
+    if (far > 1e12f || far < 1e-8f || far > 4096.0f * ext) return;
     if (prims.size() / 2 * sizeof(PrimRec) > UINT32_MAX) return;
-    Builder b(in, prims, src);
+    // A quad is tested in its own space: what the walk sees of its rounding and of the disagreement of its
+    // matrices, as a part of the largest coordinate.
+    double off = 0.0;
+    for (uint32_t q = 0; q < in.nquads; q++) {
+        const float *m = in.quads[q].mat, *v = in.quads[q].inv;
+        for (int k = 0; k < 4; k++)
+            if (m[12 + k] != (k == 3 ? 1.0f : 0.0f) || v[12 + k] != (k == 3 ? 1.0f : 0.0f)) return;
+        for (int k = 0; k < 3; k++) {
+            double wrong = 0.0, shift = m[4 * k + 3], round = 0.0;
+            for (int j = 0; j < 3; j++) {
+                double e = k == j ? -1.0 : 0.0, row = 0.0;
+                for (int i = 0; i < 3; i++) {
+                    e += (double)m[4 * k + i] * v[4 * i + j];
+                    row += 16.0 * std::fabs((double)v[4 * j + i]);
+                }
+                wrong += std::fabs(e);
+                shift += (double)m[4 * k + j] * v[4 * j + 3];
+                round += std::fabs((double)m[4 * k + j]) * (row + 4.0 * std::fabs((double)v[4 * j + 3]) / far);
+            }
+            const double axis = wrong + std::fabs(shift) / far + round * kUnit;
+            if (!(axis <= 1.0 / 4096)) return;
+            off = std::max(off, axis);
+        }
+    }
+    Builder b(in, prims, src, bbox, ext);
     b.run(prims.size() < 16384 ? 1u : threads, out);
     if (!out.stack) out = WalkTree();
+    out.pad = std::max(kPadUnits * kUnit, (float)off * 1.0001f + kPadOther * kUnit);
 }
 
 }  // namespace sortgpu

@@ -213,3 +213,78 @@ def test_windows_of_one_float(gpu_ctx, n):
         rays = scenes.make_rays(o, d, lo, at)
         found = _check(acc, ob, rays, f"{ulps} ulps, {n} triangles")
         assert np.mean(found[:, 1].view(np.uint32) != MISS) > 0.5
+
+
+def _sheets(n):
+    """Two parallel tilted sheets of n x n squares, and a function for points of the first one's plane."""
+    c, a, b = np.array([0.1, 0.05, 0.2]), np.array([0.9, 0.31, -0.17]), np.array([-0.23, 0.77, 0.41])
+    up = np.cross(a, b) / np.linalg.norm(np.cross(a, b))
+    at = lambda i, j, k: (c + a * i / n + b * j / n + 0.25 * k * up).astype(np.float32)
+    tris = []
+    for k in (0, 1):
+        for i in range(n):
+            for j in range(n):
+                p = [at(i, j, k), at(i + 1, j, k), at(i + 1, j + 1, k), at(i, j + 1, k)]
+                tris += [np.stack(p[:3]), np.stack([p[0], p[2], p[3]])]
+    return scenes.tris_to_mesh(tris), lambda x, y, off: (c + x[:, None] * a + y[:, None] * b + off[:, None] * up).astype(np.float32)
+
+
+@pytest.mark.parametrize("width", [8, 4])
+@pytest.mark.parametrize("n", [4, 16, 48])
+def test_rays_in_the_plane_of_a_tilted_sheet(gpu_ctx, width, n):
+    """Edge-on, the triangle test accepts rays far beside a triangle; every such hit of the Fast-BVH has to be
+    there, in the lanes' form, the quads', through a pool, and with windows."""
+    g = np.random.default_rng(n)
+    mesh, point = _sheets(n)
+    acc, ob = _build(gpu_ctx, width, mesh, None)
+    m = 30000
+    for off in (0.0, 1e-6, 1e-5):
+        o, e = (point(g.uniform(-0.2, 1.2, m), g.uniform(-0.2, 1.2, m), g.uniform(-off, off, m)) for _ in range(2))
+        o[::3] = mesh[0][g.integers(0, len(mesh[0]) // 2, len(o[::3]))]
+        rays = scenes.make_rays(o, (e - o).astype(np.float32), 0.0, FLT_MAX)
+        hits = _check(acc, ob, rays, f"sheet {n} off {off}")
+        tmin = g.uniform(0, 0.5, m).astype(np.float32)
+        _check(acc, ob, scenes.make_rays(o, (e - o).astype(np.float32), tmin, tmin + np.float32(0.3)), "windowed")
+        pool = batch.Pool(gpu_ctx, [acc, acc])
+        got = pool.trace(torch.from_numpy(rays).cuda(), torch.from_numpy((np.arange(m) % 2).astype(np.int32)).cuda()).cpu().numpy()
+        assert np.array_equal(got.view(np.uint32), hits.view(np.uint32))
+        pool.close()
+
+
+@pytest.mark.parametrize("width", [8, 4])
+@pytest.mark.parametrize("tiny", [3e-6, 1e-6, 1e-7, 1e-19])
+def test_tiny_triangles_and_needles_among_others(gpu_ctx, width, tiny):
+    """Half of the triangles at the size of the arithmetic's rounding (or the whole scene below underflow),
+    a tenth of the others long needles; rays at vertices and along the needles."""
+    g = np.random.default_rng(int(-np.log10(tiny)))
+    n = 4000
+    size = np.where(np.arange(n) % 2, 0.2, max(tiny, 1e-7))[:, None, None] * np.ones((n, 1, 3))
+    size[np.arange(n) % 20 == 1] = [1e-6, 1e-6, 0.4]
+    t = (g.uniform(0, 1, (n, 1, 3)) + g.uniform(-0.5, 0.5, (n, 3, 3)) * size) * (tiny if tiny < 1e-10 else 1.0)
+    mesh = scenes.tris_to_mesh(list(t.astype(np.float32)))
+    acc, ob = _build(gpu_ctx, width, mesh, None)
+    o, d = _rays(g, 40000, mesh)
+    k = np.arange(len(o))
+    needle = mesh[0].reshape(-1, 3, 3)[g.integers(0, n // 20, len(o)) * 20 + 1]
+    along = (needle[:, 1] - needle[:, 0]) * np.float32(1.0)
+    o = np.where((k % 3 == 0)[:, None], needle[:, 0] - 2 * along, o).astype(np.float32)
+    d = np.where((k % 3 == 0)[:, None], along, d).astype(np.float32)
+    if tiny > 1e-10:
+        d /= np.maximum(np.linalg.norm(d, axis=1, keepdims=True), 1e-20).astype(np.float32)
+    _check(acc, ob, scenes.make_rays(o, d, 0.0, FLT_MAX), f"tiny {tiny}")
+
+
+def test_directions_below_the_slab_clamp(gpu_ctx):
+    """The Fast-BVH steps through its boxes along a direction of no component below 1e-5: rays with smaller
+    ones, of several lengths, in a flat scene and a soup."""
+    g = np.random.default_rng(17)
+    for mesh in (_sheets(16)[0], scenes.tris_to_mesh(list((g.uniform(0, 1, (4000, 1, 3)) + g.uniform(-0.05, 0.05, (4000, 3, 3))).astype(np.float32)))):
+        acc, ob = _build(gpu_ctx, 8, mesh, None)
+        o, d = _rays(g, 32000, mesh)
+        k = np.arange(len(o))
+        d[k, k % 3] = g.uniform(-1.2e-5, 1.2e-5, len(o))
+        d[k % 5 == 0] *= np.float32(1e-3)
+        d[k % 5 == 1, 0] = 0.0
+        d[k % 7 == 2] *= np.float32(30.0)
+        o[k % 2 == 0] = (mesh[0][g.integers(0, len(mesh[0]), len(o))] - 0.7 * d)[k % 2 == 0]
+        _check(acc, ob, scenes.make_rays(o, d.astype(np.float32), 0.0, FLT_MAX), "clamped directions")

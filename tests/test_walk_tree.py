@@ -8,8 +8,8 @@ CSRC = os.path.join(ROOT, "sort_amd", "csrc")
 
 def _run(tmp_path, name):
     exe = str(tmp_path / name)
-    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-pthread", "-I", CSRC, "-o", exe,
-                    os.path.join(ROOT, "tests", "native", name + ".cpp"), os.path.join(CSRC, "bvh_build.cpp"),
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-pthread", "-Wno-unknown-pragmas", "-I", CSRC,
+                    "-I", os.path.join(ROOT, "tests", "native", "host_hip"), "-o", exe, os.path.join(ROOT, "tests", "native", name + ".cpp"), os.path.join(CSRC, "bvh_build.cpp"),
                     os.path.join(CSRC, "walk_tree.cpp")], check=True)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
@@ -21,3 +21,7 @@ def test_walk_tree_invariants(tmp_path):
 
 def test_no_triangle_record_holds_a_nan(tmp_path):
     _run(tmp_path, "walk_tree_nan_check")
+
+
+def test_a_walk_reaches_every_triangle_that_decides(tmp_path):
+    _run(tmp_path, "walk_complete_check")

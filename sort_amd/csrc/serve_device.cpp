@@ -534,8 +534,10 @@ class HostDevice : public Device {
         int rc = prepare_scene(ctx_, acc, desc, true, im);
         if (rc) return (err = sortgpu_last_error(ctx_), rc);
         *bytes = im.block_bytes();
+        lean_.push_back(im.walk.stack ? im.block_bytes(true) : 0);
         return SORTGPU_OK;
     }
+    size_t lean_bytes(uint32_t id) const override { return lean_[id]; }
     int load_scene(uint32_t, std::string&) override { return SORTGPU_OK; }
     void unload_scene(uint32_t) override {}
     int alloc_film(Request& r, std::string&) override {
@@ -596,6 +598,7 @@ class HostDevice : public Device {
     }
 
   private:
+    std::vector<size_t> lean_;
     sortgpu_ctx* ctx_;
     uint32_t cap_, polls_;
     std::vector<std::vector<float>*> films_;

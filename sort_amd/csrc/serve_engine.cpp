@@ -324,17 +324,22 @@ void Engine::admit() {
         size_t need = (s.resident ? 0 : s.bytes) + r->film_bytes;
         bool lean = false;
         if (!evict_for(need, r->p.scene)) {
-            // the whole budget is not enough for it: its smaller form, if that fits
-            const size_t small = s.resident ? 0 : dev_->lean_bytes(r->p.scene);
-            if (active_.empty() && inflight_.empty() && small && evict_for(small + r->film_bytes, r->p.scene)) {
-                lean = true;
-            } else if (active_.empty() && inflight_.empty()) {
+            if (!active_.empty() || !inflight_.empty()) return;
+            // The whole budget is not enough for it: the scene's smaller form, if that fits. A larger one that
+            // an earlier request loaded makes way for it.
+            const size_t small = dev_->lean_bytes(r->p.scene);
+            if (small && s.resident && s.held > small && used_ - s.held + small + r->film_bytes <= o_.budget) {
+                dev_->unload_scene(r->p.scene);
+                s.resident = false;
+                used_ -= s.held;
+                n_evict_++;
+            }
+            lean = small && !s.resident && evict_for(small + r->film_bytes, r->p.scene);
+            if (!lean) {
                 finish(r, SORTGPU_REQ_FAILED, SORTGPU_ERR_BUDGET,
                        "needs " + std::to_string(need) + " bytes; the HBM budget is " + std::to_string(o_.budget) +
                            " with " + std::to_string(used_) + " in use");
                 continue;
-            } else {
-                return;
             }
         }
         std::string err;

@@ -54,6 +54,8 @@ class ThreadDevice : public Device {
         *bytes = 300000;
         return SORTGPU_OK;
     }
+    size_t lean_bytes(uint32_t) const override { return 200000; }
+    void use_lean(uint32_t, bool lean) override { leans_ += lean; }
     int load_scene(uint32_t, std::string&) override { return SORTGPU_OK; }
     void unload_scene(uint32_t) override {}
     int alloc_film(Request& r, std::string& err) override {
@@ -110,6 +112,7 @@ class ThreadDevice : public Device {
         return SORTGPU_OK;
     }
     void counters(uint64_t out[3]) override { out[0] = out[1] = out[2] = 0; }
+    uint64_t leans() const { return leans_; }
 
   private:
     struct Part {
@@ -146,7 +149,7 @@ class ThreadDevice : public Device {
         }
     }
     uint32_t cap_;
-    std::atomic<uint64_t> allocs_{0};
+    std::atomic<uint64_t> allocs_{0}, leans_{0};
     std::mutex mu_;
     std::condition_variable cv_, cv_done_;
     std::deque<Job> jobs_;
@@ -171,13 +174,16 @@ bool check_image(const std::vector<float>& rgb, uint64_t seed, uint32_t scene, u
 // One run of six clients against one engine. manual: no worker thread; the clients' own wait and
 // drain calls drive the engine, so several threads poll it at once and take turns waiting on the
 // device with the engine's lock released.
-int run(bool manual) {
+// tight: room for one scene only, with a small film in its full form and any film in its smaller one.
+int run(bool manual, bool tight = false) {
     Options o;
     o.budget = (1 << 20) + 4 * 300000 + 64 * 64 * 16 * 6;  // workspace + 4 scenes + six 64^2 films
+    if (tight) o.budget = (1 << 20) + 300000 + 20 * 20 * 16;
     o.max_active = 6;
     o.inflight = 3;
     o.manual = manual;
-    Engine eng(std::unique_ptr<Device>(new ThreadDevice(4096)), o);
+    ThreadDevice* dev = new ThreadDevice(4096);
+    Engine eng(std::unique_ptr<Device>(dev), o);
     std::string err;
     if (eng.start(err)) {
         std::fprintf(stderr, "start: %s\n", err.c_str());
@@ -239,11 +245,13 @@ int run(bool manual) {
                 (unsigned long long)st[0], (unsigned long long)st[5], (unsigned long long)st[8],
                 (unsigned long long)st[14]);
     if (st[8] > st[14]) bad++;
+    if (tight && !dev->leans()) bad++;
     return bad.load() == 0 && done.load() > 100 ? 0 : 1;
 }
 
 int main() {
     const int a = run(false);
     const int b = run(true);
-    return a | b;
+    const int c = run(false, true), d = run(true, true);
+    return a | b | c | d;
 }

@@ -132,6 +132,44 @@ def test_eviction_and_cancellation_leave_results_unchanged(gpu_ctx, world):
     srv.close()
 
 
+@pytest.mark.parametrize("graphs", [False, True])
+def test_scenes_without_their_second_tree_for_the_budget(gpu_ctx, world, graphs):
+    """A budget that holds the largest scene (2) only without its walk tree, or with it and a small film: loaded
+    so at once, loaded whole first and then again, and in one wave with a scene (3) that has its walk tree."""
+    probe, ids = _server(gpu_ctx, world, wave_paths=1 << 16, manual=True, graphs=graphs)
+    fixed, sizes = probe.stats()["workspace_bytes"], {}
+    for k in (2, 3):
+        before = probe.stats()["bytes_in_use"]
+        probe.submit(ids[k], S.random_camera(np.random.default_rng(0)), 8, 8, 1)
+        probe.drain()
+        sizes[k] = probe.stats()["bytes_in_use"] - before
+    probe.close()
+    budget = fixed + sizes[2] + 8 * 8 * 16
+    g = np.random.default_rng(31)
+    for order in ([(2, 64), (2, 8)], [(2, 8), (2, 64)], [(2, 64), (3, 64)], [(2, 8), (2, 64), (3, 64)]):
+        srv, ids = _server(gpu_ctx, world, wave_paths=1 << 16, hbm_budget=budget, manual=True, graphs=graphs)
+        for again in range(3):  # a captured wave graph is replayed
+            reqs = [(k, n, S.random_camera(g), 700 + 10 * again + i) for i, (k, n) in enumerate(order)]
+            together = order[-1][0] != order[0][0]
+            rids = []
+            for i, (k, n, cam, seed) in enumerate(reqs):
+                rids.append(srv.submit(ids[k], cam, n, n, 4, 5, seed))
+                if not together or i < len(reqs) - 2:
+                    srv.drain()
+            waves = srv.stats()["waves"]
+            srv.drain()
+            if together:
+                assert srv.stats()["waves"] == waves + 1
+            print(f"[serve] {order} graphs {graphs}: {srv.stats()}", flush=True)
+            for (k, n, cam, seed), rid in zip(reqs, rids):
+                assert srv.info(rid)["state"] == "done", (order, srv.message(rid))
+                ref = _plain(world, k, cam, n, n, 4, 5, seed)
+                assert np.array_equal(srv.result(rid).view(np.uint32), ref.view(np.uint32)), (order, k, n)
+                srv.release(rid)
+            assert srv.stats()["peak_bytes"] <= budget
+        srv.close()
+
+
 def test_multi_wave_render_equals_served(gpu_ctx, world):
     """A frame the single-request render splits into waves (1024^2 at 8 spp: three waves of 3, 3 and
     2 samples on its three streams) equals, bit for bit, the server's result for the same request

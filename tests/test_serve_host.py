@@ -116,6 +116,29 @@ def test_budget_eviction_lru(hctx, built):
     s.close()
 
 
+@pytest.mark.parametrize("order", [(8, 64, 8), (64, 8, 64), (8, 64, 64, 8, 64)])
+def test_larger_film_on_a_resident_scene_takes_its_smaller_form(hctx, built, order):
+    """A budget that holds a scene with a small film, and with a large one only the scene's form without its
+    second tree: the requests succeed in any order, with the results of an unbounded server."""
+    probe, ids = make_server(hctx, built, manual=True, wave_paths=4096)
+    fixed = probe.stats()["workspace_bytes"]
+    probe.submit(ids[3], CAM, 8, 8, 1)
+    probe.drain()
+    scene = probe.stats()["bytes_in_use"] - fixed
+    probe.close()
+    s, ids = make_server(hctx, built, manual=True, wave_paths=4096, hbm_budget=fixed + scene + 8 * 8 * 16)
+    for k, size in enumerate(order):
+        rid = s.submit(ids[3], CAM, size, size, 3, seed=40 + k)
+        s.drain()
+        assert s.info(rid)["state"] == "done", (k, s.message(rid))
+        ref = alone(hctx, built, 3, size, size, 3, 40 + k)
+        assert np.array_equal(s.result(rid).view(np.uint32), ref.view(np.uint32))
+        s.release(rid)
+    st = s.stats()
+    assert st["failed"] == 0 and st["peak_bytes"] <= st["budget"]
+    s.close()
+
+
 def test_request_over_budget_fails_cleanly(hctx, built):
     probe, _ = make_server(hctx, built, manual=True, wave_paths=1 << 16)
     fixed = probe.stats()["workspace_bytes"]

@@ -7,20 +7,26 @@
 
 namespace sortgpu {
 
+static void free_walk(sortgpu_accel* acc) {
+    void* ptrs[] = {acc->d_wnodes, acc->d_wrecs, acc->d_waux, acc->d_wgates};
+    for (void* p : ptrs)
+        if (p) hipFree(p);
+    acc->d_wnodes = nullptr;
+    acc->d_wrecs = nullptr;
+    acc->d_waux = nullptr;
+    acc->d_wgates = nullptr;
+}
+
 void free_accel_device(sortgpu_accel* acc) {
     if (!acc || !acc->ctx || acc->ctx->host_only) return;
     ctx_bind(acc->ctx);
-    void* ptrs[] = {acc->d_nodes, acc->d_prims,  acc->d_quads,    acc->d_wnodes, acc->d_wrecs,
-                    acc->d_waux,  acc->d_wgates, acc->d_counters, acc->d_error,  acc->d_stats};
+    free_walk(acc);
+    void* ptrs[] = {acc->d_nodes, acc->d_prims, acc->d_quads, acc->d_counters, acc->d_error, acc->d_stats};
     for (void* p : ptrs)
         if (p) hipFree(p);
     acc->d_nodes = nullptr;
     acc->d_prims = nullptr;
     acc->d_quads = nullptr;
-    acc->d_wnodes = nullptr;
-    acc->d_wrecs = nullptr;
-    acc->d_waux = nullptr;
-    acc->d_wgates = nullptr;
     acc->d_counters = nullptr;
     acc->d_error = nullptr;
     acc->d_stats = nullptr;
@@ -53,14 +59,6 @@ int upload_accel(sortgpu_accel* acc) {
         (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_prims), h.prims.data(), pb, "hipMalloc(prims)")) ||
         (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_quads), qb ? h.quads.data() : nullptr, qb,
                              "hipMalloc(quads)")) ||
-        (wb && ((rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_wnodes), h.walk.nodes.data(), wb,
-                                     "hipMalloc(walk nodes)")) ||
-                (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_wrecs), h.walk.recs.data(), rb,
-                                     "hipMalloc(walk records)")) ||
-                (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_waux), h.walk.aux.data(), xb,
-                                     "hipMalloc(walk leaf boxes)")) ||
-                (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_wgates), h.walk.gates.data(), gb,
-                                     "hipMalloc(walk gates)")))) ||
         (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_counters), nullptr,
                              kCounterSlots * kCounterStride * sizeof(uint32_t), "hipMalloc(counters)")) ||
         (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_error), nullptr, 16, "hipMalloc(error)")) ||
@@ -68,7 +66,28 @@ int upload_accel(sortgpu_accel* acc) {
         free_accel_device(acc);
         return rc;
     }
-    acc->device_bytes = nb + pb + qb + wb + rb + xb + gb;
+    // The walk tree makes queries faster and is done without where its memory is not to be had.
+    size_t walk = 0;
+    if (wb) {
+        if ((rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_wnodes), h.walk.nodes.data(), wb,
+                                 "hipMalloc(walk nodes)")) ||
+            (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_wrecs), h.walk.recs.data(), rb,
+                                 "hipMalloc(walk records)")) ||
+            (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_waux), h.walk.aux.data(), xb,
+                                 "hipMalloc(walk leaf boxes)")) ||
+            (rc = dev_alloc_copy(ctx, reinterpret_cast<void**>(&acc->d_wgates), h.walk.gates.data(), gb,
+                                 "hipMalloc(walk gates)"))) {
+            if (rc != SORTGPU_ERR_OOM) {
+                free_accel_device(acc);
+                return rc;
+            }
+            (void)hipGetLastError();
+            free_walk(acc);
+        } else {
+            walk = wb + rb + xb + gb;
+        }
+    }
+    acc->device_bytes = nb + pb + qb + walk;
     acc->view.nodes = acc->d_nodes;
     acc->view.prims = acc->d_prims;
     acc->view.quads = acc->d_quads;
@@ -76,7 +95,7 @@ int upload_accel(sortgpu_accel* acc) {
     acc->view.wrecs = acc->d_wrecs;
     acc->view.waux = acc->d_waux;
     acc->view.wgates = acc->d_wgates;
-    acc->view.walk_stack = h.walk.stack;
+    acc->view.walk_stack = walk ? h.walk.stack : 0;
     acc->view.walk_pad = h.walk.pad;
     return 0;
 }

@@ -563,7 +563,11 @@ bool build_tree(const BuildInput& in, BuiltTree& out, std::string& err) {
         out.prims = std::move(F.prims);
         out.dump = std::move(F.dump);
     }
-    build_walk_tree(in, B.P, source_nodes(root.get(), out.n_inner + out.n_leaves), out.bbox, nthreads, out.walk);
+    try {
+        build_walk_tree(in, B.P, source_nodes(root.get(), out.n_inner + out.n_leaves), out.bbox, nthreads, out.walk);
+    } catch (const std::bad_alloc&) {
+        out.walk = WalkTree();
+    }
     out.build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return true;
 }

@@ -63,9 +63,10 @@ int sortgpu_pool_create(sortgpu_ctx* ctx, sortgpu_accel* const* accels, uint32_t
         walk_stack = std::max(walk_stack, a->host.walk.stack);
     }
     if (!walk) walk_stack = 0;
+    size_t walk_total = 0;
     for (uint32_t i = 0; i < n && walk_stack; i++) {
         const WalkTree& w = accels[i]->host.walk;
-        total += align256(w.nodes.size() * sizeof(WalkNode)) + align256(w.recs.size() * sizeof(PrimRec)) +
+        walk_total += align256(w.nodes.size() * sizeof(WalkNode)) + align256(w.recs.size() * sizeof(PrimRec)) +
                  align256(w.aux.size() * sizeof(WalkAux)) + align256(w.gates.size() * sizeof(uint32_t));
     }
     if (!width) width = 8;
@@ -83,15 +84,26 @@ int sortgpu_pool_create(sortgpu_ctx* ctx, sortgpu_accel* const* accels, uint32_t
     p->n = n;
     p->width = width;
     p->max_stack = max_stack;
-    p->walk_stack = walk_stack;
-    for (uint32_t i = 0; i < n && walk_stack; i++) p->walk_bytes += walk_bytes(accels[i]->host);
     hipError_t e;
     auto fail = [&](hipError_t err, const char* what) {
         int r = hip_fail(ctx, err, what);
         sortgpu_pool_destroy(p);
         return r;
     };
-    if ((e = hipMalloc(&p->d_block, std::max<size_t>(total, 256))) != hipSuccess) return fail(e, "hipMalloc(pool)");
+    e = hipMalloc(&p->d_block, std::max<size_t>(total + walk_total, 256));
+    if (e == hipErrorOutOfMemory && walk_total) {  // without the walk trees, which only make queries faster
+        (void)hipGetLastError();
+        walk_stack = 0;
+        walk_total = 0;
+        e = hipMalloc(&p->d_block, std::max<size_t>(total, 256));
+    }
+    if (e != hipSuccess) {
+        p->d_block = nullptr;
+        return fail(e, "hipMalloc(pool)");
+    }
+    total += walk_total;
+    p->walk_stack = walk_stack;
+    for (uint32_t i = 0; i < n && walk_stack; i++) p->walk_bytes += walk_bytes(accels[i]->host);
     if ((e = hipMalloc(reinterpret_cast<void**>(&p->d_views), std::max<size_t>(n, 1) * sizeof(TreeView))) != hipSuccess)
         return fail(e, "hipMalloc(pool views)");
     if ((e = hipMalloc(reinterpret_cast<void**>(&p->d_counters), kCounterSlots * kCounterStride * sizeof(uint32_t))) !=

@@ -345,9 +345,15 @@ void Engine::admit() {
         std::string err;
         int rc;
         if (!s.resident) {
-            const size_t bytes = lean ? dev_->lean_bytes(r->p.scene) : s.bytes;
+            size_t bytes = lean ? dev_->lean_bytes(r->p.scene) : s.bytes;
             dev_->use_lean(r->p.scene, lean);
-            if ((rc = reserve(bytes, err)) || (rc = dev_->load_scene(r->p.scene, err))) {
+            if ((rc = reserve(bytes, err)) == 0 && (rc = dev_->load_scene(r->p.scene, err)) == SORTGPU_ERR_OOM &&
+                !lean && dev_->lean_bytes(r->p.scene)) {  // the device has less than the budget says
+                bytes = dev_->lean_bytes(r->p.scene);
+                dev_->use_lean(r->p.scene, true);
+                rc = dev_->load_scene(r->p.scene, err);
+            }
+            if (rc) {
                 finish(r, SORTGPU_REQ_FAILED, rc, "scene load failed: " + err);
                 continue;
             }

@@ -8,6 +8,7 @@
 #include <cstring>
 #include <limits>
 #include <memory>
+#include <new>
 #include <thread>
 
 #include "bvh_build.h"
@@ -57,18 +58,31 @@ void parallel_for(uint32_t n, uint32_t grain, unsigned threads, F f) {
         return;
     }
     std::atomic<uint32_t> next{0};
+    std::atomic<bool> short_of_memory{false};  // an exception may not leave a thread
     auto work = [&] {
-        while (true) {
-            const uint32_t a = next.fetch_add(grain);
-            if (a >= n) return;
-            const uint32_t b = std::min(n, a + grain);
-            for (uint32_t i = a; i < b; i++) f(i);
+        try {
+            while (!short_of_memory) {
+                const uint32_t a = next.fetch_add(grain);
+                if (a >= n) return;
+                const uint32_t b = std::min(n, a + grain);
+                for (uint32_t i = a; i < b; i++) f(i);
+            }
+        } catch (const std::bad_alloc&) {
+            short_of_memory = true;
         }
     };
     std::vector<std::thread> th;
-    for (unsigned w = 1; w < want; w++) th.emplace_back(work);
+    th.reserve(want);
+    for (unsigned w = 1; w < want; w++) {
+        try {
+            th.emplace_back(work);
+        } catch (const std::exception&) {
+            break;  // no more threads to be had: those there are do the work
+        }
+    }
     work();
     for (auto& t : th) t.join();
+    if (short_of_memory) throw std::bad_alloc();
 }
 
 uint32_t float_bits(float f) {
@@ -603,8 +617,12 @@ void build_walk_tree(const BuildInput& in, const std::vector<BuildPrim>& prims, 
             off = std::max(off, axis);
         }
     }
-    Builder b(in, prims, src, bbox, ext);
-    b.run(prims.size() < 16384 ? 1u : threads, out);
+    try {
+        Builder b(in, prims, src, bbox, ext);
+        b.run(prims.size() < 16384 ? 1u : threads, out);
+    } catch (const std::bad_alloc&) {  // queries go without
+        out.stack = 0;
+    }
     if (!out.stack) out = WalkTree();
     out.pad = std::max(kPadUnits * kUnit, (float)off * 1.0001f + kPadOther * kUnit);
 }

@@ -61,7 +61,7 @@ constexpr double kGateReach = 52.0 * kUnit, kGateLeaf = 18.0 * kUnit, kGateShape
 // Leaves `out` empty when the tree cannot have a walk tree: boxes not finite, past 1e12 or below 1e-8 (the
 // kernel's error bounds need products that neither overflow nor underflow), far smaller than their distance from the origin
 // (its padding would swallow them), a quad whose two matrices are not each other's inverse, records past 4 GiB,
-// or a deeper stack than kWalkMaxStack.
+// or a deeper stack than kWalkMaxStack, or no host memory for it.
 void build_walk_tree(const BuildInput& in, const std::vector<BuildPrim>& prims, const std::vector<SrcNode>& src,
                      const float bbox[6], unsigned threads, WalkTree& out);
 

@@ -361,7 +361,7 @@ static int trace_common(sortgpu_accel* acc, const sortgpu_ray* d_rays, uint32_t 
     }
     // traversal order (results do not depend on it; the counter launch keeps index order)
     RayOrder ro;
-    if (!stats) a.order = traversal_order(acc, d_rays, n, reorder_pays(n, acc->view.walk_stack ? walk_bytes(acc->host) : 0), s, ro);
+    if (!stats) a.order = traversal_order(acc, d_rays, n, reorder_pays(n, walked_bytes(acc)), s, ro);
     hipError_t e = launch_trace(a, any, stats, s, ctx->num_cus);
     if (ro.order) release_order(ro, s);
     if (e != hipSuccess) return hip_fail(ctx, e, "trace launch");
@@ -418,7 +418,7 @@ int sortgpu_trace_closest_noalloc(sortgpu_accel* acc, const sortgpu_ray* d_rays,
     a.error = acc->d_error;
     apply_tuning(ctx, a);
     const uint32_t reorder = ctx->tuning.reorder;
-    if (reorder == 2 || (reorder != 1 && reorder_pays(n, acc->view.walk_stack ? walk_bytes(acc->host) : 0))) {
+    if (reorder == 2 || (reorder != 1 && reorder_pays(n, walked_bytes(acc)))) {
         void* base = nullptr;
         hipError_t e = scratch_base(ctx->device, &base);
         if (e != hipSuccess) return hip_fail(ctx, e, "trace_closest_noalloc: scratch address");

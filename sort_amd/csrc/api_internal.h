@@ -92,6 +92,8 @@ constexpr uint32_t kReorderMinMulti = 1u << 20;
 inline size_t walk_bytes(const BuiltTree& t) {
     return t.walk.nodes.size() * sizeof(WalkNode) + t.walk.recs.size() * sizeof(PrimRec);
 }
+// The same of an accelerator as it lies on the device (its upload may have left the walk tree out).
+inline size_t walked_bytes(const sortgpu_accel* a) { return a->view.walk_stack ? walk_bytes(a->host) : 0; }
 // The default for closest- and any-hit batches on walk trees of `bytes` together (0: no walk tree).
 inline bool reorder_pays(uint32_t n, size_t bytes) {
     return bytes ? n >= kReorderMinWalkRays && bytes >= kReorderMinWalkBytes : n >= kReorderMinRays;

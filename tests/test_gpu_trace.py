@@ -174,11 +174,11 @@ def test_select_form_slab_tests(gpu_ctx, width):
 
 
 def test_traversal_order_changes_no_result(gpu_ctx):
-    """Large batches are traced in coherence order (sorted by origin and direction cell); the
-    order must not change a single bit of any result: never (1), always (2) and the default (0,
-    which sorts these 300K-ray batches) agree with each other and with the oracle, also for a
-    batch whose rays all share one sort key and for two streams tracing one accelerator at once
-    (each with its own stream-ordered sort buffers)."""
+    """Batches may be traced in traversal order (sorted by origin cell); the order must not change a
+    single bit of any result: never (1), always (2) and the default (0, which sorts larger batches on
+    larger trees only) agree with each other and with the oracle, also for a batch whose rays all share
+    one sort key and for two streams tracing one accelerator at once (each sorting in stream-ordered
+    buffers of its own)."""
     from sort_amd import batch
     pos, idx = scenes.soup(1 << 16, seed=41)
     acc, ob = _pair(gpu_ctx, pos, idx)
@@ -193,6 +193,7 @@ def test_traversal_order_changes_no_result(gpu_ctx):
             res[mode] = [acc.get_intersect(d_rays).cpu().numpy(), acc.is_occluded(d_rays).cpu().numpy(),
                          acc.get_intersect(d_one).cpu().numpy(), acc.is_occluded(d_one).cpu().numpy()]
         print("[order] two streams", flush=True)
+        batch.set_tuning(gpu_ctx, reorder=2)
         s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
         h1 = torch.empty((len(rays), 4), dtype=torch.float32, device="cuda")
         h2 = torch.empty((len(rays), 4), dtype=torch.float32, device="cuda")
@@ -213,6 +214,22 @@ def test_traversal_order_changes_no_result(gpu_ctx):
     ref = ob.closest(rays, threads=16)
     assert np.array_equal(res[0][0].view(np.uint32), ref.view(np.uint32))
     assert np.array_equal(res[0][1], ob.occluded(rays, threads=16))
+
+
+def test_default_order_on_a_tree_past_the_caches(gpu_ctx):
+    """The default sorts 2^21 rays on a walk tree of 192 MiB; closest and any hit agree with index order."""
+    from sort_amd import batch
+    acc = Obvh(gpu_ctx).build(*scenes.soup(3_700_000, seed=43))
+    d = torch.from_numpy(scenes.random_rays(1 << 21, 44, lo=-0.2, hi=1.2)).cuda()
+    print("[order] default, 2^21 rays, 3.7M triangles", flush=True)
+    got = acc.get_intersect(d), acc.is_occluded(d)
+    try:
+        batch.set_tuning(gpu_ctx, reorder=1)
+        ref = acc.get_intersect(d), acc.is_occluded(d)
+    finally:
+        batch.set_tuning(gpu_ctx)
+    assert torch.equal(got[0].view(torch.int32), ref[0].view(torch.int32)) and torch.equal(got[1], ref[1])
+    assert (ref[0].view(torch.int32)[:, 1] != -1).float().mean() > 0.3
 
 
 @pytest.mark.parametrize("width", [8, 4])

@@ -288,3 +288,25 @@ def test_directions_below_the_slab_clamp(gpu_ctx):
         d[k % 7 == 2] *= np.float32(30.0)
         o[k % 2 == 0] = (mesh[0][g.integers(0, len(mesh[0]), len(o))] - 0.7 * d)[k % 2 == 0]
         _check(acc, ob, scenes.make_rays(o, d.astype(np.float32), 0.0, FLT_MAX), "clamped directions")
+
+
+def test_pool_in_which_one_scene_has_no_walk_tree(gpu_ctx):
+    """A scene past the origin by more than 4,096 times its size has none; the pool's rays then all take the
+    Fast-BVH, closest and any hit, with the results that each scene gives alone."""
+    g = np.random.default_rng(23)
+    accs, rays = [], []
+    for n, shift in ((3000, 0.0), (2000, 3e4), (500, 0.0)):
+        t = g.uniform(0, 1, (n, 1, 3)) + g.uniform(-0.1, 0.1, (n, 3, 3)) + shift
+        mesh = scenes.tris_to_mesh(list(t.astype(np.float32)))
+        accs.append(_build(gpu_ctx, 8, mesh, None)[0])
+        rays.append(scenes.make_rays(*_rays(g, 5000, mesh), 0.0, FLT_MAX))
+    pool = batch.Pool(gpu_ctx, accs)
+    sid = np.repeat(np.arange(3), 5000).astype(np.int32)
+    d, ids = torch.from_numpy(np.concatenate(rays)).cuda(), torch.from_numpy(sid).cuda()
+    hits, occ = pool.trace(d, ids).cpu().numpy(), pool.trace(d, ids, any_hit=True).cpu().numpy()
+    pool.check_errors()
+    for i, acc in enumerate(accs):
+        one = torch.from_numpy(rays[i]).cuda()
+        assert np.array_equal(hits[sid == i].view(np.uint32), acc.get_intersect(one).cpu().numpy().view(np.uint32))
+        assert np.array_equal(occ[sid == i], acc.is_occluded(one).cpu().numpy())
+    pool.close()

@@ -41,15 +41,21 @@ def test_noalloc_equals_closest_on_successive_batches(gpu_ctx, soup_acc):
     acc = soup_acc
     rays = scenes.random_rays(LIMIT, 0xA110C, lo=-0.2, hi=1.2, tmin=1e-4)
     d_all = torch.from_numpy(rays).to("cuda:0")
-    for n, label in [(LIMIT, "full"), (300_000, "smaller"), (1000, "below the sort threshold")]:
+    # sorted, up to what the resident scratch array holds, and in index order
+    for n, label, reorder in [(LIMIT, "full", 2), (300_000, "smaller", 2), (1000, "in index order", 0)]:
         print(f"[noalloc] {label}: {n} rays", flush=True)
         d = d_all[:n].contiguous()
+        set_tuning(gpu_ctx, reorder=1)
         ref = acc.get_intersect(d).cpu().numpy()
+        set_tuning(gpu_ctx, reorder=reorder)
         out = torch.empty((n, 4), dtype=torch.float32, device="cuda:0")  # the caller's output
         gc.collect()  # objects of earlier tests free their device memory now, not during the call
         torch.cuda.synchronize()
         free0 = torch.cuda.mem_get_info(0)[0]
-        _noalloc(acc, d, out=out)
+        try:
+            _noalloc(acc, d, out=out)
+        finally:
+            set_tuning(gpu_ctx)
         torch.cuda.synchronize()
         free1 = torch.cuda.mem_get_info(0)[0]
         got = out.cpu().numpy()

@@ -14,6 +14,7 @@ visited + 36 * triangles tested, with the visit counts from the traversal's own 
 to the oracle's on these rays); achieved = bytes per launch / mean launch time (HIP events on
 the launch stream). Those are the bytes of the Fast-BVH walk, which defines the query's results; the
 kernel finds them through a smaller tree (walk.hip), so this fraction and the next may pass 1.
+roofline.traffic_frac is the kernel's own: the profiled bytes past the L2 of one launch over its time.
 roofline.memory_pipeline adds the ceiling that the Fast-BVH walk meets: lanes
 read their own records, so compute units return 16-byte chunks at a bounded rate; a probe kernel
 measures that rate for the traversal's two access patterns and gives the launch time it allows.
@@ -600,6 +601,8 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": profiled_traffic(a),
                      "traffic_source": TRAFFIC_PROFILE if profiled_traffic(a) else None,
+                     "traffic_frac": (round(profiled_traffic(a) / (mean_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)
+                                      if profiled_traffic(a) else None),
                      "bytes_per_ray": round(b_inc, 1), "launch_ms_mean": round(mean_ms, 4),
                      "launch_ms_median": round(med_ms, 4),
                      "visits_per_ray": {"inner_nodes": round(st_inc["inner_nodes"] / n, 3),

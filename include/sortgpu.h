@@ -83,8 +83,9 @@ const char* sortgpu_last_error(const sortgpu_ctx* ctx);
  * pos: nverts x 3 floats; idx: ntris x 3 vertex indices; quads: nquads records. The SAH
  * 8-wide (or 4-wide) tree is built on the host, flattened into the device layout and
  * uploaded, with a second tree over the same primitives that closest- and any-hit queries step
- * through to the same results (about 70 MB for a million triangles; scenes whose coordinates are not
- * finite, pass 1e12 or lie 4,096 times their size from the origin go without). Input arrays are copied; the caller keeps ownership. An empty scene yields a
+ * through to the same results (about 80 MB for a million triangles; left out where the memory is not to be
+ * had, where coordinates are not finite, pass 1e12, stay below 1e-8 or lie 4,096 times the scene's size from the
+ * origin, and where a quad's matrices are not each other's inverse). Input arrays are copied; the caller keeps ownership. An empty scene yields a
  * valid handle whose queries all miss (m_isValid = false, fast_bvh.hpp:112-114). At most
  * 2^30 - 1 primitives (triangles + quads) per tree (SORTGPU_ERR_ARG beyond). */
 int sortgpu_accel_build(sortgpu_ctx* ctx, const float* pos, uint32_t nverts, const uint32_t* idx,
@@ -372,8 +373,8 @@ typedef struct sortgpu_server sortgpu_server;
 
 typedef struct sortgpu_server_opts {
     uint64_t hbm_budget;     /* bytes the server may hold: scenes + films + workspace (0 = 96 GiB);
-                                a scene that would not fit alone is loaded without the second tree
-                                of its accelerator (sortgpu_accel_build) */
+                                a scene that would not fit alone with a request's film is loaded
+                                without the second tree of its accelerator (sortgpu_accel_build) */
     uint32_t wave_paths;     /* path slots per wave (0 = 33,554,432; 248 B of workspace each) */
     uint32_t max_active;     /* requests admitted at once, 1..32 (0 = 32) */
     uint32_t inflight_waves; /* waves in flight at once, 1..4 (0 = 3), each on a stream and path

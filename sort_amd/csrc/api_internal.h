@@ -73,13 +73,14 @@ void free_accel_device(sortgpu_accel* acc);
 // rays, and a sorted batch reads its rays and writes its results scattered; what it saves is
 // traffic past the caches. Measured on rays in random order, sorted against index order:
 //   walk tree (closest, any): pays once the tree outgrows the caches and the batch is large. 4M rays
-//     through 1M triangles (57 MB of nodes and records) 1.76 against 1.52 ms, 4M triangles (230 MB)
-//     1.91 / 1.95, 8M 1.94 / 2.19, 16M 2.01 / 2.41; shadow segments 1M 1.79 / 1.69, 4M 1.93 / 2.34,
-//     16M 2.13 / 3.07; 2M rays: 4M triangles 1.16 / 1.11 (shadow 1.16 / 1.31), 16M 1.20 / 1.36;
-//     1M rays: 0.86 / 0.77 through 8M triangles; a pool of 64 scenes and 8M triangles, rays shuffled
-//     over the scenes, 4.63 / 6.83;
+//     through 1M triangles (58 MB of nodes and records) 2.36 against 2.21 ms, 3.6M triangles (209 MB)
+//     2.46 / 2.91, 8M 2.68 / 3.43, 16M 2.67 / 3.76; shadow segments 1M 2.33 / 2.47, 3.6M 2.47 / 3.52,
+//     16M 2.78 / 4.68; 2M rays: 1M triangles 1.35 / 1.26 (shadow 1.35 / 1.39), 3.6M 1.51 / 1.66 (shadow
+//     1.43 / 1.93), 16M 1.59 / 2.13; 1M rays: 1M 0.99 / 0.84, 3.6M 0.97 / 0.95 (shadow 1.02 / 1.16), 8M
+//     1.11 / 1.15 (no line at 1M rays serves both kinds on such trees);
 //   transparent shadows: 524K rays through 200K triangles 1.99 / 1.90 ms, through 1M 2.63 / 2.75; 1M
-//     rays 2.96 / 2.97 and 3.80 / 4.10; 2M 4.94 / 5.11 and 6.38 / 6.82;
+//     rays 2.96 / 2.97 and 3.80 / 4.10; 2M 4.94 / 5.11 and 6.38 / 6.82 (the line looks at the rays alone: at
+//     524K it costs the smaller of these trees 5% and gives the larger 4%);
 //   multi-hit probes: 524K into 200K triangles 0.45 / 0.38, into 1M 0.56 / 0.51; 1M 0.62 / 0.69 and
 //     0.84 / 0.95; 4M 1.80 / 2.58 and 2.62 / 3.50;
 //   Fast-BVH walk (trees without a walk tree): batches of 256K rays and more.

@@ -3,7 +3,7 @@
 // (integrator/integratormethod.cpp:28-30,100-192), restructured as stages over fixed path slots:
 //
 //   raygen   camera rays (PerspectiveCamera::GenerateRay, camera/perspective.cpp:66-104) or caller rays
-//   extend   closest-hit traversal of the live queue (k_trace, device-side count)
+//   extend   closest-hit traversal of the live queue (k_walk, or k_trace without walk trees; device-side count)
 //   shade    emission at the first vertex, NEE (up to two shadow rays per vertex, written to
 //            per-path slots), BSDF continuation, Russian roulette, compaction of survivors by
 //            wave ballots + one atomic per queue and workgroup
@@ -47,7 +47,7 @@ __device__ __forceinline__ int sample_discrete(const float* cdf, uint32_t count,
 }
 
 // Where a workgroup's threads append to two queues whose counts lie side by side: one 64-bit atomic per
-// workgroup. Every thread of the workgroup calls it, `turn` counting the calls. A thread adds up to
+// workgroup. Every thread of the workgroup calls it. A thread adds up to
 // one entry to the first queue and two to the second, in thread order within its wave (the wave's
 // first entries of the second queue before its second ones).
 // An atomic on one address takes about 8.5 ns of the whole chip's time, so three atomics per wave bound
@@ -58,16 +58,15 @@ struct AppendSlots {
     uint32_t a, b0, b1;
 };
 struct AppendShared {
-    uint32_t cnt[2][2][kPtBlock / 64];
+    uint32_t cnt[2][kPtBlock / 64];
     unsigned long long base;
 };
-__device__ __forceinline__ AppendSlots block_append(AppendShared& sh, uint32_t turn, bool a, bool b0, bool b1,
-                                                    uint32_t* counts) {
+__device__ __forceinline__ AppendSlots block_append(AppendShared& sh, bool a, bool b0, bool b1, uint32_t* counts) {
     const uint32_t lane = __lane_id(), wave = threadIdx.x / 64;
     const uint64_t ma = __ballot(a), m0 = __ballot(b0), m1 = __ballot(b1);
     const uint64_t below = (1ull << lane) - 1ull;
-    // two sets of counts: a wave may write its next ones while another still reads these
-    uint32_t(*cnt)[kPtBlock / 64] = sh.cnt[turn & 1u];
+    // read between the two barriers: the second one keeps a wave's next counts off these
+    uint32_t(*cnt)[kPtBlock / 64] = sh.cnt;
     if (lane == 0) {
         cnt[0][wave] = (uint32_t)__popcll(ma);
         cnt[1][wave] = (uint32_t)(__popcll(m0) + __popcll(m1));
@@ -117,13 +116,15 @@ __device__ __forceinline__ void init_path(PathState ps, uint32_t p, uint32_t pix
     r[3] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// Camera rays of every chunk (PerspectiveCamera::GenerateRay in closed form: raster -> camera
-// through the inverse of Scale(W,H,1) Scale(.5,-.5,1) Translate(1,-1,0) Perspective(xs, ys),
-// then the orthonormal ViewLookat basis).
+// A wave's counts as its first bounce finds them (Queues::count).
 __device__ __forceinline__ void init_counts(uint32_t* count, uint32_t paths) {
     count[0] = paths;
     for (int k = 1; k < 6; k++) count[k] = 0;
 }
+
+// Camera rays of every chunk (PerspectiveCamera::GenerateRay in closed form: raster -> camera
+// through the inverse of Scale(W,H,1) Scale(.5,-.5,1) Translate(1,-1,0) Perspective(xs, ys),
+// then the orthonormal ViewLookat basis).
 __global__ __launch_bounds__(kPtBlock) void k_raygen(const WaveDesc* __restrict__ w, PathState ps, Queues q) {
     const ChunkTable& ct = w->ct;
     const uint32_t p = blockIdx.x * kPtBlock + threadIdx.x;
@@ -384,7 +385,6 @@ __global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(4))) v
     __shared__ AppendShared append;
     const uint32_t n = q.count[2 * cur];
     const int nxt = cur ^ 1;
-    uint32_t turn = 0;
     for (uint32_t base = blockIdx.x * kPtBlock; base < n; base += gridDim.x * kPtBlock) {
         const uint32_t k = base + threadIdx.x;
         const uint32_t i = (order && k < n) ? order[k] : k;
@@ -522,7 +522,7 @@ __global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(4))) v
             pr[3] = c1;
         }
         // compaction of survivors and shadow rays
-        const AppendSlots slot = block_append(append, turn++, cont, sh0, sh1, &q.count[2 * nxt]);
+        const AppendSlots slot = block_append(append, cont, sh0, sh1, &q.count[2 * nxt]);
         if (cont) {
             const uint32_t ci = slot.a;
             put_ray(q.ray[nxt], ci, ro, 0.0001f, rd, FLT_MAX);

@@ -27,7 +27,7 @@ struct TraceArgs {
     uint32_t refill;               // idle lanes that trigger a refill (default 16)
     uint32_t lds_entries;          // LDS stack entries per lane: 8 or 16 (default 16)
     uint32_t blocks_per_cu;        // cap on resident workgroups per CU (default: occupancy limit)
-    uint32_t leaf_batch;           // lanes holding a leaf that end a node phase (default 32)
+    uint32_t leaf_batch;           // lanes holding a leaf that end a node phase (default: walk.hip 24 of 64 at work, trace.hip 32)
     uint32_t leaf_min;             // a leaf phase ends below this many lanes holding a leaf (default 1)
     bool counter_clear = false;    // the work before this launch on its stream leaves the counter at 0
     // optional traversal order: the k-th ray taken from the work counter is rays[order[k]] (a

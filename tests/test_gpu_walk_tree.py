@@ -310,3 +310,37 @@ def test_pool_in_which_one_scene_has_no_walk_tree(gpu_ctx):
         assert np.array_equal(hits[sid == i].view(np.uint32), acc.get_intersect(one).cpu().numpy().view(np.uint32))
         assert np.array_equal(occ[sid == i], acc.is_occluded(one).cpu().numpy())
     pool.close()
+
+
+@pytest.mark.parametrize("wrong", [0.0, 1e-5, 0.05])
+def test_turned_quads(gpu_ctx, wrong):
+    """Quad lights turned and scaled any way among triangles, hit head-on, along their planes and at their edges;
+    with an inverse that is off by rounding, by 1e-5 and by more than a walk tree is built for."""
+    g = np.random.default_rng(29)
+    quads = []
+    for _ in range(12):
+        q, _ = np.linalg.qr(g.normal(size=(3, 3)))
+        m = np.eye(4)
+        m[:3, :3] = q * np.exp(g.uniform(-1, 1))
+        m[:3, 3] = g.uniform(0, 1, 3)
+        inv = np.linalg.inv(m)
+        inv[:3] += wrong * g.uniform(-1, 1, (3, 4))
+        quads.append(dict(mat=m.astype(np.float32).ravel(), inv=inv.astype(np.float32).ravel(), size_x=0.3, size_y=0.2))
+    t = g.uniform(0, 1, (600, 1, 3)) + g.uniform(-0.05, 0.05, (600, 3, 3))
+    mesh = scenes.tris_to_mesh(list(t.astype(np.float32)))
+    acc, ob = _build(gpu_ctx, 8, mesh, quads)
+    n = 24000
+    k = np.arange(n)
+    mats = np.stack([np.asarray(q["mat"], np.float64).reshape(4, 4) for q in quads])[k % 12]
+    local = np.stack([g.uniform(-0.2, 0.2, n), np.zeros(n), g.uniform(-0.15, 0.15, n)], 1)
+    local[k % 5 == 1, 0] = 0.15
+    at = np.einsum("nij,nj->ni", mats[:, :3, :3], local) + mats[:, :3, 3]
+    d = g.normal(size=(n, 3))
+    flat = k % 3 == 0  # along the quad's plane, or within 1e-6 of it
+    side = np.stack([g.normal(size=n), g.choice([0.0, 1e-6, 1e-3], n), g.normal(size=n)], 1)
+    d[flat] = np.einsum("nij,nj->ni", mats[:, :3, :3], side)[flat]
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    o = at - d * g.uniform(0.01, 2.0, (n, 1))
+    hits = _check(acc, ob, scenes.make_rays(o.astype(np.float32), d.astype(np.float32), 0.0, FLT_MAX), f"quads off by {wrong}")
+    prim = hits[:, 1].view(np.uint32)
+    assert np.mean((prim >= 600) & (prim != MISS)) > 0.1
